@@ -191,7 +191,7 @@ nsp_status nsp_remesh_weights(int nr_old, int nr_new, int flags, double* RM);
  * out[NR][NTP][NZF+2] doubles, NTP = 3NT/2, NZF = 3(NZ-1): row (i, j) holds
  * u(r_i, theta_j = 2 pi j/NTP, z_n = n LZ/NZF) for n < NZF, then the two
  * padding doubles of the in-place real transform (zero).  where: NSP_HOST or
- * NSP_DEVICE.  Uses the nonlinear-term workspace (nothing else changes). */
+ * NSP_DEVICE.  Uses the linear sweep's workspace (nothing else changes). */
 nsp_status nsp_physical_field(nsp_handle* h, int comp, double* out, int where);
 
 /* Cross-section integrals at the NZF axial points (wrt_qcr, wrt_ucr,

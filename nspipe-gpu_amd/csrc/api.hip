@@ -1022,18 +1022,18 @@ nsp_status nsp_remesh(nsp_handle* dst, nsp_handle* src, int flags) {
     if (s_) return s_;       \
   } while (0)
 
-// Workspace of the physical-space output: the nonlinear-term intermediates,
-// which hold nothing between steps.  Wt (NR*NTP*NZ complex) first, then the
-// physical rows (NR*NTP rows of NZF+2 doubles).
+// Workspace of the physical-space output: the sweep buffers, which hold
+// nothing between steps (W's padding columns have to stay zero for the pair z
+// pass).  Wt (NR*NTP*NZ complex) in E, the physical rows (NR*NTP rows of NZF+2
+// doubles) in SR.
 static nsp_status phys_scratch(nsp_handle* h, double2** Wt, double** F) {
   const Geom& g = h->g;
-  char* base = h->nb.mixed ? reinterpret_cast<char*>(h->nb.W32) : reinterpret_cast<char*>(h->nb.W);
-  const size_t cap = 9 * h->nb.wstride * (h->nb.mixed ? sizeof(float2) : sizeof(double2));
+  const size_t cap = 3 * sw_field(g) * sizeof(double2);
   const size_t wt = (size_t)g.nr * g.ntp * g.nz * sizeof(double2);
   const size_t fb = (size_t)g.nr * g.ntp * (g.nzf + 2) * sizeof(double);
-  if (wt + fb > cap) return fail(NSP_ERR_INVALID, "physical-space output exceeds the workspace");
-  *Wt = reinterpret_cast<double2*>(base);
-  *F = reinterpret_cast<double*>(base + wt);
+  if (wt > cap || fb > cap) return fail(NSP_ERR_INVALID, "physical-space output exceeds the workspace");
+  *Wt = h->E;
+  *F = reinterpret_cast<double*>(h->SR);
   return NSP_OK;
 }
 
@@ -1065,8 +1065,10 @@ nsp_status nsp_cross_sections(nsp_handle* h, double* q, double* u2) {
   double* F;
   CHECK(phys_scratch(h, &Wt, &F));
   const size_t pitch = g.nzf + 2;
-  double* q1 = reinterpret_cast<double*>(h->SR);
+  double* q1 = reinterpret_cast<double*>(h->SP);
   double* qd = q1 + (size_t)g.nr * g.nzf;
+  if (((size_t)g.nr + 1) * g.nzf * sizeof(double) > sw_field(g) * sizeof(double2))
+    return fail(NSP_ERR_INVALID, "cross-section integrals exceed the workspace");
   for (int which = 0; which < 2; which++) {
     double* dst = which == 0 ? q : u2;
     if (!dst) continue;

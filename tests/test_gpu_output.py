@@ -205,3 +205,23 @@ def test_driver_writes_diagnostics_and_restart(tmp_path):
     assert "restart at t=2.00000000e-01, step 20" in out.stdout
     meta = dict(line.split() for line in open(save1 / "restart.txt"))
     assert int(meta["step"]) == 25 and abs(float(meta["time"]) - 0.25) < 1e-12
+
+
+@pytest.mark.parametrize("prec", [nsp.FP64, nsp.MIXED], ids=["fp64", "mixed"])
+def test_output_leaves_the_nonlinear_workspace(prec):
+    """The pair z pass reads the padding columns of its input as zero modes:
+    physical-space output between two evaluations must not touch them."""
+    shape = dict(nr=8, nt=64, nz=65, lz=4 * np.pi, re=2000.0, dt=0.005)
+    print(f"[gpu] output between nonlinear evaluations, precision {prec}", flush=True)
+    p = nsp.Pipe(**shape, precision=prec)
+    p.seeded_ic(7, 6, 6, 1, 0.1)
+    p.set_tuning(dict(theta_inv=dict(alg=0, tl=8, nthr=256, pad=0, ord=1),
+                      theta_fwd=dict(alg=1, tl=8, nthr=256, pad=0, ord=1), z_alg=4, z_nthr=512, z_pad=1, z_pf=0))
+    u = p.get_state()
+    before = p.nonlinear(*u)
+    p.cross_sections()
+    p.physical(0)
+    after = p.nonlinear(*u)
+    p.close()
+    for c in range(3):
+        assert np.array_equal(before[c], after[c])
