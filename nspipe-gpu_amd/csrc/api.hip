@@ -283,6 +283,17 @@ nsp_status nsp_default_params(nsp_params* p, int nr, int nt, int nz, double lz, 
   return NSP_OK;
 }
 
+// The kernel forms of a pipe that has not been tuned, by transform length and
+// precision.  z pass: the row-pair form, the fastest of those that keep the
+// accuracy of one transform per field (the figures are at zpass5_ct).  Loading
+// the next field during the LDS passes pays except where its registers take
+// a workgroup off the CU (FP32 rows of 4608: 1.32 against 1.56 ms for 24 x 576
+// rows; rows of 9216: no gain).
+static NlVariant default_variant(const Geom& g, bool mixed) {
+  const int pf = g.nh <= 1536 || (g.nh <= 2304 && !mixed) ? 1 : 0;
+  return NlVariant{ThetaVar{0, 8, 256, 0, 1}, ThetaVar{0, 8, 256, 0, 1}, 5, 256, 0, pf, 1, 1};
+}
+
 // share: a handle with identical parameters whose operator data (LU factors,
 // pressure homogeneous solution, influence-matrix column, flux profile) this
 // one uses instead of computing its own; it must outlive this handle.
@@ -369,18 +380,15 @@ static nsp_status create_handle(const nsp_params* p, int device, const nsp_handl
   h->nb.wstride = size_t(g.nr) * tp_plane(g);  // tile-major planes (tp_plane)
   h->nb.use_ct = false;
   h->nb.mixed = p->precision != NSP_FP64;
-  h->nb.var = NlVariant{ThetaVar{0, 8, 256, 0, 1}, ThetaVar{0, 8, 256, 0, 1}, 1, 256, 0, 0, 1, 1};
-  if (!ct_has_zreg(g.nh)) {  // long axial rows: the 512-thread LDS form
-    h->nb.var.z_alg = 0;
-    h->nb.var.z_nthr = 512;
-  }
+  h->nb.var = default_variant(g, h->nb.mixed);
   const bool have_ct = ct_has_theta(g.ntp) && ct_has_zhalf(g.nh);
   if (h->nb.mixed && !have_ct)
     return bail(fail(NSP_ERR_INVALID, "the mixed form needs compiled transform plans for 3NT/2 and 3(NZ-1)/2"));
   if (have_ct && (h->nb.mixed || !getenv("NSP_GENERIC_FFT"))) {
     const auto twt = pass_twiddles(ct_radices(g.ntp, true));
     // the half-length plan's pass twiddles, then those of the pair form's
-    // full-length plan and the compact table of its last pass
+    // full-length plan and the compact table of its last pass, then those of
+    // the row-pair form's plan
     auto twh = pass_twiddles(ct_radices(g.nh, false));
     const auto rpair = ct_pair_radices(g.nh);
     if (!rpair.empty()) {
@@ -389,6 +397,8 @@ static nsp_status create_handle(const nsp_params* p, int device, const nsp_handl
       const auto twc = compact_twiddles(rpair);
       twh.insert(twh.end(), twc.begin(), twc.end());
     }
+    const auto twr = pass_twiddles(ct_row_radices(g.nh, h->nb.mixed));
+    twh.insert(twh.end(), twr.begin(), twr.end());
     if (h->nb.mixed) {
       TRY(upload(h, &h->nb.ct_tw_t32, to_float2(twt)));
       TRY(upload(h, &h->nb.ct_tw_h32, to_float2(twh)));
@@ -704,6 +714,15 @@ nsp_status nsp_autotune(nsp_handle* h, int reps) {
         const double t = time_it(1, v, lab);
         if (t >= 0 && t < bt) { bt = t; best.z_alg = alg; best.z_pad = pad; best.z_pf = pf; }
       }
+  for (int pf = 0; pf < 2; pf++) {
+    NlVariant v = best;
+    v.z_alg = 5;
+    v.z_pf = pf;
+    char lab[64];
+    std::snprintf(lab, sizeof lab, "zpass row pairs pf=%d", pf);
+    const double t = time_it(1, v, lab);
+    if (t >= 0 && t < bt) { bt = t; best.z_alg = 5; best.z_pf = pf; }
+  }
   // the nonlinear stage in level chunks on two streams (z pass of one chunk
   // beside the theta inverse of the next) or stage after stage
   bt = 1e30;

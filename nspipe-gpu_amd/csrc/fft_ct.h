@@ -184,6 +184,49 @@ template <typename T, int SIGN> struct DFT<T, 16, SIGN> {
 template <typename T, int SIGN> struct DFT<T, 18, SIGN> {
   __device__ __forceinline__ static void run(cpx<T>* v) { dft_composite<T, 9, 2, SIGN>(v); } };
 
+// Inverse or forward DFT of a radix R divisible by 3 whose inputs R/3 < q <
+// 2R/3 are zero (not read): R = 3 (R/3), so the middle input of every
+// three-point DFT but the first is one of them.
+template <typename T, int R, int SIGN>
+__device__ __forceinline__ void dft_zero_mid(cpx<T>* v) {
+  static_assert(R % 3 == 0, "thirds");
+  constexpr int R2 = R / 3;
+  constexpr T h = T(-0.5);
+  constexpr T sn = T(SIGN) * T(0.86602540378443864676372317075294L);
+  cpx<T> y[3][R2];
+#pragma unroll
+  for (int n2 = 0; n2 < R2; ++n2) {
+    if (n2 == 0) {
+      cpx<T> a[3] = {v[0], v[R2], v[2 * R2]};
+      DFT<T, 3, SIGN>::run(a);
+#pragma unroll
+      for (int k1 = 0; k1 < 3; ++k1) y[k1][0] = a[k1];
+    } else {
+      const cpx<T> a = v[n2], c = v[2 * R2 + n2];
+      const cpx<T> m{a.x + h * c.x, a.y + h * c.y};
+      y[0][n2] = {a.x + c.x, a.y + c.y};
+      const cpx<T> z[2] = {{m.x + sn * c.y, m.y - sn * c.x}, {m.x - sn * c.y, m.y + sn * c.x}};
+#pragma unroll
+      for (int k1 = 1; k1 < 3; ++k1) {
+        const int e = (n2 * k1) % R;
+        const cpx<T> b = z[k1 - 1];
+        if (4 * e == R) {
+          y[k1][n2] = {T(SIGN) * -b.y, T(SIGN) * b.x};
+        } else {
+          const T tc = T(kTw<R>.c[e]), ts = T(SIGN) * T(kTw<R>.s[e]);
+          y[k1][n2] = {b.x * tc - b.y * ts, b.x * ts + b.y * tc};
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int k1 = 0; k1 < 3; ++k1) {
+    if constexpr (R2 > 1) DFT<T, R2, SIGN>::run(y[k1]);
+#pragma unroll
+    for (int k2 = 0; k2 < R2; ++k2) v[k1 + 3 * k2] = y[k1][k2];
+  }
+}
+
 // ---------------------------------------------------------------- plans
 template <int... R>
 struct Plan {
@@ -460,9 +503,11 @@ __device__ __forceinline__ void fft_run_tw(Plan<R...>, cpx<T>* buf, const cpx<T>
 // digit-reversed positions are Plan::digitrev(n0) + q, so the radix-R0
 // butterfly (no twiddles at sub-length 1) runs on them directly and stores
 // its outputs there; no scatter through LDS is needed.
-template <typename T, int SIGN, typename LY, int NCOL, int R0, int... Rest>
+// ZMID: the inputs R0/3 < q < 2 R0/3 are zero (and not read).
+template <typename T, int SIGN, typename LY, int NCOL, bool ZMID = false, int R0, int... Rest>
 __device__ __forceinline__ void first_pass_store(Plan<R0, Rest...>, cpx<T>* v, cpx<T>* buf, int n0, int col = 0) {
-  DFT<T, R0, SIGN>::run(v);
+  if constexpr (ZMID && R0 % 3 == 0) dft_zero_mid<T, R0, SIGN>(v);
+  else DFT<T, R0, SIGN>::run(v);
   // digitrev(n0) = R0 * (n0's position in the plan of the remaining radices)
   unsigned j = 0;
   if constexpr (sizeof...(Rest) > 0) j = (unsigned)Plan<Rest...>::digitrev(n0);
@@ -479,6 +524,55 @@ template <typename T, int NTHR, int SIGN, typename LY, int TWL, int TWC, int R0,
 __device__ __forceinline__ void fft_rest_tw(Plan<R0, Rest...>, cpx<T>* buf, const cpx<T>* __restrict__ tw,
                                             const cpx<T>* twl, const cpx<T>* twc, int tid) {
   dit_passes<T, Plan<R0, Rest...>::L, 1, NTHR, SIGN, LY, TWL, TWC, R0, R0 - 1, Rest...>(buf, tw, twl, twc, tid);
+}
+// The passes between the first and the last one (after first_pass_store and a
+// barrier); ends with a barrier.  The first TWL twiddle entries are read from
+// their LDS copy twl.
+template <typename T, int L, int NTHR, int SIGN, typename LY, int TWL, int S, int TWO, int R, int... Rest>
+__device__ __forceinline__ void dit_mid(cpx<T>* buf, const cpx<T>* __restrict__ tw, const cpx<T>* twl, int tid) {
+  if constexpr (sizeof...(Rest) > 0) {
+    constexpr int TOT = L / R;
+    constexpr int ITER = (TOT + NTHR - 1) / NTHR;
+    __builtin_assume((unsigned)tid < (unsigned)NTHR);
+#pragma unroll
+    for (int it = 0; it < ITER; ++it) {
+      const int b = tid + it * NTHR;
+      if ((TOT % NTHR) == 0 || b < TOT) {
+        cpx<T> v[R];
+        const Group<LY, 1, S, R> gr(b);
+        dit_butterfly<T, L, 1, SIGN, LY, TWL, 0, S, TWO, R>(buf, tw, twl, nullptr, gr, v);
+        dit_store<T, 1, LY, S, R>(buf, v, gr);
+      }
+    }
+    __syncthreads();
+    dit_mid<T, L, NTHR, SIGN, LY, TWL, S * R, TWO + S * (R - 1), Rest...>(buf, tw, twl, tid);
+  }
+}
+template <typename T, int NTHR, int SIGN, typename LY, int TWL, int R0, int... Rest>
+__device__ __forceinline__ void fft_mid(Plan<R0, Rest...>, cpx<T>* buf, const cpx<T>* __restrict__ tw, const cpx<T>* twl,
+                                        int tid) {
+  dit_mid<T, Plan<R0, Rest...>::L, NTHR, SIGN, LY, TWL, R0, R0 - 1, Rest...>(buf, tw, twl, tid);
+}
+// The last pass's butterfly tid (< L / R_last): its outputs, the elements
+// tid + (L / R_last) q, in v.
+template <typename T, int SIGN, typename LY, int TWL, int... R>
+__device__ __forceinline__ void fft_last(Plan<R...>, cpx<T>* buf, const cpx<T>* __restrict__ tw, const cpx<T>* twl,
+                                         int tid, cpx<T>* v) {
+  using PL = Plan<R...>;
+  constexpr int RL = PL::rad[PL::P - 1];
+  constexpr int S = PL::L / RL;
+  __builtin_assume((unsigned)tid < (unsigned)S);
+  // the twiddles of the earlier passes are the first S - 1 entries
+  dit_butterfly<T, PL::L, 1, SIGN, LY, TWL, 0, S, S - 1, RL>(buf, tw, twl, nullptr, Group<LY, 1, S, RL>(tid), v);
+}
+// The last pass with its outputs stored in natural order; ends with a barrier.
+template <typename T, int NTHR, int SIGN, typename LY, int TWL, int... R>
+__device__ __forceinline__ void fft_last_store(Plan<R...>, cpx<T>* buf, const cpx<T>* __restrict__ tw, const cpx<T>* twl,
+                                               int tid) {
+  using PL = Plan<R...>;
+  constexpr int RL = PL::rad[PL::P - 1];
+  constexpr int S = PL::L / RL;
+  dit_passes<T, PL::L, 1, NTHR, SIGN, LY, TWL, 0, S, S - 1, RL>(buf, tw, twl, nullptr, tid);
 }
 // Remaining passes after first_pass_store of NCOL interleaved columns (and a
 // barrier): the butterflies of all columns are spread over the threads.

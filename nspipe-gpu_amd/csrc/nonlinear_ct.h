@@ -21,6 +21,14 @@ __device__ __forceinline__ int opaque(int x) {
   return x;
 }
 
+// Fixes a value where it is formed: without it the compiler sinks a product
+// past the following transform to its use and holds the factors' registers.
+template <typename T>
+__device__ __forceinline__ void pin(cpx<T>& v) {
+  asm volatile("" : "+v"(v.x));
+  asm volatile("" : "+v"(v.y));
+}
+
 // Raw buffer loads.  A load whose byte offset lies past num_records returns
 // zero instead of touching memory, which gives the zero padding of a row
 // beyond its stored modes without clamps or selects.  The resource is the
@@ -1064,6 +1072,287 @@ __global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(sizeof(T) 
   }
 }
 
+// ------------------------------------------------------------------ z pass, row-pair form
+// Two rows (th, th + 1) of one level together: the real transforms of a field
+// on the two rows run as one complex transform of the full length NZF,
+// z = a + i b with a the first row and b the second, from Z[k] = A[k] + i B[k]
+// with A[NZF - k] = conj A[k] (the stored modes k < NZ, zero up to NZF/2; the
+// l = 0 mode enters with its real part only, as in the C2R forms).  The
+// forward transform of a product takes both rows the same way, separated
+// afterwards: A[k] = (Z[k] + conj Z[NZF - k]) / 2, B[k] = (Z[k] - conj
+// Z[NZF - k]) / 2i.  15 complex transforms per pair of rows, no even/odd
+// split, no split twiddles.  A pair is rounded at the scale of its larger
+// member; the two rows carry the same field, so both keep the accuracy of a
+// transform of their own.  (Pairing different fields of one row rounded the
+// smaller one at the larger one's scale: N_t of the FP32 form was 6e-7 off
+// instead of 1.7e-7 on a k^(-5/3) spectrum.)  The mean flow and its shear
+// (the l = 0 modes of u_z and d_r u_z, constant along the row and an order of
+// magnitude above the fluctuations) are kept out of their transforms and
+// added to the samples afterwards.
+//
+// Where the plan's first and last radix are equal (R0), with NB1 = NZF / R0
+// butterflies each, one per thread, the thread that feeds the first pass
+// x[n0 + NB1 q] from global memory also runs the last pass's butterfly n0,
+// whose outputs are the samples n0 + NB1 q.  Its samples of every field stay
+// in registers from the last pass of an inverse transform through the
+// products to the first pass of the forward one, so an inverse transform
+// moves through LDS only between its passes.  Modes NZF/3 < n < 2 NZF/3 are
+// the 3/2 padding: the first pass leaves out the inputs that lie there for
+// every thread (a third of a radix divisible by 3).
+//
+// Where the plan's first and last radix differ (rows of 4608 and 9216: the
+// equal-radix plans need 12 samples per thread, which leaves six waves per CU
+// at their registers, or nine waves of 8) the last pass stores its outputs and
+// the thread reads its samples back.
+//
+// Bound by VALU issue and LDS; the twiddles are read from LDS (they fill the
+// vector cache's bandwidth otherwise).  Layout: rows of NZF / R_last elements
+// padded by one slot (bank model of the passes).  Measured, z pass of one
+// nonlinear evaluation, this form against the register form (zpass2_ct), ms:
+// 32 x 96 rows of 192 FP64 0.026 / 0.35, 64 x 288 of 1152 FP64 0.66 / 1.58 and
+// FP32 0.32 / 0.84, 48 x 144 of 1536 FP32 0.15 / 0.32, 64 x 192 of 3072 FP64
+// 1.14 / 2.73, 24 x 576 of 4608 FP64 2.33 / 4.0 and FP32 1.32 / 1.6 (the pair
+// form with two rows per workgroup: 2.22 and 1.08, less accurate).
+
+// Waves per SIMD the registers are allotted for (FP32 without prefetch; the
+// others take what they need).
+template <typename T, int PFE, typename PF>
+constexpr int zrow_waves() {
+  return sizeof(T) == 4 && !PFE ? (PF::rad[0] >= 16 ? 2 : (PF::rad[0] == 9 ? 4 : 3)) : 1;
+}
+template <typename T, int PFE, typename PF, int BAT>
+__global__ __launch_bounds__(PF::L / PF::rad[0]) __attribute__((amdgpu_waves_per_eu((zrow_waves<T, PFE, PF>())))) void zpass5_ct(
+    Geom g, const cpx<T>* __restrict__ tw, const double* __restrict__ r, const cpx<T>* __restrict__ W, size_t ws,
+    cpx<T>* __restrict__ Y, const NlMember* tab) {
+  if constexpr (BAT != 0) {
+    const NlMember& m = tab[blockIdx.y];
+    g = m.g;
+    r = gmem(tab, m.r);
+    W = gmem(tab, reinterpret_cast<const cpx<T>*>(m.W));
+    Y = gmem(tab, reinterpret_cast<cpx<T>*>(m.Y));
+    ws = m.ws;
+  }
+  if (step_done(g)) return;
+  constexpr int NF = PF::L;
+  constexpr int NH = NF / 2;
+  constexpr int R0 = PF::rad[0];
+  constexpr int NB1 = NF / R0;
+  constexpr int RL = PF::rad[PF::P - 1];
+  constexpr bool SYM = R0 == RL;  // the last pass's outputs are the thread's own samples
+  using LY = Lay<NF / RL, 1>;
+  constexpr int BUF = LY::size(NF);
+  // The pass twiddles in LDS, within the workgroup's share of the CU's 160 KB:
+  // all of them, or those of every pass but the last (rows of 9216, where
+  // copying the whole table per workgroup costs more than it saves: FP32 1.43
+  // against 1.38 ms on 12 x 576 rows)
+  constexpr int WPE = zrow_waves<T, PFE, PF>() > 2 ? zrow_waves<T, PFE, PF>() : 2;
+  constexpr int PERCU = WPE * 256 / NB1 > 1 ? WPE * 256 / NB1 : 1;
+  constexpr int ROOM = (163840 / PERCU - BUF * (int)sizeof(cpx<T>)) / (int)sizeof(cpx<T>);
+  constexpr int TWL = NF - 1 <= ROOM && NF <= 4608 ? NF - 1 : (NF / RL - 1 <= ROOM ? NF / RL - 1 : 0);
+  __shared__ cpx<T> buf[BUF];
+  __shared__ cpx<T> twl[TWL ? TWL : 1];
+  const cpx<T>* __restrict__ twf = tw;  // the plan's pass twiddles
+  const int t0 = threadIdx.x;
+  // row pairs of this member (or level chunk); NTP is even, so a pair lies in one level
+  if ((int)blockIdx.x >= g.nlv * g.ntp / 2) return;
+  const int row = g.lv0 * g.ntp + 2 * (int)blockIdx.x;
+  const int i = row / g.ntp;
+  const int nz = g.nz;
+  const int t64 = g.ntp * 64;
+  const T kz0 = T(g.kz0);
+  const cpx<T> zero{T(0), T(0)};
+  constexpr int CS = (int)sizeof(cpx<T>);
+  const T rad = T(r[i]);
+  const T irad = T(1) / rad;
+  const int th = row - i * g.ntp;
+  const size_t roff = (size_t)i * tp_plane(g) + (size_t)th * 64;
+  const int rbytes = (int)((tp_plane(g) - (size_t)th * 64) * sizeof(cpx<T>));
+  // inputs of the first pass that lie in the padding for every thread
+  auto pad_q = [](int q) constexpr -> bool { return 3 * NB1 * q > NF && 3 * (NB1 * (q + 1) - 1) < 2 * NF; };
+  // sample n = n0 + NB1 q reads mode m = n (n <= NZF/2) or NZF - n (conjugated)
+  auto conj_of = [](int lt, int q) -> bool {
+    if (NB1 * (q + 1) <= NH + 1) return false;  // every lane: n <= NH
+    if (NB1 * q > NH) return true;              // every lane: n > NH
+    return lt + NB1 * q > NH;
+  };
+  // byte offset of the stored mode of sample n: columns nz <= m < 64 ceil(nz / 64)
+  // are W's zero padding (W starts zeroed and is written at m < nz only),
+  // columns beyond lie past the end of the row's plane, where the buffer range
+  // check returns zero (for both rows: the second lies 64 values further in
+  // the same tile).  With NB1 and NZF multiples of 64 the offsets are affine in q.
+  auto offset = [&](int lt, int q) -> int {
+    const int n = lt + NB1 * q;
+    if constexpr (NB1 % 64 == 0 && NF % 64 == 0) {
+      const int dq = (NB1 / 64) * t64 * CS;
+      const int ok = ((lt >> 6) * t64 + (lt & 63)) * CS + q * dq;
+      const int oc = (((NF >> 6) - ((lt + 63) >> 6)) * t64 + ((-lt) & 63)) * CS - q * dq;
+      return conj_of(lt, q) ? oc : ok;
+    } else {
+      const int m = conj_of(lt, q) ? NF - n : n;
+      return ((m >> 6) * t64 + (m & 63)) * CS;  // tp_col(g, m)
+    }
+  };
+  if constexpr (TWL != 0) {  // read after the barrier that follows the first pass of the first field
+    for (int e = t0; e < TWL; e += NB1) twl[e] = twf[e];
+  }
+  // LDS position of output n = lt + NB1 q (0 <= lt < NB1): with rows of RW
+  // elements and NB1 <= RW, the row of n is that of NB1 q or the next one, so
+  // one comparison replaces the division
+  auto out_pos = [](int lt, int q) -> int {
+    constexpr int RW = NF / RL;
+    if constexpr (NB1 <= RW) {
+      const int c = NB1 * q;
+      return lt + c + c / RW + (lt >= RW - c % RW ? 1 : 0);
+    } else {
+      return LY::pos(lt + NB1 * q);
+    }
+  };
+  cpx<T> A[R0], B[R0];
+  auto load = [&](int f) {  // the two rows' modes of field f
+    const int lt = opaque(t0);
+    const nsp_i4v rs = buf_rsrc(W + f * ws + roff, rbytes);
+#pragma unroll
+    for (int q = 0; q < R0; q++) {
+      if (pad_q(q)) continue;
+      const int o = offset(lt, q);
+      A[q] = buf_load<T>(rs, o);
+      B[q] = buf_load<T>(rs, o + 64 * CS);
+    }
+  };
+  // inverse transform of A, B (differentiated in z where DZ; sub0: without the
+  // l = 0 mode) into the samples s.  PFE 1 issues the loads of field fnext (if
+  // any) right after the first pass (in flight during the LDS passes); with
+  // PFE 0 the caller loads once it has used s (fewer live registers)
+  auto inverse = [&](auto dz_tag, bool sub0, int fnext, cpx<T>(&s)[R0]) {
+    constexpr bool DZ = decltype(dz_tag)::value;
+    const int lt = opaque(t0);
+    {
+      cpx<T> v[R0];
+#pragma unroll
+      for (int q = 0; q < R0; q++) {
+        if (pad_q(q)) {
+          v[q] = zero;
+          continue;
+        }
+        const int n = lt + NB1 * q;
+        const bool cj = conj_of(lt, q);
+        cpx<T> a = A[q], b = B[q];
+        if (q == 0 && n == 0) {
+          a = cpx<T>{sub0 ? T(0) : a.x, T(0)};
+          b = cpx<T>{sub0 ? T(0) : b.x, T(0)};
+        }
+        cpx<T> z = cj ? cpx<T>{a.x + b.y, b.x - a.y} : cpx<T>{a.x - b.y, a.y + b.x};
+        if constexpr (DZ) {  // derivz_k (mod_deriv.cu:24-35): i kz on the signed wavenumber
+          const T km = kz0 * T(cj ? n - NF : n);
+          z = cpx<T>{-km * z.y, km * z.x};
+        }
+        v[q] = z;
+      }
+      first_pass_store<T, +1, LY, 1, pad_q(R0 / 3 + 1)>(PF{}, v, buf, lt);
+    }
+    if (PFE && fnext >= 0) load(fnext);
+    __syncthreads();
+    fft_mid<T, NB1, +1, LY, TWL>(PF{}, buf, twf, twl, lt);
+    if constexpr (SYM) {
+      fft_last<T, +1, LY, TWL>(PF{}, buf, twf, twl, lt, s);
+    } else {
+      fft_last_store<T, NB1, +1, LY, TWL>(PF{}, buf, twf, twl, lt);
+#pragma unroll
+      for (int q = 0; q < R0; q++) s[q] = buf[out_pos(lt, q)];
+    }
+    __syncthreads();
+  };
+  auto next = [&](int f) {
+    if (!PFE && f >= 0) load(f);
+  };
+  // forward transform of the two rows' products v (N = -v), separated into rows d, d + 64 of Y
+  auto forward = [&](cpx<T>(&v)[R0], cpx<T>* d) {
+    const int lt = opaque(t0);
+    first_pass_store<T, -1, LY, 1>(PF{}, v, buf, lt);
+    __syncthreads();
+    fft_mid<T, NB1, -1, LY, TWL>(PF{}, buf, twf, twl, lt);
+    fft_last_store<T, NB1, -1, LY, TWL>(PF{}, buf, twf, twl, lt);
+    for (int k = lt; k < nz; k += NB1) {
+      cpx<T> xa = zero, xb = zero;
+      if (k < nz - 1) {
+        const cpx<T> zk = buf[LY::pos(k)], zc = buf[LY::pos(k == 0 ? 0 : NF - k)];
+        xa = cpx<T>{T(-0.5) * (zk.x + zc.x), T(-0.5) * (zk.y - zc.y)};
+        xb = cpx<T>{T(-0.5) * (zk.y + zc.y), T(0.5) * (zk.x - zc.x)};
+      }
+      cpx<T>* const o = d + (k >> 6) * t64 + (k & 63);  // tp_col(g, k)
+      o[0] = xa;
+      o[64] = xb;
+    }
+    __syncthreads();
+  };
+  using NoDz = std::integral_constant<bool, false>;
+  using Dz = std::integral_constant<bool, true>;
+  // field index in W: u_r, u_t, u_z (0-2), d_r u_c (3 + c), d_theta u_c / r (6 + c)
+  cpx<T> ur[R0], ut[R0], uz[R0], s[R0];
+  load(2);
+  // l = 0 modes of u_z and d_r u_z on the two rows
+  const cpx<T> m0z{W[2 * ws + roff].x, W[2 * ws + roff + 64].x}, m0d{W[5 * ws + roff].x, W[5 * ws + roff + 64].x};
+  inverse(NoDz{}, true, 1, uz);
+#pragma unroll
+  for (int q = 0; q < R0; q++) {
+    uz[q] = cpx<T>{uz[q].x + m0z.x, uz[q].y + m0z.y};
+    pin(uz[q]);
+  }
+  next(1);
+  inverse(NoDz{}, false, 0, ut);
+#pragma unroll
+  for (int q = 0; q < R0; q++) pin(ut[q]);
+  next(0);
+  inverse(NoDz{}, false, 3, ur);
+#pragma unroll
+  for (int q = 0; q < R0; q++) pin(ur[q]);
+  next(3);
+  // calcNonlinear_k (mod_io_nonlinear.cu:142-170), summed in its order
+#pragma unroll 1
+  for (int c = 0; c < 3; c++) {
+    cpx<T> acc[R0];
+    inverse(NoDz{}, c == 2, 6 + c, s);
+    const cpx<T> m0 = c == 2 ? m0d : zero;
+#pragma unroll
+    for (int q = 0; q < R0; q++) {
+      acc[q] = cpx<T>{ur[q].x * (s[q].x + m0.x), ur[q].y * (s[q].y + m0.y)};
+      pin(acc[q]);
+    }
+    next(6 + c);
+    inverse(NoDz{}, false, c, s);
+#pragma unroll
+    for (int q = 0; q < R0; q++) {
+      acc[q].x += ut[q].x * s[q].x;
+      acc[q].y += ut[q].y * s[q].y;
+      pin(acc[q]);
+    }
+    next(c);
+    const int fn = c < 2 ? 4 + c : -1;
+    inverse(Dz{}, false, fn, s);
+#pragma unroll
+    for (int q = 0; q < R0; q++) {
+      acc[q].x = acc[q].x + uz[q].x * s[q].x;
+      acc[q].y = acc[q].y + uz[q].y * s[q].y;
+    }
+    if (c < 2) {
+      // x / r: the FP32 form multiplies by the reciprocal, the FP64 form
+      // divides.  The divisor is opaque to the compiler, which would otherwise
+      // form the curvature products before the loop and hold them in registers.
+      T rr = c == 0 ? (sizeof(T) == 4 ? -irad : -rad) : (sizeof(T) == 4 ? irad : rad);
+      asm volatile("" : "+v"(rr));
+#pragma unroll
+      for (int q = 0; q < R0; q++) {
+        const cpx<T> w = c == 0 ? ut[q] : ur[q];
+        const cpx<T> o = sizeof(T) == 4 ? cpx<T>{ut[q].x * rr, ut[q].y * rr} : cpx<T>{ut[q].x / rr, ut[q].y / rr};
+        acc[q].x = acc[q].x + w.x * o.x;
+        acc[q].y = acc[q].y + w.y * o.y;
+      }
+    }
+    forward(acc, Y + c * ws + roff);
+    next(fn);
+  }
+}
+
 // ------------------------------------------------------------------ theta forward
 template <typename T, int TL, int NTHR, typename LY, typename PL, int BAT>
 __global__ __launch_bounds__(NTHR) void theta_fwd_ct(Geom g, const cpx<T>* __restrict__ tw,
@@ -1361,6 +1650,36 @@ struct ZPair {
 NSP_ZPAIR_PLANS(X)
 #undef X
 
+// Full-length plans of the row-pair form, keyed by NH: FP32, FP64.
+#define NSP_ZROW_PLANS(X)                             \
+  X(96, Plan<4, 3, 4, 4>, Plan<4, 3, 4, 4>)           \
+  X(576, Plan<6, 4, 8, 6>, Plan<6, 4, 8, 6>)          \
+  X(768, Plan<8, 3, 8, 8>, Plan<8, 3, 8, 8>)          \
+  X(1536, Plan<16, 12, 16>, Plan<8, 6, 8, 8>)         \
+  X(2304, Plan<9, 8, 8, 8>, Plan<9, 8, 8, 8>)         \
+  X(4608, Plan<18, 8, 8, 8>, Plan<18, 8, 8, 8>)
+
+template <int NH, typename T>
+struct ZRow {
+  using P = void;
+};
+template <typename A, typename B>
+struct TwoPlans {
+  using P32 = A;
+  using P64 = B;
+};
+#define X(LL, ...)                                 \
+  template <>                                      \
+  struct ZRow<LL, float> {                         \
+    using P = typename TwoPlans<__VA_ARGS__>::P32; \
+  };                                               \
+  template <>                                      \
+  struct ZRow<LL, double> {                        \
+    using P = typename TwoPlans<__VA_ARGS__>::P64; \
+  };
+NSP_ZROW_PLANS(X)
+#undef X
+
 #define NSP_ZHALF_PLANS(X)    \
   X(96, Plan<6, 16>)          \
   X(576, Plan<4, 9, 16>)      \
@@ -1368,6 +1687,15 @@ NSP_ZPAIR_PLANS(X)
   X(1536, Plan<6, 16, 16>)    \
   X(2304, Plan<9, 16, 16>)    \
   X(4608, Plan<9, 2, 16, 16>)
+
+// Offset of the row-pair plan's pass twiddles in a pipe's z twiddle table:
+// after the half-length plan's (NH - 1 entries) and the pair plan's (NZF - 1,
+// and 3 NZF / 8 of the compact table where its last radix is 8).
+template <int NH>
+constexpr int zrow_tw() {
+  using P4 = typename ZPair<NH>::P;
+  return NH - 1 + 2 * NH - 1 + (P4::rad[P4::P - 1] == 8 ? 3 * (2 * NH / 8) : 0);
+}
 
 // ------------------------------------------------------------------ stage launchers
 // A form is compiled for a plan only if its LDS buffer fits the 160 KB of a CU.
@@ -1532,6 +1860,21 @@ bool zpass_plan(const NlVariant& v, const Geom& g, const cpx<T>* tw, const cpx<T
         if (v.z_alg == 3) return v.z_pf ? go(I1{}, I1{}) : go(I0{}, I1{});
         return v.z_pf ? go(I1{}, I2{}) : go(I0{}, I2{});
       }
+    }
+    return false;
+  }
+  if (v.z_alg == 5) {  // row pairs
+    using PP = typename ZRow<LL, T>::P;
+    constexpr int NT5 = PP::L / PP::rad[0];
+    if constexpr (lds_fits<T, Lay<PP::L / PP::rad[PP::P - 1], 1>>(PP::L)) {
+      const dim3 nbr = bt ? dim3(bt->max_nr * g.ntp / 2, bt->count) : dim3(g.nlv * g.ntp / 2);
+      // the plan's twiddles follow the half-length and the pair plans'
+      const cpx<T>* twr = tw + zrow_tw<LL>();
+      if (v.z_pf)
+        zpass5_ct<T, 1, PP, BAT><<<nbr, NT5, 0, s>>>(g, twr, r, W, ws, Y, tab);
+      else
+        zpass5_ct<T, 0, PP, BAT><<<nbr, NT5, 0, s>>>(g, twr, r, W, ws, Y, tab);
+      return true;
     }
     return false;
   }

@@ -18,13 +18,6 @@ bool ct_has_theta(int L) {
 #undef X
   return false;
 }
-// the register form of the z pass (one first-pass butterfly per thread of 256)
-bool ct_has_zreg(int L) {
-#define X(LL, ...) if (L == LL) return LL / __VA_ARGS__::rad[0] <= 256;
-  NSP_ZHALF_PLANS(X)
-#undef X
-  return false;
-}
 bool ct_has_zhalf(int L) {
 #define X(LL, ...) if (L == LL) return true;
   NSP_ZHALF_PLANS(X)
@@ -54,6 +47,19 @@ std::vector<int> ct_pair_radices(int nh) {
     return std::vector<int>(PP::rad, PP::rad + PP::P);                             \
   }
   NSP_ZPAIR_PLANS(X)
+#undef X
+  return {};
+}
+// radix list of the row-pair form's plan for half length NH (empty if none)
+std::vector<int> ct_row_radices(int nh, bool f32) {
+#define X(LL, ...)                                                                 \
+  if (nh == LL) {                                                                  \
+    using P32 = typename ZRow<LL, float>::P;                                       \
+    using P64 = typename ZRow<LL, double>::P;                                      \
+    return f32 ? std::vector<int>(P32::rad, P32::rad + P32::P)                     \
+               : std::vector<int>(P64::rad, P64::rad + P64::P);                    \
+  }
+  NSP_ZROW_PLANS(X)
 #undef X
   return {};
 }

@@ -247,12 +247,13 @@ struct NlVariant {
   ThetaVar inv, fwd;
   int z_alg;   // z pass: 0 LDS-scatter form, 1 register form (256 threads), 2 register form with the
                // inverse transforms in triples, 3 pair form (two real transforms as one full-length
-               // complex transform), 4 pair form with two rows per workgroup
+               // complex transform), 4 pair form with two rows per workgroup, 5 row-pair form (a field's
+               // real transforms on two rows as one full-length complex transform)
   int z_nthr;  // scatter form: threads per row (256 or 512)
   int z_pad;   // scatter form: 1 = one LDS slot per 16 elements, 2 = row padding as the register form;
                // triples: row padding of the three-column layout 0, 1 or R0 slots; pairs: row
                // padding 0, 1 or R0 slots
-  int z_pf;    // register and pair forms: load the next transform's inputs before the LDS passes
+  int z_pf;    // register, pair and row-pair forms: load the next transform's inputs before the LDS passes
   int s_ord;   // linear sweep: 1 = the chunks of an azimuthal row XCD-contiguous, 0 = dispatch order
   int nl_chunks;  // nonlinear stage: 1 = stage after stage; K > 1 = the theta inverse and the z pass
                   // in K level chunks on two streams, the z pass of chunk c overlapping the theta
@@ -354,9 +355,9 @@ struct Profiler {
 // Compiled-plan support (nonlinear_ct64.hip).
 bool ct_has_theta(int L);
 bool ct_has_zhalf(int L);
-bool ct_has_zreg(int L);
 std::vector<int> ct_radices(int L, bool theta);
 std::vector<int> ct_pair_radices(int nh);
+std::vector<int> ct_row_radices(int nh, bool f32);
 // per-pass twiddles of a plan: for each pass (radix R, sub-length S) S*(R-1)
 // entries exp(-2 pi i q k / (S R)) at [k*(R-1) + q-1]
 std::vector<double2> pass_twiddles(const std::vector<int>& radices);

@@ -267,6 +267,30 @@ def test_mixed_forms_keep_fp32_accuracy():
     assert not bad, bad
 
 
+@pytest.mark.parametrize("prec,tol", [(nsp.FP64, 1e-12), (nsp.MIXED, 1e-6)], ids=["fp64", "mixed"])
+@pytest.mark.parametrize("nz", [65, 385, 513, 1025, 1537, 3073])
+def test_row_pair_z_pass(nz, prec, tol):
+    """The row-pair z pass of every compiled axial plan, with and without
+    prefetch, against the oracle; after an evaluation of another field, so
+    that nothing of an earlier one is left in the transform buffers' padding."""
+    shape = dict(nr=8, nt=64, nz=nz, lz=4 * np.pi, re=2000.0, dt=0.005)
+    print(f"[gpu] row-pair z pass {shape} precision {prec}", flush=True)
+    p = nsp.Pipe(**shape, precision=prec)
+    o = Oracle(**shape)
+    p.seeded_ic(SEED1, 20, nz - 2, 0, 0.1)
+    other = p.get_state()
+    p.seeded_ic(SEED1 + 1, 31, nz - 2, 1, 0.1)
+    u = p.get_state()
+    b = o.nonlinear(*u)
+    for pf in (0, 1):
+        p.set_tuning(dict(theta_inv=dict(alg=0, tl=8, nthr=256, pad=0, ord=1),
+                          theta_fwd=dict(alg=0, tl=8, nthr=256, pad=0, ord=1),
+                          z_alg=5, z_nthr=256, z_pad=0, z_pf=pf))
+        p.nonlinear(*other)
+        fields_close(p.nonlinear(*u), b, tol)
+    p.close()
+
+
 # the longest compiled plans: theta 1152 (NT = 768) and half-z 4608 (NZ = 3073)
 LONG = [dict(nr=8, nt=768, nz=65, lz=4 * np.pi, re=19000.0, dt=0.0005),
         dict(nr=8, nt=64, nz=3073, lz=4 * np.pi, re=19000.0, dt=0.0005)]
