@@ -284,14 +284,36 @@ nsp_status nsp_default_params(nsp_params* p, int nr, int nt, int nz, double lz, 
 }
 
 // The kernel forms of a pipe that has not been tuned, by transform length and
-// precision.  z pass: the row-pair form, the fastest of those that keep the
-// accuracy of one transform per field (the figures are at zpass5_ct).  Loading
-// the next field during the LDS passes pays except where its registers take
-// a workgroup off the CU (FP32 rows of 4608: 1.32 against 1.56 ms for 24 x 576
+// precision (members of an ensemble class share both).
+//
+// z pass: the row-pair form, the fastest of those that keep the accuracy of
+// one transform per field (the figures are at zpass5_ct).  Loading the next
+// field during the LDS passes pays except where its registers take a
+// workgroup off the CU (FP32 rows of 4608: 1.32 against 1.56 ms for 24 x 576
 // rows; rows of 9216: no gain).
+//
+// theta inverse: 16 columns per block (128-byte runs of W in FP32), on as many
+// threads as keep the transforms' inputs in registers; 8 columns where a
+// 16-column tile does not fit LDS (FP64, 1152).  16 against 8 columns, with the
+// radial derivative, ms: FP32 48x96x513 0.141 / 0.162, 64x192x385 0.294 / 0.329,
+// 96x384x1537 3.13 / 3.3, 24x768x3073 3.46 / 3.87; FP64 96x384x1537 4.89 / 5.03,
+// 64x192x385 equal.
+//
+// theta forward: the register form; 16 columns where its inputs fit the
+// registers (FP32 up to 576, FP64 up to 144), else 8.  Against the scatter form
+// with 8 columns, ms: FP32 24x768x3073 0.79 / 1.86, 64x192x385 0.057 / 0.080;
+// FP64 64x192x385 0.125 / 0.175, 32x64x65 0.010 / 0.026.
 static NlVariant default_variant(const Geom& g, bool mixed) {
   const int pf = g.nh <= 1536 || (g.nh <= 2304 && !mixed) ? 1 : 0;
-  return NlVariant{ThetaVar{0, 8, 256, 0, 1}, ThetaVar{0, 8, 256, 0, 1}, 5, 256, 0, pf, 1, 1};
+  ThetaVar inv{0, 16, 256, 0, 1}, fwd{1, 8, 256, 0, 1};
+  if (g.ntp > 576) {
+    if (mixed) inv.nthr = 1024;
+    else inv.tl = 8;
+  } else if (g.ntp > 192) {
+    inv.nthr = 512;
+  }
+  if (g.ntp <= (mixed ? 576 : 144)) fwd.tl = 16;
+  return NlVariant{inv, fwd, 5, 256, 0, pf, 1, 1};
 }
 
 // share: a handle with identical parameters whose operator data (LU factors,
