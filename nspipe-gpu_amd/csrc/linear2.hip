@@ -238,6 +238,8 @@ template <>
 struct Scr<false> {
   double2* p;
   __device__ static Scr at(double2* base, size_t) { return Scr{base}; }
+  using V = double2;
+  __device__ V raw(size_t i) const { return p[i]; }
   __device__ double2 ld(size_t i) const { return p[i]; }
   __device__ void st(size_t i, double2 v) const { p[i] = v; }
 };
@@ -245,11 +247,68 @@ template <>
 struct Scr<true> {
   float2* p;
   __device__ static Scr at(double2* base, size_t region0) { return Scr{reinterpret_cast<float2*>(base) + region0}; }
+  using V = float2;
+  __device__ V raw(size_t i) const { return p[i]; }
   __device__ double2 ld(size_t i) const {
     const float2 v = p[i];
     return make_double2(v.x, v.y);
   }
   __device__ void st(size_t i, double2 v) const { p[i] = make_float2(float(v.x), float(v.y)); }
+};
+
+__device__ __forceinline__ double2 wide(double2 v) { return v; }
+__device__ __forceinline__ double2 wide(float2 v) { return make_double2(v.x, v.y); }
+
+constexpr int kLatRing = 3;
+
+// Walks rows t0, t0 + DIR, ... (t1 excluded) whose first PD are loaded in ring.
+template <int PD, int DIR, typename Row, typename L, typename F>
+__device__ __forceinline__ void walk_ring(Row (&ring)[PD], int t0, int t1, L&& load, F&& work) {
+  int t = t0;
+  for (; DIR * (t1 - t) >= PD; t += DIR * PD) {
+#pragma unroll
+    for (int q = 0; q < PD; q++) {
+      const Row cur = ring[q];
+      load(t + DIR * (q + PD), ring[q]);
+      work(t + DIR * q, cur);
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < PD - 1; q++)
+    if (DIR * (t1 - t) > q) work(t + DIR * q, ring[q]);
+}
+
+// Walks rows t0, t0 + DIR, ... (t1 excluded): load(t, row) issues a row's loads
+// (it clamps rows beyond the grid), work(t, row) does its arithmetic and
+// stores.  PD = 0 loads each row as it is reached; PD > 0 keeps the loads of
+// PD rows in flight (a ring of rows in registers).
+template <int PD, int DIR, typename Row, typename L, typename F>
+__device__ __forceinline__ void walk_rows(int t0, int t1, L&& load, F&& work) {
+  if constexpr (PD == 0) {
+    for (int t = t0; t != t1; t += DIR) {
+      Row r;
+      load(t, r);
+      work(t, r);
+    }
+  } else {
+    Row ring[PD];
+#pragma unroll
+    for (int q = 0; q < PD; q++) load(t0 + DIR * q, ring[q]);
+    walk_ring<PD, DIR>(ring, t0, t1, load, work);
+  }
+}
+// A radial table: through the scalar cache, or (LAT kernels) from LDS.
+template <int LAT>
+struct Tab {
+  ctab g;
+  __device__ double operator[](int i) const { return g[i]; }
+  __device__ Tab operator+(int o) const { return Tab{g + o}; }
+};
+template <>
+struct Tab<1> {
+  const double* l;
+  __device__ double operator[](int i) const { return l[i]; }
+  __device__ Tab operator+(int o) const { return Tab{l + o}; }
 };
 
 // ------------------------------------------------------------------ sweep
@@ -275,8 +334,19 @@ struct Scr<true> {
 //   C:   wall rows -u^n (so that u^n + delta vanishes there);
 //   D:   back substitution gives delta; u^n + delta takes the place of the
 //        solution from there on (wall divergence, correction, output).
-template <int PASS, int PRED, int B, int HOLD = 0, int INC = 0>
+// LAT = 1 (grids with few workgroups, Lin2Args::lat): the walk is bound by the
+// latency of each row's loads and of its arithmetic, not by bandwidth, and
+// registers cost nothing (less than one wave per SIMD).  Each pass then keeps
+// the loads of kLatRing rows in flight, reads the radial tables from an LDS
+// copy (a first touch of a table row through the scalar cache is another
+// memory round trip per row) and multiplies by tabled 1/r.  Pass D holds the
+// wall rows (as HOLD = 1).  Sweeps, predictor / corrector, us: 32x64x65 FP64
+// 139 / 155 -> 117 / 117, 45x80x161 FP64 238 / 278 -> 154 / 189, 24x64x385
+// FP64 152 / 175 -> 108 / 126 and refined 161 / 148 -> 121 / 121, 64x64x513
+// mixed 370 / 409 -> 307 / 359 (a ring of 2 rows is equal, of 1 or 4 slower).
+template <int PASS, int PRED, int B, int HOLD = 0, int INC = 0, int LAT = 0>
 __global__ __launch_bounds__(128) void sweep_kernel(Lin2Args A, const Lin2Args* tab) {
+  extern __shared__ double lat_tab[];  // LAT: 1/r [nr], D [2][nr][7], Lu [2][nr][7]
   if constexpr (B != 0) {
     A = tab[blockIdx.y];
     A.r = gmem(tab, A.r);
@@ -298,7 +368,8 @@ __global__ __launch_bounds__(128) void sweep_kernel(Lin2Args A, const Lin2Args* 
     A.SR = gmem(tab, A.SR);
     A.SP = gmem(tab, A.SP);
     A.norm = gmem(tab, A.norm);
-    if constexpr (PASS == 3) {  // members of the other form are the other launch's
+    if (A.lat != LAT) return;  // members of the other kind are the other launch's
+    if constexpr (PASS == 3 && !LAT) {  // so are members of the other form
       // The form is tested on a copy the compiler cannot see through: knowing
       // the form past this test would let it drop the other form's paths
       // and then contract the remaining arithmetic differently from the
@@ -318,6 +389,15 @@ __global__ __launch_bounds__(128) void sweep_kernel(Lin2Args A, const Lin2Args* 
   const int nth = g.nt / 2;
   const int it = (threadIdx.x < 64) ? pair : (pair == 0 ? nth : g.nt - pair);
   const int l = ch * 64 + (threadIdx.x & 63);
+  if constexpr (LAT) {
+    const int n7 = 2 * STEN * g.nr;
+    for (int e = threadIdx.x; e < g.nr; e += 128) lat_tab[e] = 1.0 / A.r[e];
+    for (int e = threadIdx.x; e < n7; e += 128) {
+      lat_tab[g.nr + e] = A.Dc[e];
+      lat_tab[g.nr + n7 + e] = A.Luc[e];
+    }
+    __syncthreads();
+  }
   if (l >= g.nz) return;
   const int k = it * g.nz + l;
   const ModeQ q = modeq(g, k);
@@ -352,9 +432,33 @@ __global__ __launch_bounds__(128) void sweep_kernel(Lin2Args A, const Lin2Args* 
   // NT/2), and the row index of a pass is uniform.
   const int par_u = __builtin_amdgcn_readfirstlane(abs((abs(q.m) % 2) - 1));  // parity table of ur, ut (u+, u-)
   const int par_p = 1 - par_u;                                                 // parity table of uz, p
-  const ctab Dcu = ctab(A.Dc) + par_u * STEN * nr;
-  const ctab Dcp = ctab(A.Dc) + par_p * STEN * nr;
-  const ctab rt = ctab(A.r);
+  using TB = Tab<LAT>;
+  TB rt, Dt, Lt;
+  if constexpr (LAT) {
+    rt.l = lat_tab;
+    Dt.l = lat_tab + nr;
+    Lt.l = lat_tab + nr + 2 * STEN * nr;
+  } else {
+    rt.g = ctab(A.r);
+    Dt.g = ctab(A.Dc);
+    Lt.g = ctab(A.Luc);
+  }
+  // x / r and x / r^2 at row i: the LAT kernels multiply by the tabled
+  // reciprocal (an IEEE division is a chain of a dozen dependent instructions)
+  auto over_r = [&](double x, int i) -> double {
+    if constexpr (LAT) return x * rt[i];
+    else return x / rt[i];
+  };
+  auto over_r2 = [&](double x, int i) -> double {
+    if constexpr (LAT) {
+      return x * (rt[i] * rt[i]);
+    } else {
+      const double r2 = rt[i] * rt[i];
+      return x / r2;
+    }
+  };
+  const TB Dcu = Dt + par_u * STEN * nr;
+  const TB Dcp = Dt + par_p * STEN * nr;
   const double2 z2 = make_double2(0.0, 0.0);
   // Column scratch precision of this workgroup: the mixed form holds SR, SP
   // and E of |m| >= m32 as FP32 pairs (the rhs, eliminated rows and pressure
@@ -372,6 +476,11 @@ __global__ __launch_bounds__(128) void sweep_kernel(Lin2Args A, const Lin2Args* 
   const Scr<S32> SR = Scr<S32>::at(A.SR, (size_t)lb * nr * 384);
   const Scr<S32> SP = Scr<S32>::at(A.SP, (size_t)lb * nr * 128);
   const Scr<S32> E = Scr<S32>::at(A.E, (size_t)lb * nr * 384);
+  using SV = typename Scr<S32>::V;
+  using NV = std::conditional_t<N32, float2, double2>;
+  using FT = std::conditional_t<F32W, float, double>;
+  const NV* const Nv = reinterpret_cast<const NV*>(A.N);
+  auto row_of = [&](int t) { return t < 0 ? 0 : (t < nr ? t : nr - 1); };
 
   // ============================== pass A1 (up, INC predictor): E', Dh
   if constexpr (PASS == 4) {
@@ -388,17 +497,25 @@ __global__ __launch_bounds__(128) void sweep_kernel(Lin2Args A, const Lin2Args* 
 #pragma unroll
     for (int w = 0; w < 4; w++) Ht[w] = Hz[w] = z2;
     const double ire = 1.0 / g.re, aim = d_im / g.re, idt = 1.0 / g.dt;
-    for (int t = 0; t < nr + 6; t++) {
+    struct Row1 {
+      double2 u[3];  // u^n row t
+      NV n[3];       // N(u^n) row t - 3
+    };
+    auto load1 = [&](int t, Row1& R) {
+      const size_t h = (size_t)row_of(t) * MS + k, hn = nb0 + (size_t)row_of(t - 3) * npl;
+#pragma unroll
+      for (int c = 0; c < 3; c++) {
+        R.u[c] = A.u[c * n + h];
+        R.n[c] = Nv[c * ncs + hn];
+      }
+    };
+    auto work1 = [&](int t, const Row1& R) {
       double2 a = z2, b = z2, c = z2;
-      {  // row t, or zero past the wall: the loads themselves stay in bounds
-        const size_t h = (size_t)(t < nr ? t : nr - 1) * MS + k;
-        const double2 a0 = A.u[h], b0 = A.u[n + h], c0 = A.u[2 * n + h];
-        if (t < nr) {
-          a = a0;
-          b = b0;
-          c = c0;
-          pm_of(a, b);
-        }
+      if (t < nr) {  // zero past the wall
+        a = R.u[0];
+        b = R.u[1];
+        c = R.u[2];
+        pm_of(a, b);
       }
 #pragma unroll
       for (int w = 0; w < 6; w++) {
@@ -412,25 +529,12 @@ __global__ __launch_bounds__(128) void sweep_kernel(Lin2Args A, const Lin2Args* 
       const int j = t - 3;  // row whose 7-point window is complete
       double2 H0 = z2, H1 = z2, H2 = z2;
       if (j >= 0 && j < nr) {
-        const size_t hn = nb0 + (size_t)j * npl;  // tile-major N(u^n)
-        double2 nn[3];
-        if constexpr (N32) {
-          const float2* N32 = reinterpret_cast<const float2*>(A.N);
-          const float2 f0 = N32[hn], f1 = N32[ncs + hn], f2 = N32[2 * ncs + hn];
-          nn[0] = make_double2(f0.x, f0.y);
-          nn[1] = make_double2(f1.x, f1.y);
-          nn[2] = make_double2(f2.x, f2.y);
-        } else {
-          nn[0] = A.N[hn];
-          nn[1] = A.N[ncs + hn];
-          nn[2] = A.N[2 * ncs + hn];
-        }
+        double2 nn[3] = {wide(R.n[0]), wide(R.n[1]), wide(R.n[2])};
         pm_of(nn[0], nn[1]);
-        const double rj = rt[j], r2 = rj * rj;
         double2 hu[3];
 #pragma unroll
         for (int cc = 0; cc < 3; cc++) {  // L'u^n as in addLap_k (mod_linear.cu:12-51)
-          const ctab Lc = ctab(A.Luc) + ((cc < 2) ? par_u : par_p) * STEN * nr + STEN * j;
+          const TB Lc = Lt + (((cc < 2) ? par_u : par_p) * STEN * nr + STEN * j);
           double px = 0.0, py = 0.0;
 #pragma unroll
           for (int w = 0; w < 7; w++) {
@@ -438,9 +542,9 @@ __global__ __launch_bounds__(128) void sweep_kernel(Lin2Args A, const Lin2Args* 
             py += Lc[w] * uw[cc][w].y;
           }
           const double2 aux = uw[cc][3];
-          double de = -q.kz * q.kz - q.kt * q.kt / r2;
-          if (cc == 0) de += -(1.0 / r2) - (2.0 * q.kt / r2);
-          else if (cc == 1) de += -(1.0 / r2) + (2.0 * q.kt / r2);
+          double de = -q.kz * q.kz - over_r2(q.kt * q.kt, j);
+          if (cc == 0) de += -over_r2(1.0, j) - over_r2(2.0 * q.kt, j);
+          else if (cc == 1) de += -over_r2(1.0, j) + over_r2(2.0 * q.kt, j);
           px += de * aux.x;
           py += de * aux.y;
           E.st(sb3 + (size_t)j * 384 + cc * 128,
@@ -466,26 +570,26 @@ __global__ __launch_bounds__(128) void sweep_kernel(Lin2Args A, const Lin2Args* 
       if (i >= 0 && i < nr) {  // div_k (mod_radialFD.cu:67-96) of H u^n, wall row zero
         double2 dv = z2;
         if (i < nr - 1) {
-          const ctab Dr = Dcu + STEN * i;
+          const TB Dr = Dcu + STEN * i;
           double px = 0.0, py = 0.0;
 #pragma unroll
           for (int w = 0; w < 7; w++) {
             px += Dr[w] * Hr[w].x;
             py += Dr[w] * Hr[w].y;
           }
-          const double rK = rt[i];
           const double2 ur = Hr[3], ut = Ht[0], uz = Hz[0];
-          px += ur.x / rK;
-          py += ur.y / rK;
-          px += -q.kt * ut.y / rK;
-          py += q.kt * ut.x / rK;
+          px += over_r(ur.x, i);
+          py += over_r(ur.y, i);
+          px += over_r(-q.kt * ut.y, i);
+          py += over_r(q.kt * ut.x, i);
           px += -q.kz * uz.y;
           py += q.kz * uz.x;
           dv = make_double2(px, py);
         }
         DH.st(sb1 + (size_t)i * 128, dv);
       }
-    }
+    };
+    walk_rows<LAT ? kLatRing : 0, 1, Row1>(0, nr + 6, load1, work1);
   }
 
   // ============================== pass A (up)
@@ -508,18 +612,42 @@ __global__ __launch_bounds__(128) void sweep_kernel(Lin2Args A, const Lin2Args* 
 #pragma unroll
     for (int w = 0; w < 3; w++) yp[w] = z2;
     const double cn = (1.0 - d_im) / g.re, idt = 1.0 / g.dt;
-    for (int t = 0; t < nr + LAG; t++) {
+    // A row's loads are issued together before its stores, which the compiler
+    // would not move loads across (one memory round trip per row)
+    struct RowA {
+      double2 u[3];  // predictor: u^n row t
+      NV n[3];       // N(u) row j
+      SV e[3];       // E row j
+      double fl[3];  // pressure L factors of row i = j - 3
+      SV dh;         // INC: Dh row i
+    };
+    auto loada = [&](int t, RowA& R) {
+      const int j = XPRED ? t - 3 : t;
+      const size_t hn = nb0 + (size_t)row_of(j) * npl;  // tile-major N(u)
+      if constexpr (XPRED) {
+        const size_t h = (size_t)row_of(t) * MS + k;
+#pragma unroll
+        for (int c = 0; c < 3; c++) R.u[c] = A.u[c * n + h];
+      } else {
+        const size_t he = sb3 + (size_t)row_of(j) * 384;
+#pragma unroll
+        for (int c = 0; c < 3; c++) R.e[c] = E.raw(he + c * 128);
+      }
+      const double* fpi = A.F + fb_p + (size_t)row_of(j - 3) * FR_ABS;
+#pragma unroll
+      for (int w = 0; w < 3; w++) R.fl[w] = fpi[w * 64];
+      if constexpr (INC) R.dh = DH.raw(sb1 + (size_t)row_of(j - 3) * 128);
+#pragma unroll
+      for (int c = 0; c < 3; c++) R.n[c] = Nv[c * ncs + hn];
+    };
+    auto worka = [&](int t, const RowA& R) {
       if (XPRED) {
         double2 a = z2, b = z2, c = z2;
-        {  // row t, or zero past the wall: the loads themselves stay in bounds
-          const size_t h = (size_t)(t < nr ? t : nr - 1) * MS + k;
-          const double2 a0 = A.u[h], b0 = A.u[n + h], c0 = A.u[2 * n + h];
-          if (t < nr) {
-            a = a0;
-            b = b0;
-            c = c0;
-            pm_of(a, b);
-          }
+        if (t < nr) {  // zero past the wall
+          a = R.u[0];
+          b = R.u[1];
+          c = R.u[2];
+          pm_of(a, b);
         }
 #pragma unroll
         for (int w = 0; w < 6; w++) {
@@ -533,39 +661,19 @@ __global__ __launch_bounds__(128) void sweep_kernel(Lin2Args A, const Lin2Args* 
       }
       // rhs row j
       const int j = XPRED ? t - 3 : t;
-      // pressure elimination row i = j - 3: its factors (and Dh) are loaded
-      // before this iteration's stores, which the compiler would not move
-      // loads across (one memory round trip per row instead of two)
-      const int i = j - 3;
-      const int ic = i < 0 ? 0 : (i < nr ? i : nr - 1);
-      const double* fpi = A.F + fb_p + (size_t)ic * FR_ABS;
-      const double fl0 = fpi[0], fl1 = fpi[64], fl2 = fpi[128];
-      double2 dhi = z2;
-      if constexpr (INC) dhi = DH.ld(sb1 + (size_t)ic * 128);
+      const int i = j - 3;  // pressure elimination row
       double2 R0 = z2, R1 = z2, R2 = z2;
       if (j >= 0 && j < nr) {
-        const size_t hn = nb0 + (size_t)j * npl;  // tile-major N(u)
-        double2 n0, n1, n2;
-        if constexpr (N32) {
-          const float2* N32 = reinterpret_cast<const float2*>(A.N);
-          const float2 f0 = N32[hn], f1 = N32[ncs + hn], f2 = N32[2 * ncs + hn];
-          n0 = make_double2(f0.x, f0.y);
-          n1 = make_double2(f1.x, f1.y);
-          n2 = make_double2(f2.x, f2.y);
-        } else {
-          n0 = A.N[hn];
-          n1 = A.N[ncs + hn];
-          n2 = A.N[2 * ncs + hn];
-        }
+        double2 n0 = wide(R.n[0]), n1 = wide(R.n[1]);
+        const double2 n2 = wide(R.n[2]);
         pm_of(n0, n1);
         double2 rh[3];
         if (XPRED) {
           // addLap_k (mod_linear.cu:12-51) on u^n, then rhs = N + that
-          const double rj = rt[j], r2 = rj * rj;
-          const double2 nn[3] = {n0, n1, n2};
+            const double2 nn[3] = {n0, n1, n2};
 #pragma unroll
           for (int c = 0; c < 3; c++) {
-            const ctab Lc = ctab(A.Luc) + ((c < 2) ? par_u : par_p) * STEN * nr + STEN * j;
+            const TB Lc = Lt + (((c < 2) ? par_u : par_p) * STEN * nr + STEN * j);
             double px = 0.0, py = 0.0;
 #pragma unroll
             for (int w = 0; w < 7; w++) {
@@ -573,9 +681,9 @@ __global__ __launch_bounds__(128) void sweep_kernel(Lin2Args A, const Lin2Args* 
               py += Lc[w] * uw[c][w].y;
             }
             const double2 aux = uw[c][3];
-            double de = -q.kz * q.kz - q.kt * q.kt / r2;
-            if (c == 0) de += -(1.0 / r2) - (2.0 * q.kt / r2);
-            else if (c == 1) de += -(1.0 / r2) + (2.0 * q.kt / r2);
+            double de = -q.kz * q.kz - over_r2(q.kt * q.kt, j);
+            if (c == 0) de += -over_r2(1.0, j) - over_r2(2.0 * q.kt, j);
+            else if (c == 1) de += -over_r2(1.0, j) + over_r2(2.0 * q.kt, j);
             px += de * aux.x;
             py += de * aux.y;
             px *= cn;
@@ -587,8 +695,7 @@ __global__ __launch_bounds__(128) void sweep_kernel(Lin2Args A, const Lin2Args* 
                  make_double2(px + (1.0 - d_im) * nn[c].x, py + (1.0 - d_im) * nn[c].y));
           }
         } else {
-          const size_t he = sb3 + (size_t)j * 384;
-          const double2 e0 = E.ld(he), e1 = E.ld(he + 128), e2 = E.ld(he + 256);
+          const double2 e0 = wide(R.e[0]), e1 = wide(R.e[1]), e2 = wide(R.e[2]);
           rh[0] = make_double2(e0.x + d_im * n0.x, e0.y + d_im * n0.y);
           rh[1] = make_double2(e1.x + d_im * n1.x, e1.y + d_im * n1.y);
           rh[2] = make_double2(e2.x + d_im * n2.x, e2.y + d_im * n2.y);
@@ -616,28 +723,28 @@ __global__ __launch_bounds__(128) void sweep_kernel(Lin2Args A, const Lin2Args* 
       if (i >= 0 && i < nr) {
         double2 dv = z2;
         if (i < nr - 1) {  // div_k (mod_radialFD.cu:67-96), wall row zero
-          const ctab Dr = Dcu + STEN * i;
+          const TB Dr = Dcu + STEN * i;
           double px = 0.0, py = 0.0;
 #pragma unroll
           for (int w = 0; w < 7; w++) {
             px += Dr[w] * Rr[w].x;
             py += Dr[w] * Rr[w].y;
           }
-          const double rK = rt[i];
           const double2 ur = Rr[3], ut = Rt[0], uz = Rz[0];
-          px += ur.x / rK;
-          py += ur.y / rK;
-          px += -q.kt * ut.y / rK;
-          py += q.kt * ut.x / rK;
+          px += over_r(ur.x, i);
+          py += over_r(ur.y, i);
+          px += over_r(-q.kt * ut.y, i);
+          py += over_r(q.kt * ut.x, i);
           px += -q.kz * uz.y;
           py += q.kz * uz.x;
           dv = make_double2(px, py);
           if constexpr (INC) {  // div(rhs) = div(rhs - H u^n) + div(H u^n)
+            const double2 dhi = wide(R.dh);
             dv.x += dhi.x;
             dv.y += dhi.y;
           }
         }
-        const double l0 = fl0, l1 = fl1, l2 = fl2;
+        const double l0 = R.fl[0], l1 = R.fl[1], l2 = R.fl[2];
         dv.x -= l0 * yp[0].x;
         dv.y -= l0 * yp[0].y;
         dv.x -= l1 * yp[1].x;
@@ -649,7 +756,8 @@ __global__ __launch_bounds__(128) void sweep_kernel(Lin2Args A, const Lin2Args* 
         yp[1] = yp[2];
         yp[2] = dv;
       }
-    }
+    };
+    walk_rows<LAT ? kLatRing : 0, 1, RowA>(0, nr + LAG, loada, worka);
   }
 
   // ============================== pass B (down)
@@ -657,12 +765,19 @@ __global__ __launch_bounds__(128) void sweep_kernel(Lin2Args A, const Lin2Args* 
     double2 pw[3];  // p rows t+1..t+3
 #pragma unroll
     for (int w = 0; w < 3; w++) pw[w] = z2;
-    for (int t = nr - 1; t >= 0; t--) {
-      const double* fp = A.F + fb_p + (size_t)t * FR_ABS;
-      const double ru = fp[3 * 64];
-      const double u1 = fp[4 * 64], u2 = fp[5 * 64], u3 = fp[6 * 64];
-      const size_t h = sb1 + (size_t)t * 128;
-      double2 x = SP.ld(h);
+    struct RowB {
+      double f[4];  // 1/U_ii, U1..U3
+      SV x;
+    };
+    auto loadb = [&](int t, RowB& R) {
+      const double* fp = A.F + fb_p + (size_t)row_of(t) * FR_ABS;
+#pragma unroll
+      for (int w = 0; w < 4; w++) R.f[w] = fp[(3 + w) * 64];
+      R.x = SP.raw(sb1 + (size_t)row_of(t) * 128);
+    };
+    auto workb = [&](int t, const RowB& R) {
+      const double ru = R.f[0], u1 = R.f[1], u2 = R.f[2], u3 = R.f[3];
+      double2 x = wide(R.x);
       x.x -= u1 * pw[0].x;
       x.y -= u1 * pw[0].y;
       x.x -= u2 * pw[1].x;
@@ -670,11 +785,12 @@ __global__ __launch_bounds__(128) void sweep_kernel(Lin2Args A, const Lin2Args* 
       x.x -= u3 * pw[2].x;
       x.y -= u3 * pw[2].y;
       const double2 pn = make_double2(x.x * ru, x.y * ru);
-      SP.st(h, pn);
+      SP.st(sb1 + (size_t)t * 128, pn);
       pw[2] = pw[1];
       pw[1] = pw[0];
       pw[0] = pn;
-    }
+    };
+    walk_rows<LAT ? 8 : 0, -1, RowB>(nr - 1, -1, loadb, workb);
   }
 
   // ============================== pass C (up)
@@ -687,48 +803,52 @@ __global__ __launch_bounds__(128) void sweep_kernel(Lin2Args A, const Lin2Args* 
       for (int w = 0; w < 3; w++) yw[c][w] = z2;
 #pragma unroll
     for (int w = 0; w < 7; w++) pw[w] = z2;
-    for (int t = 0; t < nr + IW; t++) {
-#pragma unroll
-      for (int w = 0; w < 6; w++) pw[w] = pw[w + 1];
-      {  // row t, or zero past the wall: the load itself stays in bounds
-        const double2 pv = SP.ld(sb1 + (size_t)(t < nr ? t : nr - 1) * 128);
-        pw[6] = (t < nr) ? pv : z2;
-      }
-      const int j = t - IW;
-      if (j < 0) continue;
-      // the L factors of the three solves at row j, loaded before the
-      // row's stores (the compiler does not move loads across them)
-      double Lc3[3][IW];
+    // the L factors of the three solves at row j and its rhs are loaded before
+    // the row's stores (the compiler does not move loads across them)
+    struct RowC {
+      SV p;             // p row t
+      FT lc[3][IW];     // L factors row j = t - 3
+      SV r[3];          // rhs row j
+    };
+    auto loadc = [&](int t, RowC& R) {
+      R.p = SP.raw(sb1 + (size_t)row_of(t) * 128);
+      const int j = row_of(t - IW);
 #pragma unroll
       for (int c = 0; c < 3; c++) {
         // u+, u-: rows of FR_UP, slots of 128; uz: rows of FR_ABS, slots of 64
         const size_t fo = c == 0 ? fb_up + (size_t)j * FR_UP
                                  : (c == 1 ? fb_um + (size_t)j * FR_UP : fb_uz + (size_t)j * FR_ABS);
         const int fs = c == 2 ? 64 : 128;
-        if constexpr (F32W) {
 #pragma unroll
-          for (int w = 0; w < IW; w++) Lc3[c][w] = A.F32[fo + w * fs];
-        } else {
-#pragma unroll
-          for (int w = 0; w < IW; w++) Lc3[c][w] = A.F[fo + w * fs];
+        for (int w = 0; w < IW; w++) {
+          if constexpr (F32W) R.lc[c][w] = A.F32[fo + w * fs];
+          else R.lc[c][w] = A.F[fo + w * fs];
         }
       }
+#pragma unroll
+      for (int c = 0; c < 3; c++) R.r[c] = SR.raw(sb3 + (size_t)j * 384 + c * 128);
+    };
+    auto workc = [&](int t, const RowC& R) {
+#pragma unroll
+      for (int w = 0; w < 6; w++) pw[w] = pw[w + 1];
+      pw[6] = (t < nr) ? wide(R.p) : z2;  // zero past the wall
+      const int j = t - IW;
+      if (j < 0) return;
       // addGrad_k (mod_radialFD.cu:115-143)
       const size_t h = sb3 + (size_t)j * 384;
-      const ctab Dr = Dcp + STEN * j;
+      const TB Dr = Dcp + STEN * j;
       double px = 0.0, py = 0.0;
 #pragma unroll
       for (int w = 0; w < 7; w++) {
         px += Dr[w] * pw[w].x;
         py += Dr[w] * pw[w].y;
       }
-      const double rK = rt[j];
       const double2 ph = pw[3];
-      double2 rh[3] = {SR.ld(h), SR.ld(h + 128), SR.ld(h + 256)};
+      double2 rh[3] = {wide(R.r[0]), wide(R.r[1]), wide(R.r[2])};
       rh[0].x -= px;
       rh[0].y -= py;
-      rh[1].x -= -q.kt * ph.y / rK;
-      rh[1].y -= q.kt * ph.x / rK;
+      rh[1].x -= over_r(-q.kt * ph.y, j);
+      rh[1].y -= over_r(q.kt * ph.x, j);
       rh[2].x -= -q.kz * ph.y;
       rh[2].y -= q.kz * ph.x;
       pm_of(rh[0], rh[1]);
@@ -746,7 +866,7 @@ __global__ __launch_bounds__(128) void sweep_kernel(Lin2Args A, const Lin2Args* 
       }
 #pragma unroll
       for (int c = 0; c < 3; c++) {  // forward elimination
-        const double* Lc = Lc3[c];
+        const double Lc[IW] = {R.lc[c][0], R.lc[c][1], R.lc[c][2]};
         double2 y = rh[c];
         y.x -= Lc[0] * yw[c][0].x;
         y.y -= Lc[0] * yw[c][0].y;
@@ -759,7 +879,8 @@ __global__ __launch_bounds__(128) void sweep_kernel(Lin2Args A, const Lin2Args* 
         yw[c][1] = yw[c][2];
         yw[c][2] = y;
       }
-    }
+    };
+    walk_rows<LAT ? kLatRing : 0, 1, RowC>(0, nr + IW, loadc, workc);
   }
 
   // ============================== pass D (down)
@@ -827,19 +948,92 @@ __global__ __launch_bounds__(128) void sweep_kernel(Lin2Args A, const Lin2Args* 
         xo[2] = make_double2(xo[2].x + c.x, xo[2].y + c.y);
       }
     };
+    struct RowD {
+      FT f[3][4];      // ru, u1, u2, u3 of the u+, u-, uz solves
+      double2 x[3];    // eliminated column rows
+      double pd[2];    // dr p_h, p_h
+      double2 uc[3];   // corrector: previous iterate
+      double2 un[3];   // INC: u^n (+/- form for the velocity pair)
+    };
+    auto loadrow = [&](int i, RowD& R) {
+#pragma unroll
+      for (int c = 0; c < 3; c++) {
+        const size_t fo = c == 0 ? fb_up + (size_t)i * FR_UP
+                                 : (c == 1 ? fb_um + (size_t)i * FR_UP : fb_uz + (size_t)i * FR_ABS);
+        const int fs = c == 2 ? 64 : 128;
+#pragma unroll
+        for (int w = 0; w < 4; w++) {
+          if constexpr (F32W) R.f[c][w] = A.F32[fo + (3 + w) * fs];
+          else R.f[c][w] = A.F[fo + (3 + w) * fs];
+        }
+        R.x[c] = SR.ld(sb3 + (size_t)i * 384 + c * 128);
+      }
+      R.pd[0] = A.PH[phb + (size_t)i * 128];
+      R.pd[1] = A.PH[phb + (size_t)i * 128 + 64];
+      const size_t h = (size_t)i * MS + k;
+      if constexpr (!PRED) {
+#pragma unroll
+        for (int c = 0; c < 3; c++) R.uc[c] = A.u[c * n + h];
+      }
+      if constexpr (INC) {
+#pragma unroll
+        for (int c = 0; c < 3; c++) R.un[c] = A.un[c * n + h];
+      }
+    };
+    auto solve = [&](int i, const RowD& R, double2* xo, double* ho) {
+#pragma unroll
+      for (int c = 0; c < 3; c++) {
+        const double ru = R.f[c][0], u1 = R.f[c][1], u2 = R.f[c][2], u3 = R.f[c][3];
+        double2 x = R.x[c];
+        x.x -= u1 * xw[c][0].x;
+        x.y -= u1 * xw[c][0].y;
+        x.x -= u2 * xw[c][1].x;
+        x.y -= u2 * xw[c][1].y;
+        x.x -= u3 * xw[c][2].x;
+        x.y -= u3 * xw[c][2].y;
+        x = make_double2(x.x * ru, x.y * ru);
+        double hh = (i == nr - 1) ? 1.0 : 0.0;
+        hh -= u1 * xh[c][0];
+        hh -= u2 * xh[c][1];
+        hh -= u3 * xh[c][2];
+        hh *= ru;
+        xw[c][2] = xw[c][1];
+        xw[c][1] = xw[c][0];
+        xw[c][0] = x;
+        xh[c][2] = xh[c][1];
+        xh[c][1] = xh[c][0];
+        xh[c][0] = hh;
+        xo[c] = x;
+        ho[c] = hh;
+      }
+      if constexpr (INC) {  // the solution is u^n + delta (FP64)
+        double2 a = R.un[0], b = R.un[1];
+        pm_of(a, b);
+        const double2 c = R.un[2];
+        xo[0] = make_double2(xo[0].x + a.x, xo[0].y + a.y);
+        xo[1] = make_double2(xo[1].x + b.x, xo[1].y + b.y);
+        xo[2] = make_double2(xo[2].x + c.x, xo[2].y + c.y);
+      }
+    };
     // wall divergence of the provisional solution (divWall_k on r/theta
     // form) from the four wall rows. Without HOLD the walk that emits the
     // solution repeats their back substitution (same arithmetic, same
     // values), which keeps the pass at 3 waves per SIMD instead of 2.
     double2 urw[4], utw = z2, uzw = z2;
-    double2 xs[HOLD ? 4 : 1][3];  // HOLD: wall rows NR-1..NR-4
-    double xhs[HOLD ? 4 : 1][3];
+    double2 xs[HOLD || LAT ? 4 : 1][3];  // HOLD, LAT: wall rows NR-1..NR-4
+    double xhs[HOLD || LAT ? 4 : 1][3];
+    RowD ring[LAT ? 4 : 1];
+    if constexpr (LAT) {
+#pragma unroll
+      for (int s = 0; s < 4; s++) loadrow(nr - 1 - s, ring[s]);
+    }
 #pragma unroll
     for (int s = 0; s < 4; s++) {
       double2 xo[3];
       double ho[3];
-      backsub(nr - 1 - s, xo, ho);
-      if constexpr (HOLD) {
+      if constexpr (LAT) solve(nr - 1 - s, ring[s], xo, ho);
+      else backsub(nr - 1 - s, xo, ho);
+      if constexpr (HOLD || LAT) {
 #pragma unroll
         for (int c = 0; c < 3; c++) {
           xs[s][c] = xo[c];
@@ -854,7 +1048,7 @@ __global__ __launch_bounds__(128) void sweep_kernel(Lin2Args A, const Lin2Args* 
         uzw = xo[2];
       }
     }
-    if constexpr (!HOLD) {
+    if constexpr (!HOLD && !LAT) {
 #pragma unroll
       for (int c = 0; c < 3; c++)
 #pragma unroll
@@ -865,7 +1059,7 @@ __global__ __launch_bounds__(128) void sweep_kernel(Lin2Args A, const Lin2Args* 
     }
     double2 dv;
     {
-      const ctab Dr = Dcu + STEN * (nr - 1);
+      const TB Dr = Dcu + STEN * (nr - 1);
       double px = 0.0, py = 0.0;
 #pragma unroll
       for (int w = 0; w < 4; w++) {  // columns NR-4..NR-1 = urw[3..0]
@@ -898,7 +1092,7 @@ __global__ __launch_bounds__(128) void sweep_kernel(Lin2Args A, const Lin2Args* 
       // pressure-gradient homogeneous solution: (dr p_h -+ kt p_h / r, 0), (0, kz p_h)
       const double dph = pd ? pd[0] : A.PH[phb + (size_t)i * 128];
       const double ph = pd ? pd[1] : A.PH[phb + (size_t)i * 128 + 64];
-      const double tq = q.kt * ph / rt[i];
+      const double tq = over_r(q.kt * ph, i);
       const double2 hp[3] = {make_double2(dph - tq, 0.0), make_double2(dph + tq, 0.0), make_double2(-0.0, q.kz * ph)};
       const double2 hv[3] = {make_double2(ho[0], 0.0), make_double2(ho[1], 0.0), make_double2(0.0, ho[2])};
       double2 o[3] = {xo[0], xo[1], xo[2]};
@@ -925,7 +1119,21 @@ __global__ __launch_bounds__(128) void sweep_kernel(Lin2Args A, const Lin2Args* 
       A.out[n + h] = o[1];
       A.out[2 * n + h] = o[2];
     };
-    if constexpr (HOLD) {
+    if constexpr (LAT) {
+      auto loadd = [&](int i, RowD& R) { loadrow(row_of(i), R); };
+      RowD nxt[kLatRing];
+#pragma unroll
+      for (int s = 0; s < 4; s++) {
+        if (s < kLatRing) loadd(nr - 5 - s, nxt[s < kLatRing ? s : 0]);
+        emit(nr - 1 - s, xs[s], xhs[s], ring[s].pd, PRED ? nullptr : ring[s].uc);
+      }
+      walk_ring<kLatRing, -1>(nxt, nr - 5, -1, loadd, [&](int i, const RowD& R) {
+        double2 xo[3];
+        double ho[3];
+        solve(i, R, xo, ho);
+        emit(i, xo, ho, R.pd, PRED ? nullptr : R.uc);
+      });
+    } else if constexpr (HOLD) {
 #pragma unroll
       for (int s = 0; s < 4; s++) emit(nr - 1 - s, xs[s], xhs[s]);
       for (int i = nr - 5; i >= 0; i--) {
@@ -940,74 +1148,6 @@ __global__ __launch_bounds__(128) void sweep_kernel(Lin2Args A, const Lin2Args* 
       // row i is solved and stored, so each row's memory latency overlaps
       // the previous row's arithmetic (the compiler does not move loads
       // across the stores of a row by itself).  Same arithmetic as backsub.
-      using FT = std::conditional_t<F32W, float, double>;
-      struct RowD {
-        FT f[3][4];      // ru, u1, u2, u3 of the u+, u-, uz solves
-        double2 x[3];    // eliminated column rows
-        double pd[2];    // dr p_h, p_h
-        double2 uc[3];   // corrector: previous iterate
-        double2 un[3];   // INC: u^n (+/- form for the velocity pair)
-      };
-      auto loadrow = [&](int i, RowD& R) {
-#pragma unroll
-        for (int c = 0; c < 3; c++) {
-          const size_t fo = c == 0 ? fb_up + (size_t)i * FR_UP
-                                   : (c == 1 ? fb_um + (size_t)i * FR_UP : fb_uz + (size_t)i * FR_ABS);
-          const int fs = c == 2 ? 64 : 128;
-#pragma unroll
-          for (int w = 0; w < 4; w++) {
-            if constexpr (F32W) R.f[c][w] = A.F32[fo + (3 + w) * fs];
-            else R.f[c][w] = A.F[fo + (3 + w) * fs];
-          }
-          R.x[c] = SR.ld(sb3 + (size_t)i * 384 + c * 128);
-        }
-        R.pd[0] = A.PH[phb + (size_t)i * 128];
-        R.pd[1] = A.PH[phb + (size_t)i * 128 + 64];
-        const size_t h = (size_t)i * MS + k;
-        if constexpr (!PRED) {
-#pragma unroll
-          for (int c = 0; c < 3; c++) R.uc[c] = A.u[c * n + h];
-        }
-        if constexpr (INC) {
-#pragma unroll
-          for (int c = 0; c < 3; c++) R.un[c] = A.un[c * n + h];
-        }
-      };
-      auto solve = [&](int i, const RowD& R, double2* xo, double* ho) {
-#pragma unroll
-        for (int c = 0; c < 3; c++) {
-          const double ru = R.f[c][0], u1 = R.f[c][1], u2 = R.f[c][2], u3 = R.f[c][3];
-          double2 x = R.x[c];
-          x.x -= u1 * xw[c][0].x;
-          x.y -= u1 * xw[c][0].y;
-          x.x -= u2 * xw[c][1].x;
-          x.y -= u2 * xw[c][1].y;
-          x.x -= u3 * xw[c][2].x;
-          x.y -= u3 * xw[c][2].y;
-          x = make_double2(x.x * ru, x.y * ru);
-          double hh = (i == nr - 1) ? 1.0 : 0.0;
-          hh -= u1 * xh[c][0];
-          hh -= u2 * xh[c][1];
-          hh -= u3 * xh[c][2];
-          hh *= ru;
-          xw[c][2] = xw[c][1];
-          xw[c][1] = xw[c][0];
-          xw[c][0] = x;
-          xh[c][2] = xh[c][1];
-          xh[c][1] = xh[c][0];
-          xh[c][0] = hh;
-          xo[c] = x;
-          ho[c] = hh;
-        }
-        if constexpr (INC) {  // the solution is u^n + delta (FP64)
-          double2 a = R.un[0], b = R.un[1];
-          pm_of(a, b);
-          const double2 c = R.un[2];
-          xo[0] = make_double2(xo[0].x + a.x, xo[0].y + a.y);
-          xo[1] = make_double2(xo[1].x + b.x, xo[1].y + b.y);
-          xo[2] = make_double2(xo[2].x + c.x, xo[2].y + c.y);
-        }
-      };
       RowD cur, nxt;
       loadrow(nr - 1, cur);
       for (int i = nr - 1; i >= 0; i--) {
@@ -1090,17 +1230,27 @@ void launch_factor(const Geom& g, const double* r, const double* Lu, const doubl
   factor_kernel<<<grid, 256, 0, s>>>(g, r, Lu, Lp, F, F32);
 }
 
-// pass D runs as HOLD = 1 for the FP64-form pipes and as HOLD = 0 for the
-// mixed-form ones (a batched launch of both forms makes both launches)
-template <int PRED>
+// Small grids run the LAT kernels: at most kLatBlocks workgroups (two per CU;
+// at 1088, 64x128x1025, the sweeps run at the memory's rate), and radial
+// tables that fit the default LDS limit.  The kind depends on the grid alone,
+// so a pipe runs the same kernels on its own and in an ensemble.
+constexpr size_t kLatBlocks = 512;
+constexpr int kLatRows = 256;
+int sweep_lat(const Geom& g) { return sw_nblk(g) <= kLatBlocks && g.nr <= kLatRows ? 1 : 0; }
+static size_t lat_lds(int nr) { return (size_t)nr * (1 + 4 * STEN) * sizeof(double); }
+
+template <int PRED, int LAT>
 static void sweep_passes_inc(const Lin2Args& a, dim3 grid, hipStream_t s) {
-  if (PRED) sweep_kernel<4, PRED, 0, 0, 1><<<grid, 128, 0, s>>>(a, nullptr);
-  sweep_kernel<0, PRED, 0, 0, 1><<<grid, 128, 0, s>>>(a, nullptr);
-  sweep_kernel<1, PRED, 0, 0, 1><<<grid, 128, 0, s>>>(a, nullptr);
-  sweep_kernel<2, PRED, 0, 0, 1><<<grid, 128, 0, s>>>(a, nullptr);
-  sweep_kernel<3, PRED, 0, 0, 1><<<grid, 128, 0, s>>>(a, nullptr);
+  const size_t lds = LAT ? lat_lds(a.g.nr) : 0;
+  if (PRED) sweep_kernel<4, PRED, 0, 0, 1, LAT><<<grid, 128, lds, s>>>(a, nullptr);
+  sweep_kernel<0, PRED, 0, 0, 1, LAT><<<grid, 128, lds, s>>>(a, nullptr);
+  sweep_kernel<1, PRED, 0, 0, 1, LAT><<<grid, 128, lds, s>>>(a, nullptr);
+  sweep_kernel<2, PRED, 0, 0, 1, LAT><<<grid, 128, lds, s>>>(a, nullptr);
+  sweep_kernel<3, PRED, 0, 0, 1, LAT><<<grid, 128, lds, s>>>(a, nullptr);
 }
 
+// pass D runs as HOLD = 1 for the FP64-form pipes and as HOLD = 0 for the
+// mixed-form ones (a batched launch of both forms makes both launches)
 template <int PRED, int B>
 static void sweep_passes(const Lin2Args& a, const Lin2Args* tab, dim3 grid, bool fp64, bool mixed, hipStream_t s) {
   sweep_kernel<0, PRED, B><<<grid, 128, 0, s>>>(a, tab);
@@ -1109,12 +1259,25 @@ static void sweep_passes(const Lin2Args& a, const Lin2Args* tab, dim3 grid, bool
   if (fp64) sweep_kernel<3, PRED, B, 1><<<grid, 128, 0, s>>>(a, tab);
   if (mixed) sweep_kernel<3, PRED, B, 0><<<grid, 128, 0, s>>>(a, tab);
 }
+template <int PRED, int B>
+static void sweep_passes_lat(const Lin2Args& a, const Lin2Args* tab, dim3 grid, int nr, hipStream_t s) {
+  const size_t lds = lat_lds(nr);
+  sweep_kernel<0, PRED, B, 0, 0, 1><<<grid, 128, lds, s>>>(a, tab);
+  sweep_kernel<1, PRED, B, 0, 0, 1><<<grid, 128, lds, s>>>(a, tab);
+  sweep_kernel<2, PRED, B, 0, 0, 1><<<grid, 128, lds, s>>>(a, tab);
+  sweep_kernel<3, PRED, B, 0, 0, 1><<<grid, 128, lds, s>>>(a, tab);
+}
 
 void launch_sweep2(const Lin2Args& a, hipStream_t s) {
   const dim3 grid((a.g.nt / 2) * ((a.g.nz + 63) / 64));
   if (a.inc) {
-    if (a.predictor) sweep_passes_inc<1>(a, grid, s);
-    else sweep_passes_inc<0>(a, grid, s);
+    if (a.predictor) a.lat ? sweep_passes_inc<1, 1>(a, grid, s) : sweep_passes_inc<1, 0>(a, grid, s);
+    else a.lat ? sweep_passes_inc<0, 1>(a, grid, s) : sweep_passes_inc<0, 0>(a, grid, s);
+    return;
+  }
+  if (a.lat) {
+    if (a.predictor) sweep_passes_lat<1, 0>(a, nullptr, grid, a.g.nr, s);
+    else sweep_passes_lat<0, 0>(a, nullptr, grid, a.g.nr, s);
     return;
   }
   const bool fp64 = a.form64 != 0;
@@ -1122,12 +1285,18 @@ void launch_sweep2(const Lin2Args& a, hipStream_t s) {
   else sweep_passes<0, 0>(a, nullptr, grid, fp64, !fp64, s);
 }
 
-void launch_sweep_batch(const Lin2Args* tab, int count, int predictor, int max_nt, int max_nz, bool fp64,
-                        bool mixed, hipStream_t s) {
-  const dim3 grid((max_nt / 2) * ((max_nz + 63) / 64), count);
+void launch_sweep_batch(const Lin2Args* tab, int count, int predictor, const SweepExtent& x, hipStream_t s) {
   Lin2Args dummy{};
-  if (predictor) sweep_passes<1, 1>(dummy, tab, grid, fp64, mixed, s);
-  else sweep_passes<0, 1>(dummy, tab, grid, fp64, mixed, s);
+  if (x.fp64 || x.mixed) {
+    const dim3 grid((x.max_nt / 2) * ((x.max_nz + 63) / 64), count);
+    if (predictor) sweep_passes<1, 1>(dummy, tab, grid, x.fp64, x.mixed, s);
+    else sweep_passes<0, 1>(dummy, tab, grid, x.fp64, x.mixed, s);
+  }
+  if (x.lat_nr > 0) {
+    const dim3 grid(x.lat_blocks, count);
+    if (predictor) sweep_passes_lat<1, 1>(dummy, tab, grid, x.lat_nr, s);
+    else sweep_passes_lat<0, 1>(dummy, tab, grid, x.lat_nr, s);
+  }
 }
 
 }  // namespace nsp

@@ -215,6 +215,16 @@ struct Lin2Args {
   unsigned long long* norm;
   int predictor;
   int ord;              // block order (NlVariant::s_ord)
+  int lat;              // small grid: the LAT kernels (sweep_lat)
+};
+int sweep_lat(const Geom& g);  // whether a grid's sweeps run the LAT kernels (linear2.hip)
+// Members of a batched sweep: the largest extents of those that run the
+// bandwidth-bound kernels, whether some of them are of the FP64 or the mixed
+// form, and the largest workgroup and row counts of those that run the LAT ones.
+struct SweepExtent {
+  int max_nt = 0, max_nz = 0;
+  bool fp64 = false, mixed = false;
+  int lat_blocks = 0, lat_nr = 0;
 };
 // F32 (may be null): FP32 copies of the u+, u-, uz factor sets, same indices
 void launch_factor(const Geom& g, const double* r, const double* Lu, const double* Lp, double* F, float* F32,
@@ -222,10 +232,8 @@ void launch_factor(const Geom& g, const double* r, const double* Lu, const doubl
 size_t factor_count(const Geom& g);    // doubles of the stored LU factors
 size_t factor32_count(const Geom& g);  // floats of the FP32 u+, u-, uz sets
 void launch_sweep2(const Lin2Args& a, hipStream_t s);
-// one launch per pass for `count` pipes (tab in device memory); max_nt/max_nz
-// are the largest extents among them; fp64/mixed: some pipe is of that form
-void launch_sweep_batch(const Lin2Args* tab, int count, int predictor, int max_nt, int max_nz, bool fp64,
-                        bool mixed, hipStream_t s);
+// one launch per pass and kind of kernel for `count` pipes (tab in device memory)
+void launch_sweep_batch(const Lin2Args* tab, int count, int predictor, const SweepExtent& x, hipStream_t s);
 // centred stencil table: w-th weight of row i multiplies column i-3+w
 std::vector<double> centred_table(int nr, const std::vector<double>& T);
 

@@ -291,6 +291,25 @@ def test_row_pair_z_pass(nz, prec, tol):
     p.close()
 
 
+@pytest.mark.parametrize("prec,tol", [(nsp.FP64, 1e-12), (nsp.MIXED, 1e-6), (nsp.MIXED_REFINED, 1e-6)],
+                         ids=["fp64", "mixed", "refined"])
+@pytest.mark.parametrize("nr", [8, 9, 10, 11, 13])
+def test_small_grid_sweeps(nr, prec, tol):
+    """The sweeps of small grids (row loads in flight, LDS tables) at row
+    counts around the ring's length and the wall rows, against the oracle."""
+    shape = dict(nr=nr, nt=64, nz=65, lz=4 * np.pi, re=2000.0, dt=0.005)
+    print(f"[gpu] small-grid sweeps {shape} precision {prec}", flush=True)
+    p = nsp.Pipe(**shape, precision=prec)
+    o = Oracle(**shape)
+    p.seeded_ic(SEED1, 10, 20, 0, 0.1)
+    o.set_state(*p.get_state())
+    n_p, _, flags = p.step(2)
+    n_o, _ = o.step(2)
+    assert np.array_equal(n_p, n_o) and not flags.any()
+    fields_close(p.get_state(), o.get_state(), tol)
+    p.close()
+
+
 # the longest compiled plans: theta 1152 (NT = 768) and half-z 4608 (NZ = 3073)
 LONG = [dict(nr=8, nt=768, nz=65, lz=4 * np.pi, re=19000.0, dt=0.0005),
         dict(nr=8, nt=64, nz=3073, lz=4 * np.pi, re=19000.0, dt=0.0005)]
