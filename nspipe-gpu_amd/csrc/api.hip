@@ -393,12 +393,13 @@ static nsp_status create_handle(const nsp_params* p, int device, const nsp_handl
 
   // FFT plans
   std::vector<int> perm_t, perm_h;
-  if (!make_fft_plan(g.ntp, h->nb.pt, perm_t) || !make_fft_plan(g.nh, h->nb.ph, perm_h))
+  if (!make_fft_plan(g.ntp, h->nb.pt, perm_t) || !make_fft_plan(g.nh, h->nb.ph, perm_h, kZRadix))
     return bail(fail(NSP_ERR_INVALID, "transform lengths must factor into 2, 3 and 5"));
   TRY(upload(h, &h->nb.perm_t, perm_t));
   TRY(upload(h, &h->nb.perm_h, perm_h));
-  TRY(upload(h, &h->nb.tw_t, twiddles(g.ntp, g.ntp)));
-  TRY(upload(h, &h->nb.tw_h, twiddles(g.nh, g.nh)));
+  auto pass_tw = [](const FftPlan& p) { return pass_twiddles(std::vector<int>(p.rad, p.rad + p.nrad)); };
+  TRY(upload(h, &h->nb.tw_t, pass_tw(h->nb.pt)));
+  TRY(upload(h, &h->nb.tw_h, pass_tw(h->nb.ph)));
   TRY(upload(h, &h->nb.tw_z, twiddles(g.nzf, g.nh + 1)));
   h->nb.wstride = size_t(g.nr) * tp_plane(g);  // tile-major planes (tp_plane)
   h->nb.use_ct = false;

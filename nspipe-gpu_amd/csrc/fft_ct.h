@@ -6,7 +6,7 @@
 // S_p into one of length S_p*R_p; the result comes out in natural order.
 // All radices, strides and divisors are compile-time constants, so index
 // arithmetic reduces to shifts and multiply-high sequences and the butterfly
-// loops unroll.  Butterflies of radix 6, 8, 9, 12, 16, 18 are composite
+// loops unroll.  Butterflies of radix 6, 8, 9, 10, 12, 15, 16, 18 are composite
 // in-register DFTs (R = R1*R2) with constant twiddles evaluated by the
 // compiler.
 //
@@ -68,6 +68,23 @@ __device__ __forceinline__ cpx<T> cx_mul(cpx<T> a, cpx<T> b) {
 template <typename T>
 __device__ __forceinline__ cpx<T> cx_mulc(cpx<T> a, cpx<T> b) {  // a * conj(b)
   return {a.x * b.x + a.y * b.y, a.y * b.x - a.x * b.y};
+}
+
+// A copy of x the compiler cannot see through.  Index arithmetic derived from
+// it is recomputed where it is used instead of being hoisted out of the
+// transform loops and kept live in registers (which cost occupancy).
+__device__ __forceinline__ int opaque(int x) {
+  asm volatile("" : "+v"(x));
+  __builtin_assume((unsigned)x < 1024u);
+  return x;
+}
+
+// Fixes a value where it is formed: without it the compiler sinks a product
+// past the following transform to its use and holds the factors' registers.
+template <typename T>
+__device__ __forceinline__ void pin(cpx<T>& v) {
+  asm volatile("" : "+v"(v.x));
+  asm volatile("" : "+v"(v.y));
 }
 
 // ---------------------------------------------------------------- small DFTs
@@ -175,6 +192,10 @@ template <typename T, int SIGN> struct DFT<T, 6, SIGN> {
   __device__ __forceinline__ static void run(cpx<T>* v) { dft_composite<T, 3, 2, SIGN>(v); } };
 template <typename T, int SIGN> struct DFT<T, 8, SIGN> {
   __device__ __forceinline__ static void run(cpx<T>* v) { dft_composite<T, 4, 2, SIGN>(v); } };
+template <typename T, int SIGN> struct DFT<T, 10, SIGN> {
+  __device__ __forceinline__ static void run(cpx<T>* v) { dft_composite<T, 5, 2, SIGN>(v); } };
+template <typename T, int SIGN> struct DFT<T, 15, SIGN> {
+  __device__ __forceinline__ static void run(cpx<T>* v) { dft_composite<T, 5, 3, SIGN>(v); } };
 template <typename T, int SIGN> struct DFT<T, 9, SIGN> {
   __device__ __forceinline__ static void run(cpx<T>* v) { dft_composite<T, 3, 3, SIGN>(v); } };
 template <typename T, int SIGN> struct DFT<T, 12, SIGN> {

@@ -102,6 +102,10 @@ __global__ __launch_bounds__(256) void dr3_kernel(Geom g, const double* __restri
 }
 
 // ------------------------------------------------------------------ theta inverse
+// Lengths without compiled plans: TL axial columns of a level, one field after
+// the other, zero rows written with the data's.  Bound by the passes' LDS round
+// trips; 45 levels of 80 x 161 FP64, radices up to 5 -> up to 16: 126 -> 81 us
+// (forward 48 -> 31).
 template <int TL>
 __global__ __launch_bounds__(256) void theta_inv_kernel(Geom g, FftPlan P, const int* __restrict__ perm,
                                                         const C* __restrict__ tw,
@@ -120,41 +124,51 @@ __global__ __launch_bounds__(256) void theta_inv_kernel(Geom g, FftPlan P, const
     const int c = f % 3, kind = f / 3;  // kind 0: u, 1: d_r u, 2: d_theta u / r
     const double2* src = u + c * g.n + (size_t)i * g.modes;
     const double2* srd = dR + c * dr_cs(g) + (size_t)i * dr_plane(g);  // tile-major d_r u
-    for (int e = tid; e < g.ntp * TL; e += nthr) buf[e] = C{0.0, 0.0};
-    __syncthreads();
-    for (int e = tid; e < g.nt * TL; e += nthr) {
-      const int it = e / TL, tl = e - it * TL, l = l0 + tl;
-      if (l < g.nz) {
+    // padded row j (padForward_k row map): j < NT/2 holds it = j, rows NT/2 <= j < NT are zero, j >= NT holds j - NT/2
+    for (int e = tid; e < g.ntp * TL; e += nthr) {
+      const int j = e / TL, tl = e - j * TL, l = l0 + tl;
+      C w{0.0, 0.0};
+      if ((j < half || j >= g.nt) && l < g.nz) {
+        const int it = j < half ? j : j - half;
         const double2 v = kind == 1 ? srd[(size_t)it * 64 + dr_col(g, l)] : src[(size_t)it * g.nz + l];
-        C w{v.x, v.y};
+        w = C{v.x, v.y};
         if (kind == 2) {  // derivt_k (mod_deriv.cu:10-21)
           const double kt = double(m_of(it, g.nt));
           w = C{-kt * v.y / ri, kt * v.x / ri};
         }
-        const int j = it < half ? it : it + half;  // padForward_k row map
-        buf[perm[j] * TL + tl] = w;
       }
+      buf[lds_pos<TL>(perm[j] * TL + tl)] = w;
     }
     __syncthreads();
-    fft_passes<double>(buf, P, TL, 1.0, tw, tid, nthr);
+    fft_passes<double, TL, +1>(buf, P, tw, tid, nthr);
     double2* dst = W + f * ws + (size_t)i * tp_plane(g);  // tile-major W
     for (int e = tid; e < g.ntp * TL; e += nthr) {
       const int j = e / TL, tl = e - j * TL, l = l0 + tl;
-      if (l < g.nz) dst[(size_t)j * 64 + tp_col(g, l)] = make_double2(buf[e].x, buf[e].y);
+      const C w = buf[lds_pos<TL>(e)];
+      if (l < g.nz) dst[(size_t)j * 64 + tp_col(g, l)] = make_double2(w.x, w.y);
     }
     __syncthreads();
   }
 }
 
 // ------------------------------------------------------------------ z pass
-// Real transforms of length N = NZF through complex transforms of length
-// NH = N/2 on z[m] = x[2m] + i x[2m+1].
+// One (level, theta) row per workgroup.  Real transforms of length N = NZF
+// through complex transforms of length NH = N/2 on z[m] = x[2m] + i x[2m+1].
 //   inverse: Z[k] = E + iO, E = X[k] + conj(X[NH-k]),
 //            O = (X[k] - conj(X[NH-k])) e^{+2 pi i k/N}
 //   forward: E = (Z[k] + conj(Z[NH-k]))/2, O = (Z[k] - conj(Z[NH-k]))/(2i),
 //            X[k] = E + e^{-2 pi i k/N} O
+// The fifteen transforms of a row share one copy of the passes (their radix
+// switch is long): the forward ones run on the inverse passes with real and
+// imaginary parts exchanged.  As many threads as give each at most MPT real
+// samples, so that a short row is one wave and many rows share a CU: the pass
+// is bound by the latency of its LDS round trips.  45 levels x 120 rows of 480:
+// 0.441 ms with radices up to 5 and one transform after the other in 256
+// threads -> 0.217; 16 x 12 rows of 24: 37 -> 27 us.  (Two rows as one
+// full-length transform, as the compiled plans do, needs twice the registers:
+// 45 x 120 rows of 480 took 0.34-0.45 ms.)
 template <int MPT>
-__global__ __launch_bounds__(256) void zpass_kernel(Geom g, FftPlan P, const int* __restrict__ perm,
+__global__ __launch_bounds__(512) void zpass_kernel(Geom g, FftPlan P, const int* __restrict__ perm,
                                                     const C* __restrict__ tw,
                                                     const C* __restrict__ twz,
                                                     const double* __restrict__ r,
@@ -167,91 +181,122 @@ __global__ __launch_bounds__(256) void zpass_kernel(Geom g, FftPlan P, const int
   const int i = row / g.ntp;
   const int tid = threadIdx.x, nthr = blockDim.x;
   const int nh = g.nh, nz = g.nz, nzf = g.nzf;
-  const double rad = r[i];
+  double rad = r[i];
+  asm volatile("" : "+v"(rad));  // keeps the divisions by it where they are used
   // row th of level i in the tile-major planes of W, Y: value k at roff + tp_col(k)
-  const size_t roff = (size_t)(row / g.ntp) * tp_plane(g) + (size_t)(row % g.ntp) * 64;
-
-  // inverse real transform of spectral row X (entries l < nz, zero beyond);
-  // dz: differentiate in z first (derivz_k, mod_deriv.cu:24-35)
-  auto c2r = [&](const double2* X, bool dz) {
-    for (int k = tid; k < nh; k += nthr) {
-      const int kc = nh - k;
-      C a{0.0, 0.0}, b{0.0, 0.0};
-      if (k < nz) { const double2 v = X[tp_col(g, k)]; a = C{v.x, v.y}; }
-      if (kc < nz) { const double2 v = X[tp_col(g, kc)]; b = C{v.x, v.y}; }
-      if (k == 0) { a.y = 0.0; b.y = 0.0; }
-      if (dz) {
-        const double ka = g.kz0 * double(k), kb = g.kz0 * double(kc);
-        a = C{-ka * a.y, ka * a.x};
-        b = C{-kb * b.y, kb * b.x};
+  const size_t roff = (size_t)i * tp_plane(g) + (size_t)(row - i * g.ntp) * 64;
+  // The inverse's inputs come in pairs Z[k] = E + iO, Z[NH-k] = conj(E) + i
+  // conj(O), k <= NH/2.  Of the owned k: LDS positions, offsets of the stored
+  // modes k and NH-k (-1 past NZ), split twiddles; the same for every field.
+  constexpr int KP = MPT / 4 + 1;
+  int pa[KP], pb[KP], oa[KP], ob[KP];
+  C wz[KP];
+#pragma unroll
+  for (int q = 0; q < KP; q++) {
+    const int k = tid + q * nthr, kc = nh - k;
+    const bool in = 2 * k <= nh;
+    pa[q] = in ? lds_pos<kPadCol>(perm[k]) : -1;
+    pb[q] = in && k > 0 && kc != k ? lds_pos<kPadCol>(perm[kc]) : -1;
+    oa[q] = in && k < nz ? (int)tp_col(g, k) : -1;
+    ob[q] = in && kc < nz ? (int)tp_col(g, kc) : -1;
+    wz[q] = twz[in ? k : 0];
+  }
+  double2 A[KP], Bv[KP];
+  // field of inverse transform f = 0..11: u_r, u_t, u_z, then per component c: d_r u_c, d_theta u_c / r, u_c
+  auto load = [&](int f) {
+    const int c = f < 3 ? 0 : (f - 3) / 3, kk = f < 3 ? 0 : (f - 3) % 3;
+    const double2* X = W + (f < 3 ? f : (kk == 2 ? c : 3 + 3 * kk + c)) * ws + roff;
+#pragma unroll
+    for (int q = 0; q < KP; q++) {
+      A[q] = Bv[q] = make_double2(0.0, 0.0);
+      if (oa[q] >= 0) A[q] = X[oa[q]];
+      if (ob[q] >= 0) Bv[q] = X[ob[q]];
+    }
+  };
+  load(0);
+  double ur[MPT] = {}, ut[MPT] = {}, uz[MPT] = {}, acc[MPT] = {};
+#pragma unroll 1
+  for (int t = 0; t < 15; t++) {
+    // transforms 0..2: u_r, u_t, u_z; then per component c: d_r u_c, d_theta u_c / r, d_z u_c, and N_c forward
+    const int c = t < 3 ? 0 : (t - 3) / 4, kind = t < 3 ? 4 : (t - 3) % 4;
+    int lt = opaque(tid);
+    if (kind == 3) {
+#pragma unroll
+      for (int q = 0; q < MPT; q++) {
+        const int n = lt + q * nthr;
+        if (n < nzf) reinterpret_cast<double*>(&buf[lds_pos<kPadCol>(perm[n >> 1])])[1 - (n & 1)] = -acc[q];
       }
-      const C E{a.x + b.x, a.y - b.y};
-      const C dlt{a.x - b.x, a.y + b.y};
-      const C w = twz[k];
-      const C O{dlt.x * w.x + dlt.y * w.y, dlt.y * w.x - dlt.x * w.y};  // dlt * conj(w)
-      buf[perm[k]] = C{E.x - O.y, E.y + O.x};
+    } else {
+#pragma unroll
+      for (int q = 0; q < KP; q++) {
+        const int k = lt + q * nthr;
+        double2 a = A[q], b = Bv[q];
+        if (k == 0) { a.y = 0.0; b.y = 0.0; }
+        if (kind == 2) {  // derivz_k (mod_deriv.cu:24-35)
+          const double ka = g.kz0 * double(k), kb = g.kz0 * double(nh - k);
+          a = make_double2(-ka * a.y, ka * a.x);
+          b = make_double2(-kb * b.y, kb * b.x);
+        }
+        const C E{a.x + b.x, a.y - b.y};
+        const C dlt{a.x - b.x, a.y + b.y};
+        const C O = cx_mulc(dlt, wz[q]);
+        if (pa[q] >= 0) buf[pa[q]] = C{E.x - O.y, E.y + O.x};
+        if (pb[q] >= 0) buf[pb[q]] = C{E.x + O.y, O.x - E.y};
+      }
+      const int f = t < 3 ? t : 3 + 3 * c + kind;
+      if (f < 11) load(f + 1);  // in flight during the passes
     }
     __syncthreads();
-    fft_passes<double>(buf, P, 1, 1.0, tw, tid, nthr);
-  };
-  auto sample = [&](int n) -> double {
-    const C v = buf[n >> 1];
-    return (n & 1) ? v.y : v.x;
-  };
-
-  double ur[MPT], ut[MPT], uz[MPT], acc[MPT];
-  c2r(W + 0 * ws + roff, false);
-#pragma unroll
-  for (int q = 0; q < MPT; q++) { const int n = tid + q * nthr; ur[q] = n < nzf ? sample(n) : 0.0; }
-  __syncthreads();
-  c2r(W + 1 * ws + roff, false);
-#pragma unroll
-  for (int q = 0; q < MPT; q++) { const int n = tid + q * nthr; ut[q] = n < nzf ? sample(n) : 0.0; }
-  __syncthreads();
-  c2r(W + 2 * ws + roff, false);
-#pragma unroll
-  for (int q = 0; q < MPT; q++) { const int n = tid + q * nthr; uz[q] = n < nzf ? sample(n) : 0.0; }
-  __syncthreads();
-
-  for (int c = 0; c < 3; c++) {
-    // calcNonlinear_k (mod_io_nonlinear.cu:142-170), summed in its order
-    c2r(W + (3 + c) * ws + roff, false);
-#pragma unroll
-    for (int q = 0; q < MPT; q++) { const int n = tid + q * nthr; acc[q] = n < nzf ? ur[q] * sample(n) : 0.0; }
-    __syncthreads();
-    c2r(W + (6 + c) * ws + roff, false);
-#pragma unroll
-    for (int q = 0; q < MPT; q++) { const int n = tid + q * nthr; if (n < nzf) acc[q] += ut[q] * sample(n); }
-    __syncthreads();
-    c2r(W + c * ws + roff, true);
-#pragma unroll
-    for (int q = 0; q < MPT; q++) { const int n = tid + q * nthr; if (n < nzf) acc[q] += uz[q] * sample(n); }
-    __syncthreads();
-#pragma unroll
-    for (int q = 0; q < MPT; q++) {
-      const int n = tid + q * nthr;
-      if (n < nzf) {
-        double v = acc[q];
-        if (c == 0) v = v - ut[q] * (ut[q] / rad);
-        else if (c == 1) v = v + ur[q] * (ut[q] / rad);
-        double* slot = reinterpret_cast<double*>(&buf[perm[n >> 1]]) + (n & 1);
-        *slot = -v;
+    fft_passes<double, kPadCol, +1, kZRadix>(buf, P, tw, lt, nthr);
+    lt = opaque(tid);
+    if (kind == 3) {
+      double2* dst = Y + c * ws + roff;
+      for (int k = lt; k < nz; k += nthr) {
+        C X{0.0, 0.0};
+        if (k < nz - 1) {
+          const C p = buf[lds_pos<kPadCol>(k)], pc = buf[lds_pos<kPadCol>(k == 0 ? 0 : nh - k)];
+          const C zk{p.y, p.x}, zc{pc.y, pc.x};  // exchanged back
+          const C E{0.5 * (zk.x + zc.x), 0.5 * (zk.y - zc.y)};
+          const C d{zk.x - zc.x, zk.y + zc.y};
+          const C O{0.5 * d.y, -0.5 * d.x};
+          const C w = twz[k];
+          X = C{E.x + (w.x * O.x - w.y * O.y), E.y + (w.x * O.y + w.y * O.x)};
+        }
+        dst[tp_col(g, k)] = make_double2(X.x, X.y);
       }
-    }
-    __syncthreads();
-    fft_passes<double>(buf, P, 1, -1.0, tw, tid, nthr);
-    double2* dst = Y + c * ws + roff;
-    for (int k = tid; k < nz; k += nthr) {
-      C X{0.0, 0.0};
-      if (k < nz - 1) {
-        const C zk = buf[k], zc = buf[k == 0 ? 0 : nh - k];
-        const C E{0.5 * (zk.x + zc.x), 0.5 * (zk.y - zc.y)};
-        const C d{zk.x - zc.x, zk.y + zc.y};
-        const C O{0.5 * d.y, -0.5 * d.x};
-        const C w = twz[k];
-        X = C{E.x + (w.x * O.x - w.y * O.y), E.y + (w.x * O.y + w.y * O.x)};
+    } else {
+      const double* smp = reinterpret_cast<const double*>(buf);
+      double sm[MPT];
+#pragma unroll
+      for (int q = 0; q < MPT; q++) {
+        const int n = lt + q * nthr;
+        sm[q] = smp[n < nzf ? 2 * lds_pos<kPadCol>(n >> 1) + (n & 1) : 0];
       }
-      dst[tp_col(g, k)] = make_double2(X.x, X.y);
+      // calcNonlinear_k (mod_io_nonlinear.cu:142-170), summed in its order
+      if (kind == 4) {
+#pragma unroll
+        for (int q = 0; q < MPT; q++) {
+          ur[q] = ut[q];
+          ut[q] = uz[q];
+          uz[q] = sm[q];
+        }
+      } else if (kind == 0) {
+#pragma unroll
+        for (int q = 0; q < MPT; q++) acc[q] = ur[q] * sm[q];
+      } else if (kind == 1) {
+#pragma unroll
+        for (int q = 0; q < MPT; q++) acc[q] += ut[q] * sm[q];
+      } else {
+#pragma unroll
+        for (int q = 0; q < MPT; q++) acc[q] = acc[q] + uz[q] * sm[q];
+        if (c == 0) {
+#pragma unroll
+          for (int q = 0; q < MPT; q++) acc[q] = acc[q] - ut[q] * (ut[q] / rad);
+        } else if (c == 1) {
+#pragma unroll
+          for (int q = 0; q < MPT; q++) acc[q] = acc[q] + ur[q] * (ut[q] / rad);
+        }
+      }
     }
     __syncthreads();
   }
@@ -278,15 +323,15 @@ __global__ __launch_bounds__(256) void theta_fwd_kernel(Geom g, FftPlan P, const
       const int j = e / TL, tl = e - j * TL, l = l0 + tl;
       C v{0.0, 0.0};
       if (l < g.nz - 1) { const double2 a = src[(size_t)j * 64 + tp_col(g, l)]; v = C{a.x, a.y}; }
-      buf[perm[j] * TL + tl] = v;
+      buf[lds_pos<TL>(perm[j] * TL + tl)] = v;
     }
     __syncthreads();
-    fft_passes<double>(buf, P, TL, -1.0, tw, tid, nthr);
+    fft_passes<double, TL, -1>(buf, P, tw, tid, nthr);
     for (int e = tid; e < g.nt * TL; e += nthr) {
       const int it = e / TL, tl = e - it * TL, l = l0 + tl;
       if (l < g.nz) {
         const int j = it < half ? it : it + half;  // padBackward_k row map
-        C v = buf[j * TL + tl];
+        C v = buf[lds_pos<TL>(j * TL + tl)];
         v.x = v.x / norm;
         v.y = v.y / norm;
         if (it == half || l == g.nz - 1) v = C{0.0, 0.0};
@@ -346,10 +391,11 @@ static void theta_dispatch(const Geom& g, const DevTables& t, const NlBufs& nb, 
 
 template <int MPT>
 static void run_z(const Geom& g, const DevTables& t, const NlBufs& nb, hipStream_t s) {
-  const size_t lds = size_t(g.nh) * sizeof(double2);
+  const size_t lds = size_t(lds_pos<kPadCol>(g.nh)) * sizeof(double2);
+  const int nthr = 64 * ((g.nzf + 64 * MPT - 1) / (64 * MPT));
   (void)hipFuncSetAttribute((const void*)zpass_kernel<MPT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-  zpass_kernel<MPT><<<g.nr * g.ntp, 256, lds, s>>>(g, nb.ph, nb.perm_h, (const C*)nb.tw_h, (const C*)nb.tw_z,
-                                                    t.r, nb.W, nb.wstride, nb.Y);
+  zpass_kernel<MPT><<<g.nr * g.ntp, nthr, lds, s>>>(g, nb.ph, nb.perm_h, (const C*)nb.tw_h, (const C*)nb.tw_z, t.r,
+                                                    nb.W, nb.wstride, nb.Y);
 }
 
 const char* kernel_name(int id) {
@@ -449,16 +495,12 @@ void launch_nonlinear(const Geom& g, const DevTables& t, const NlBufs& nb, const
   theta_dispatch(g, t, nb, u, N, s, true);
   if (pf) pf->end(s);
   if (pf) pf->begin(K_ZPASS, s);
-  const int mpt = (g.nzf + 255) / 256;
-  if (mpt <= 1) run_z<1>(g, t, nb, s);
-  else if (mpt <= 2) run_z<2>(g, t, nb, s);
-  else if (mpt <= 4) run_z<4>(g, t, nb, s);
-  else if (mpt <= 6) run_z<6>(g, t, nb, s);
-  else if (mpt <= 8) run_z<8>(g, t, nb, s);
-  else if (mpt <= 12) run_z<12>(g, t, nb, s);
-  else if (mpt <= 18) run_z<18>(g, t, nb, s);
-  else if (mpt <= 24) run_z<24>(g, t, nb, s);
-  else run_z<36>(g, t, nb, s);
+  // samples per thread: a row of up to 512 is one wave
+  if (g.nzf <= 64) run_z<1>(g, t, nb, s);
+  else if (g.nzf <= 128) run_z<2>(g, t, nb, s);
+  else if (g.nzf <= 256) run_z<4>(g, t, nb, s);
+  else if (g.nzf <= 8 * 512) run_z<8>(g, t, nb, s);
+  else run_z<18>(g, t, nb, s);
   if (pf) pf->end(s);
   if (pf) pf->begin(K_THETA_FWD, s);
   theta_dispatch(g, t, nb, u, N, s, false);

@@ -12,23 +12,6 @@ namespace nsp {
 
 __device__ __forceinline__ int m_of_ct(int it, int nt) { return it < nt / 2 ? it : it - nt; }
 
-// A copy of x the compiler cannot see through.  Index arithmetic derived from
-// it is recomputed where it is used instead of being hoisted out of the
-// transform loops and kept live in registers (which cost occupancy).
-__device__ __forceinline__ int opaque(int x) {
-  asm volatile("" : "+v"(x));
-  __builtin_assume((unsigned)x < 1024u);
-  return x;
-}
-
-// Fixes a value where it is formed: without it the compiler sinks a product
-// past the following transform to its use and holds the factors' registers.
-template <typename T>
-__device__ __forceinline__ void pin(cpx<T>& v) {
-  asm volatile("" : "+v"(v.x));
-  asm volatile("" : "+v"(v.y));
-}
-
 // Raw buffer loads.  A load whose byte offset lies past num_records returns
 // zero instead of touching memory, which gives the zero padding of a row
 // beyond its stored modes without clamps or selects.  The resource is the

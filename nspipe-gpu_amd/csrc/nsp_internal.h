@@ -34,8 +34,10 @@ struct FftPlan {
   int L;
   int nrad;
   int rad[MAXRAD];
+  unsigned mul[MAXRAD];  // ceil(2^32 / S) of the pass's sub-length S
 };
-bool make_fft_plan(int L, FftPlan& p, std::vector<int>& perm);
+constexpr int kZRadix = 10;  // largest radix of the z plan (its kernel holds four fields in registers)
+bool make_fft_plan(int L, FftPlan& p, std::vector<int>& perm, int max_radix = 16);
 
 // complex pair aligned to its size, so loads and stores are single vector ops
 template <typename T> struct alignas(2 * sizeof(T)) cpx { T x, y; };
@@ -272,8 +274,8 @@ struct NlBufs {
   FftPlan pt, ph;      // theta (length NTP) and half-length z (length NZF/2) plans
   int* perm_t;         // [NTP]
   int* perm_h;         // [NH]
-  double2* tw_t;       // [NTP] exp(-2 pi i e/NTP)
-  double2* tw_h;       // [NH]  exp(-2 pi i e/NH)
+  double2* tw_t;       // pass twiddles of the two plans (pass_twiddles)
+  double2* tw_h;
   double2* tw_z;       // [NH+1] exp(-2 pi i k/NZF)
   double2* dR;         // [3][N] radial derivatives
   double2* W;          // [9][NR*NTP*NZ] theta-inverse intermediates

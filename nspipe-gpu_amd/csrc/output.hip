@@ -68,22 +68,23 @@ __global__ __launch_bounds__(256) void phys_theta_kernel(Geom g, FftPlan P, cons
   const int tid = threadIdx.x, nthr = blockDim.x;
   const int half = g.nt / 2;
   const double2* src = u + (size_t)i * g.modes;
-  for (int e = tid; e < g.ntp * TL; e += nthr) buf[e] = C{0.0, 0.0};
+  for (int e = tid; e < g.ntp * TL; e += nthr) buf[lds_pos<TL>(e)] = C{0.0, 0.0};
   __syncthreads();
   for (int e = tid; e < g.nt * TL; e += nthr) {
     const int it = e / TL, tl = e - it * TL, l = l0 + tl;
     if (l < g.nz) {
       const double2 v = src[(size_t)it * g.nz + l];
       const int j = it < half ? it : it + half;
-      buf[perm[j] * TL + tl] = C{v.x, v.y};
+      buf[lds_pos<TL>(perm[j] * TL + tl)] = C{v.x, v.y};
     }
   }
   __syncthreads();
-  fft_passes<double>(buf, P, TL, 1.0, tw, tid, nthr);
+  fft_passes<double, TL, +1>(buf, P, tw, tid, nthr);
   double2* dst = Wt + (size_t)i * g.ntp * g.nz;
   for (int e = tid; e < g.ntp * TL; e += nthr) {
     const int j = e / TL, tl = e - j * TL, l = l0 + tl;
-    if (l < g.nz) dst[(size_t)j * g.nz + l] = make_double2(buf[e].x, buf[e].y);
+    const C w = buf[lds_pos<TL>(e)];
+    if (l < g.nz) dst[(size_t)j * g.nz + l] = make_double2(w.x, w.y);
   }
 }
 
@@ -113,15 +114,15 @@ __global__ __launch_bounds__(256) void phys_z_kernel(Geom g, FftPlan P, const in
     const C dlt{a.x - b.x, a.y + b.y};
     const C w = twz[k];
     const C O{dlt.x * w.x + dlt.y * w.y, dlt.y * w.x - dlt.x * w.y};  // dlt * conj(w)
-    buf[perm[k]] = C{E.x - O.y, E.y + O.x};
+    buf[lds_pos<kPadCol>(perm[k])] = C{E.x - O.y, E.y + O.x};
   }
   __syncthreads();
-  fft_passes<double>(buf, P, 1, 1.0, tw, tid, nthr);
+  fft_passes<double, kPadCol, +1, kZRadix>(buf, P, tw, tid, nthr);
   double* o = out + (size_t)row * pitch;
   for (size_t n = tid; n < pitch; n += nthr) {
     double v = 0.0;
     if (n < (size_t)g.nzf) {
-      const C zc = buf[n >> 1];
+      const C zc = buf[lds_pos<kPadCol>((int)n >> 1)];
       v = (n & 1) ? zc.y : zc.x;
     }
     if (mode == 0) o[n] = v;
@@ -168,7 +169,7 @@ void launch_physical(const Geom& g, const NlBufs& nb, const double2* u, double2*
     phys_theta_kernel<2><<<tg2, 256, col * 2, s>>>(g, nb.pt, nb.perm_t, (const C*)nb.tw_t, u, Wt);
   else
     phys_theta_kernel<1><<<tg1, 256, col, s>>>(g, nb.pt, nb.perm_t, (const C*)nb.tw_t, u, Wt);
-  const size_t lz = size_t(g.nh) * sizeof(double2);
+  const size_t lz = size_t(lds_pos<kPadCol>(g.nh)) * sizeof(double2);
   (void)hipFuncSetAttribute((const void*)phys_z_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lz);
   phys_z_kernel<<<g.nr * g.ntp, 256, lz, s>>>(g, nb.ph, nb.perm_h, (const C*)nb.tw_h, (const C*)nb.tw_z, Wt, out,
                                              pitch, mode);

@@ -247,21 +247,44 @@ void build_radial_tables(int nr, RadialTables& T) {
   T.dr1.assign(T.D.begin() + (nr - 1) * STEN, T.D.begin() + nr * STEN);
 }
 
-// In-place DIT plan: radices 4, 2, 3, 5 in that order; perm[n] is the LDS
-// position of input sample n (mixed-radix digit reversal: the last pass's
-// radix digit of n selects the outermost block).
-bool make_fft_plan(int L, FftPlan& p, std::vector<int>& perm) {
-  p.L = L;
-  p.nrad = 0;
-  int m = L;
-  const int order[4] = {4, 2, 3, 5};
-  for (int o = 0; o < 4; o++)
-    while (m % order[o] == 0) {
-      if (p.nrad >= MAXRAD) return false;
-      p.rad[p.nrad++] = order[o];
-      m /= order[o];
+// Radices of a length (product of 2, 3, 5) that minimise the passes' cost per
+// sample (at most max_radix): the butterfly's operations plus the LDS round trip, twiddle product
+// and barrier of a pass (taken as 12 operations).  The largest radix goes
+// first, where there are no twiddles.
+bool make_fft_plan(int L, FftPlan& p, std::vector<int>& perm, int max_radix) {
+  static const struct {
+    int r;
+    double ops;  // per sample
+  } kRad[] = {{16, 10.0}, {15, 13.5}, {12, 9.7}, {10, 9.5}, {9, 9.8}, {8, 6.5}, {6, 6.3}, {5, 7.0}, {4, 4.0}, {3, 4.0}, {2, 2.0}};
+  constexpr double kPass = 12.0;
+  // best[d] = (cost, last radix) of the divisors d of L, built upwards
+  std::vector<double> best(L + 1, -1.0);
+  std::vector<int> last(L + 1, 0);
+  best[1] = 0.0;
+  for (int d = 2; d <= L; d++) {
+    if (L % d) continue;
+    for (const auto& k : kRad) {
+      if (k.r > max_radix || d % k.r || best[d / k.r] < 0.0) continue;
+      const double c = best[d / k.r] + k.ops + kPass;
+      if (best[d] < 0.0 || c < best[d]) {
+        best[d] = c;
+        last[d] = k.r;
+      }
     }
-  if (m != 1) return false;
+  }
+  if (best[L] < 0.0) return false;
+  std::vector<int> rad;
+  for (int d = L; d > 1; d /= last[d]) rad.push_back(last[d]);
+  std::sort(rad.begin(), rad.end(), [](int x, int y) { return x > y; });
+  if (rad.size() > MAXRAD) return false;
+  p.L = L;
+  p.nrad = (int)rad.size();
+  long long S = 1;
+  for (int q = 0; q < p.nrad; q++) {
+    p.rad[q] = rad[q];
+    p.mul[q] = (unsigned)(((1ll << 32) + S - 1) / S);  // S = 1: unused
+    S *= rad[q];
+  }
   perm.assign(L, 0);
   for (int n = 0; n < L; n++) {
     int pos = 0, rem = n, len = L;

@@ -291,6 +291,22 @@ def test_row_pair_z_pass(nz, prec, tol):
     p.close()
 
 
+@pytest.mark.parametrize("nt,nz", [(30, 21), (50, 25), (100, 41), (6, 49), (160, 81), (18, 91), (72, 161), (10, 181),
+                                   (4, 1351), (10, 1441), (6, 2701)])
+def test_runtime_radix_transforms(nt, nz):
+    """Lengths without compiled plans: every radix of the run-time plans, odd
+    numbers of azimuthal points, and axial lengths around the changes of the
+    samples per thread (60, 72, 120, 144, 240, 270, 480, 540, 4050, 4320, 8100)."""
+    shape = dict(nr=8, nt=nt, nz=nz, lz=4 * np.pi, re=2000.0, dt=0.005)
+    print(f"[gpu] run-time radix transforms {shape}", flush=True)
+    p = nsp.Pipe(**shape)
+    o = Oracle(**shape)
+    p.seeded_ic(SEED1, nt // 2 - 1, nz - 2, 0, 0.1)
+    u = p.get_state()
+    fields_close(p.nonlinear(*u), o.nonlinear(*u), 1e-12)
+    p.close()
+
+
 @pytest.mark.parametrize("prec,tol", [(nsp.FP64, 1e-12), (nsp.MIXED, 1e-6), (nsp.MIXED_REFINED, 1e-6)],
                          ids=["fp64", "mixed", "refined"])
 @pytest.mark.parametrize("nr", [8, 9, 10, 11, 13])
