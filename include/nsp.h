@@ -128,8 +128,7 @@ nsp_status nsp_diagnostics(nsp_handle* h, double out[7]);
  * ends), which limits NT*NZ to 4,194,304 modes: larger grids fail with
  * NSP_ERR_INVALID.  Every call on a device shares that device's array, so
  * calls that overlap on one device (several streams, threads or handles at
- * once) race.  Sums are combined in another order than nsp_diagnostics', so
- * KE and the divergence norm agree to rounding, not bit for bit. */
+ * once) race. */
 nsp_status nsp_diagnostics_noalloc(nsp_handle* h, double* out);
 
 /* Radial tables (init_fd, mod_radialFD.cu:199-312; get_dr0 :316-350;

@@ -50,7 +50,8 @@ struct nsp_handle {
   double* Luc = nullptr;    // centred Lu table
   unsigned long long* norm = nullptr;  // device [2]
   unsigned long long* norm_h = nullptr;  // pinned host [2]
-  double* part = nullptr;   // diagnostics partials [MODES][4]
+  double* out_h = nullptr;  // pinned host, written by the output kernels: 2 NZF doubles, at least NR and 7
+  double* part = nullptr;   // diagnostics partials [diag_part_count]
   // whole-step graphs: state buffers U[0..2] (u, ui, un point into them),
   // U[loc] holds the state; one graph per starting buffer
   double2* U[3] = {};
@@ -106,6 +107,8 @@ void free_all(nsp_handle* h) {
   h->allocs.clear();
   if (h->norm_h) (void)hipHostFree(h->norm_h);
   h->norm_h = nullptr;
+  if (h->out_h) (void)hipHostFree(h->out_h);
+  h->out_h = nullptr;
   if (h->stream) (void)hipStreamDestroy(h->stream);
   h->stream = nullptr;
   if (h->nb.s2) (void)hipStreamDestroy(h->nb.s2);
@@ -392,14 +395,17 @@ static nsp_status create_handle(const nsp_params* p, int device, const nsp_handl
   }
 
   // FFT plans
-  std::vector<int> perm_t, perm_h;
-  if (!make_fft_plan(g.ntp, h->nb.pt, perm_t) || !make_fft_plan(g.nh, h->nb.ph, perm_h, kZRadix))
+  std::vector<int> perm_t, perm_h, perm_f;
+  if (!make_fft_plan(g.ntp, h->nb.pt, perm_t) || !make_fft_plan(g.nh, h->nb.ph, perm_h, kZRadix) ||
+      !make_fft_plan(g.nzf, h->nb.pf, perm_f))
     return bail(fail(NSP_ERR_INVALID, "transform lengths must factor into 2, 3 and 5"));
   TRY(upload(h, &h->nb.perm_t, perm_t));
   TRY(upload(h, &h->nb.perm_h, perm_h));
+  TRY(upload(h, &h->nb.perm_f, perm_f));
   auto pass_tw = [](const FftPlan& p) { return pass_twiddles(std::vector<int>(p.rad, p.rad + p.nrad)); };
   TRY(upload(h, &h->nb.tw_t, pass_tw(h->nb.pt)));
   TRY(upload(h, &h->nb.tw_h, pass_tw(h->nb.ph)));
+  TRY(upload(h, &h->nb.tw_f, pass_tw(h->nb.pf)));
   TRY(upload(h, &h->nb.tw_z, twiddles(g.nzf, g.nh + 1)));
   h->nb.wstride = size_t(g.nr) * tp_plane(g);  // tile-major planes (tp_plane)
   h->nb.use_ct = false;
@@ -480,8 +486,9 @@ static nsp_status create_handle(const nsp_params* p, int device, const nsp_handl
   // d_r u: three tile-major components (dr_cs), FP32 pairs in the mixed form
   TRY(dalloc(h, &h->nb.dR, h->nb.mixed ? (3 * dr_cs(g) + 1) / 2 : 3 * dr_cs(g)));
   TRY(dalloc(h, &h->norm, 2));
-  TRY(dalloc(h, &h->part, 4 * size_t(g.modes)));
+  TRY(dalloc(h, &h->part, diag_part_count(g)));
   HTRY(hipHostMalloc((void**)&h->norm_h, 2 * sizeof(unsigned long long), hipHostMallocDefault));
+  HTRY(hipHostMalloc((void**)&h->out_h, std::max({2 * g.nzf, g.nr, 7}) * sizeof(double), hipHostMallocDefault));
   HTRY(hipMemsetAsync(h->u, 0, 3 * n * sizeof(double2), h->stream));
 
   // influence matrix, homogeneous solutions and flux profile (setBCon,
@@ -1091,7 +1098,7 @@ nsp_status nsp_physical_field(nsp_handle* h, int comp, double* out, int where) {
   CHECK(phys_scratch(h, &Wt, &F));
   const size_t pitch = g.nzf + 2;
   double* dst = where == NSP_DEVICE ? out : F;
-  launch_physical(g, h->nb, h->u + (size_t)comp * g.n, Wt, dst, pitch, 0, h->stream);
+  launch_physical(g, h->nb, h->u + (size_t)comp * g.n, Wt, dst, pitch, h->stream);
   HIPCHK(hipGetLastError());
   if (where == NSP_HOST)
     HIPCHK(hipMemcpyAsync(out, F, (size_t)g.nr * g.ntp * pitch * sizeof(double), hipMemcpyDeviceToHost,
@@ -1107,25 +1114,15 @@ nsp_status nsp_cross_sections(nsp_handle* h, double* q, double* u2) {
   double2* Wt;
   double* F;
   CHECK(phys_scratch(h, &Wt, &F));
-  const size_t pitch = g.nzf + 2;
-  double* q1 = reinterpret_cast<double*>(h->SP);
-  double* qd = q1 + (size_t)g.nr * g.nzf;
   if (((size_t)g.nr + 1) * g.nzf * sizeof(double) > sw_field(g) * sizeof(double2))
     return fail(NSP_ERR_INVALID, "cross-section integrals exceed the workspace");
-  for (int which = 0; which < 2; which++) {
-    double* dst = which == 0 ? q : u2;
-    if (!dst) continue;
-    if (which == 0) {  // q0kernel_k: ur^2 + ut^2
-      launch_physical(g, h->nb, h->u, Wt, F, pitch, 1, h->stream);
-      launch_physical(g, h->nb, h->u + g.n, Wt, F, pitch, 2, h->stream);
-    } else {  // u0kernel_k: uz^2
-      launch_physical(g, h->nb, h->u + 2 * g.n, Wt, F, pitch, 1, h->stream);
-    }
-    launch_cross(g, F, pitch, h->t.rdr, q1, qd, h->stream);
-    HIPCHK(hipGetLastError());
-    HIPCHK(hipMemcpyAsync(dst, qd, g.nzf * sizeof(double), hipMemcpyDeviceToHost, h->stream));
-  }
+  if (!q && !u2) return NSP_OK;
+  // q0kernel_k: ur^2 + ut^2; u0kernel_k: uz^2
+  launch_cross(g, h->nb, h->u, h->t.rdr, reinterpret_cast<double*>(Wt), 6 * sw_field(g), h->out_h, q, u2, h->stream);
+  HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(h->stream));
+  if (q) std::copy(h->out_h, h->out_h + g.nzf, q);
+  if (u2) std::copy(h->out_h + (q ? g.nzf : 0), h->out_h + (q ? 2 : 1) * g.nzf, u2);
   return NSP_OK;
 }
 
@@ -1133,10 +1130,10 @@ nsp_status nsp_mean_profile(nsp_handle* h, double* prof) {
   if (!h || !prof) return fail(NSP_ERR_INVALID, "null argument");
   HIPCHK(hipSetDevice(h->device));
   const Geom& g = h->g;
-  // real part of uz at mode (0,0) of every level (wrt_mnp_k)
-  HIPCHK(hipMemcpy2DAsync(prof, sizeof(double), h->u + 2 * g.n, g.modes * sizeof(double2), sizeof(double), g.nr,
-                          hipMemcpyDeviceToHost, h->stream));
+  launch_profile(g, h->u, h->out_h, h->stream);
+  HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(h->stream));
+  std::copy(h->out_h, h->out_h + g.nr, prof);
   return NSP_OK;
 }
 
@@ -1210,42 +1207,15 @@ nsp_status nsp_io_close(nsp_handle* h) {
 nsp_status nsp_diagnostics(nsp_handle* h, double out[7]) {
   if (!h || !out) return fail(NSP_ERR_INVALID, "null argument");
   HIPCHK(hipSetDevice(h->device));
-  const Geom& g = h->g;
-  launch_diagnostics(g, h->t, h->u, h->part, h->stream);
+  launch_diagnostics(h->g, h->t, h->u, h->part, h->out_h, h->stream);
   HIPCHK(hipGetLastError());
-  std::vector<double> part(4 * size_t(g.modes));
-  std::vector<double2> col(3 * size_t(g.nr));
-  HIPCHK(hipMemcpyAsync(part.data(), h->part, part.size() * sizeof(double), hipMemcpyDeviceToHost, h->stream));
-  // mode (0,0) uz column for the centre-line, friction and flux values
-  HIPCHK(hipMemcpy2DAsync(col.data(), sizeof(double2), h->u + 2 * g.n, g.modes * sizeof(double2), sizeof(double2),
-                          g.nr, hipMemcpyDeviceToHost, h->stream));
   HIPCHK(hipStreamSynchronize(h->stream));
-  const RadialTables& T = h->host;
-  double uc = 0.0, du = 0.0, q = 0.0;
-  for (int i = 0; i < IW + 1; i++) uc += col[i].x * T.dr0[i];  // mod_io_nonlinear.cu:45
-  for (int i = 0; i < STEN; i++) du += col[g.nr - STEN + i].x * T.dr1[i];  // :47
-  du = std::sqrt(std::fabs(du) / g.re);
-  for (int i = 0; i < g.nr; i++) q += T.rdr[i] * col[i].x;
-  double ke = 0.0, d2 = 0.0, wall = 0.0, wdiv = 0.0;
-  for (int k = 0; k < g.modes; k++) {
-    ke += part[4 * size_t(k)];
-    d2 += part[4 * size_t(k) + 1];
-    wall = std::max(wall, part[4 * size_t(k) + 2]);
-    wdiv = std::max(wdiv, part[4 * size_t(k) + 3]);
-  }
-  out[0] = uc;
-  out[1] = du;
-  out[2] = ke;
-  out[3] = std::sqrt(d2);
-  out[4] = wall;
-  out[5] = wdiv;
-  out[6] = q;
+  std::copy(h->out_h, h->out_h + 7, out);
   return NSP_OK;
 }
 
-// Same values as nsp_diagnostics, reduced entirely on the device into out
-// (device memory): no allocation, no host synchronisation, no memset (every
-// block writes its own partial set in the static scratch array).
+// nsp_diagnostics into device memory: no allocation, no host synchronisation,
+// no memset (every block writes its own partial set in the static scratch array).
 nsp_status nsp_diagnostics_noalloc(nsp_handle* h, double* out) {
   if (!h || !out) return fail(NSP_ERR_INVALID, "null argument");
   const Geom& g = h->g;
@@ -1256,7 +1226,7 @@ nsp_status nsp_diagnostics_noalloc(nsp_handle* h, double* out) {
   HIPCHK(hipSetDevice(h->device));
   double* part = diag_scratch(h->device);
   if (!part) return fail(NSP_ERR_HIP, "diagnostics scratch not initialised on this device");
-  launch_diagnostics_noalloc(g, h->t, h->u, part, out, h->stream);
+  launch_diagnostics(g, h->t, h->u, part, out, h->stream);
   HIPCHK(hipGetLastError());
   return NSP_OK;
 }

@@ -8,9 +8,10 @@
 //   * the step record and convergence-test kernels of a captured step
 //     (single pipe and ensemble), the mixed form's N(u) widening, additive
 //     perturbations;
-//   * diag_kernel: per-mode partial sums of the diagnostics.
+//   * the diagnostics' sums and maxima over the modes.
 // Column vectors of the set-up live in mode-fastest global arrays, so every
 // access of a wavefront is one contiguous 1 KiB (FP64 complex) line.
+#include <algorithm>
 #include <mutex>
 
 #include "nsp_internal.h"
@@ -391,23 +392,40 @@ __global__ __launch_bounds__(256) void setup_influence_kernel(Geom g, DevTables 
 }
 
 // ------------------------------------------------------------------ diagnostics
-// Per-mode partial sums: [0] KE, [1] |rdr|-weighted |div|^2, [2] max wall |u|,
-// [3] |wall divergence|.
-__device__ void diag_mode(const Geom& g, const DevTables& t, const double2* u, int k, double* out) {
+// Partial sums of one mode over the rows i0..i1-1: [0] KE, [1] |rdr|-weighted
+// |div|^2 and, with the last row, [2] max wall |u|, [3] |wall divergence|.
+__device__ void diag_mode(const Geom& g, const DevTables& t, const double2* u, int k, int i0, int i1, double* out) {
   const Mode q = mode_of(g, k);
   const size_t n = g.n;
   const double w = (q.l == 0) ? 1.0 : 2.0;
   double ke = 0.0, d2 = 0.0;
-  const int ip0 = abs((abs(q.m) % 2) - 1) * STEN * g.nr;
-  for (int i = 0; i < g.nr; i++) {
-    const size_t h = at(g, i, k);
-    for (int c = 0; c < 3; c++) {
-      const double2 a = u[c * n + h];
-      ke += 0.5 * w * t.rdr[i] * (a.x * a.x + a.y * a.y);
-    }
+  const double* D = t.D + abs((abs(q.m) % 2) - 1) * STEN * g.nr;
+  const double2 zero = make_double2(0.0, 0.0);
+  double2 f[STEN];  // ur of rows i-3..i+3, each read once
+#pragma unroll
+  for (int j = 0; j < STEN; j++) f[j] = i0 - IW + j >= 0 && i0 - IW + j < g.nr ? u[at(g, i0 - IW + j, k)] : zero;
+  double2 ut = u[n + at(g, i0, k)], uz = u[2 * n + at(g, i0, k)];
+  for (int i = i0; i < i1; i++) {
+    // the next row's loads in flight
+    const int ip = min(i + 1, i1 - 1);
+    const double2 un = i + 1 + IW < g.nr ? u[at(g, i + 1 + IW, k)] : zero;
+    const double2 utn = u[n + at(g, ip, k)], uzn = u[2 * n + at(g, ip, k)];
+    const double2 ur = f[IW];
+    ke += 0.5 * w * t.rdr[i] * (ur.x * ur.x + ur.y * ur.y);
+    ke += 0.5 * w * t.rdr[i] * (ut.x * ut.x + ut.y * ut.y);
+    ke += 0.5 * w * t.rdr[i] * (uz.x * uz.x + uz.y * uz.y);
     const double rK = t.r[i];
-    double2 prod = stencil(g, t.D, ip0, i, u, k);
-    const double2 ur = u[h], ut = u[n + h], uz = u[2 * n + h];
+    // derivr_k (mod_radialFD.cu:10-30): row i of D starts at its first column inside the grid
+    const int off = STEN * i + max(0, i + IW - (g.nr - 1)) - max(0, IW - i);
+    double2 prod = zero;
+#pragma unroll
+    for (int j = 0; j < STEN; j++) {
+      if (i - IW + j >= 0 && i - IW + j < g.nr) {
+        const double de = D[off + j];
+        prod.x += de * f[j].x;
+        prod.y += de * f[j].y;
+      }
+    }
     prod.x += ur.x / rK;
     prod.y += ur.y / rK;
     prod.x += -q.kt * ut.y / rK;
@@ -415,33 +433,40 @@ __device__ void diag_mode(const Geom& g, const DevTables& t, const double2* u, i
     prod.x += -q.kz * uz.y;
     prod.y += q.kz * uz.x;
     d2 += w * fabs(t.rdr[i]) * (prod.x * prod.x + prod.y * prod.y);
+#pragma unroll
+    for (int j = 0; j + 1 < STEN; j++) f[j] = f[j + 1];
+    f[STEN - 1] = un;
+    ut = utn;
+    uz = uzn;
   }
+  out[0] = ke;
+  out[1] = d2;
+  if (i1 < g.nr) return;
   double wall = 0.0;
   for (int c = 0; c < 3; c++) {
     const double2 a = u[c * n + at(g, g.nr - 1, k)];
     wall = fmax(wall, sqrt(a.x * a.x + a.y * a.y));
   }
   const double2 dw = div_wall(g, t, q, u, u + n, u + 2 * n);
-  out[0] = ke;
-  out[1] = d2;
   out[2] = wall;
   out[3] = sqrt(dw.x * dw.x + dw.y * dw.y);
 }
 
-__global__ __launch_bounds__(256) void diag_kernel(Geom g, DevTables t, const double2* u, double* part) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= g.modes) return;
-  diag_mode(g, t, u, k, part + (size_t)k * 4);
-}
-
-// Allocation-free diagnostics: the per-mode partials of a block of 256 modes
-// are combined in the block (sums of [0], [1], maxima of [2], [3]) into one
-// partial set per block, part[4 * blockIdx.x + j]; a single block then
-// combines the block partials and adds the values of the mode (0,0) column
-// (centre-line velocity, friction velocity, bulk flux: wrt_frc_k,
-// mod_io_nonlinear.cu:40-52).  Every block writes its own partial set, so
-// nothing has to start at zero.
+// A workgroup combines the partials of 256 modes over one chunk of rows (sums
+// of [0], [1], maxima of [2], [3]) into one partial set, part[4 * block + j];
+// a single workgroup then combines the sets and adds the values of the mode
+// (0,0) column (centre-line velocity, friction velocity, bulk flux: wrt_frc_k,
+// mod_io_nonlinear.cu:40-52).  Every workgroup writes its own partial set, so
+// nothing has to start at zero.  A thread's walk is one memory round trip per
+// row, so the rows are split into as many chunks as bring about 2048 workgroups
+// (eight a CU), not below four rows each (a chunk reads three rows of ur beyond
+// its ends): 48 x 96 x 513 in one chunk, without the rows of ur kept
+// in registers, took 105 us -> 39.
 constexpr int kDiagThreads = 256;
+static int diag_blocks(const Geom& g) { return (g.modes + kDiagThreads - 1) / kDiagThreads; }
+static int diag_chunks(const Geom& g) { return std::max(1, std::min(2048 / diag_blocks(g), g.nr / 4)); }
+size_t diag_part_count(const Geom& g) { return 4 * (size_t)diag_blocks(g) * diag_chunks(g); }
+
 __device__ __forceinline__ void block_combine(double (*sm)[kDiagThreads], int tid) {
   for (int s = kDiagThreads / 2; s > 0; s >>= 1) {
     if (tid < s) {
@@ -459,20 +484,25 @@ __global__ __launch_bounds__(kDiagThreads) void diag_block_kernel(Geom g, DevTab
   __shared__ double sm[4][kDiagThreads];
   const int tid = threadIdx.x;
   const int k = blockIdx.x * kDiagThreads + tid;
+  const int i0 = (int)((long long)blockIdx.y * g.nr / gridDim.y);
+  const int i1 = (int)((long long)(blockIdx.y + 1) * g.nr / gridDim.y);
   double v[4] = {0.0, 0.0, 0.0, 0.0};
-  if (k < g.modes) diag_mode(g, t, u, k, v);
+  if (k < g.modes) diag_mode(g, t, u, k, i0, i1, v);
 #pragma unroll
   for (int j = 0; j < 4; j++) sm[j][tid] = v[j];
   __syncthreads();
   block_combine(sm, tid);
-  if (tid < 4) part[4 * (size_t)blockIdx.x + tid] = sm[tid][0];
+  if (tid < 4) part[4 * ((size_t)blockIdx.y * gridDim.x + blockIdx.x) + tid] = sm[tid][0];
 }
 
+// out: seven doubles in memory the device can write (mapped host memory too)
 __global__ __launch_bounds__(kDiagThreads) void diag_final_kernel(Geom g, DevTables t, const double2* u,
                                                                    const double* part, int nblk, double* out) {
-  __shared__ double sm[4][kDiagThreads];
+  __shared__ double sm[4][kDiagThreads], flux[kDiagThreads];
   const int tid = threadIdx.x;
-  double v[4] = {0.0, 0.0, 0.0, 0.0};
+  const double2* uz = u + 2 * g.n;  // mode (0,0) of uz at level i: uz[i * modes]
+  double v[4] = {0.0, 0.0, 0.0, 0.0}, q = 0.0;
+  for (int i = tid; i < g.nr; i += kDiagThreads) q += t.rdr[i] * uz[(size_t)i * g.modes].x;
   for (int b = tid; b < nblk; b += kDiagThreads) {
     v[0] += part[4 * (size_t)b];
     v[1] += part[4 * (size_t)b + 1];
@@ -481,14 +511,14 @@ __global__ __launch_bounds__(kDiagThreads) void diag_final_kernel(Geom g, DevTab
   }
 #pragma unroll
   for (int j = 0; j < 4; j++) sm[j][tid] = v[j];
+  flux[tid] = q;
   __syncthreads();
   block_combine(sm, tid);
   if (tid == 0) {
-    const double2* uz = u + 2 * g.n;  // mode (0,0) of uz at level i: uz[i * modes]
-    double uc = 0.0, du = 0.0, q = 0.0;
+    double uc = 0.0, du = 0.0;
     for (int i = 0; i < IW + 1; i++) uc += uz[(size_t)i * g.modes].x * t.dr0[i];
     for (int i = 0; i < STEN; i++) du += uz[(size_t)(g.nr - STEN + i) * g.modes].x * t.dr1[i];
-    for (int i = 0; i < g.nr; i++) q += t.rdr[i] * uz[(size_t)i * g.modes].x;
+    for (int i = 1; i < min(g.nr, kDiagThreads); i++) q += flux[i];
     out[0] = uc;
     out[1] = sqrt(fabs(du) / g.re);
     out[2] = sm[0][0];
@@ -558,14 +588,11 @@ void launch_setup_influence(const Geom& g, const DevTables& t, const DevInfluenc
                             double* PH, hipStream_t s) {
   setup_influence_kernel<<<(g.modes + 255) / 256, 256, 0, s>>>(g, t, b, P, U, PH);
 }
-void launch_diagnostics(const Geom& g, const DevTables& t, const double2* u, double* part, hipStream_t s) {
-  diag_kernel<<<(g.modes + 255) / 256, 256, 0, s>>>(g, t, u, part);
-}
-void launch_diagnostics_noalloc(const Geom& g, const DevTables& t, const double2* u, double* part, double* out,
-                                hipStream_t s) {
-  const int nblk = (g.modes + kDiagThreads - 1) / kDiagThreads;  // <= kDiagMaxBlocks (checked by the caller)
-  diag_block_kernel<<<nblk, kDiagThreads, 0, s>>>(g, t, u, part);
-  diag_final_kernel<<<1, kDiagThreads, 0, s>>>(g, t, u, part, nblk, out);
+void launch_diagnostics(const Geom& g, const DevTables& t, const double2* u, double* part, double* out,
+                        hipStream_t s) {
+  const int nblk = diag_blocks(g), nch = diag_chunks(g);
+  diag_block_kernel<<<dim3(nblk, nch), kDiagThreads, 0, s>>>(g, t, u, part);
+  diag_final_kernel<<<1, kDiagThreads, 0, s>>>(g, t, u, part, nblk * nch, out);
 }
 
 }  // namespace nsp

@@ -274,8 +274,11 @@ struct NlBufs {
   FftPlan pt, ph;      // theta (length NTP) and half-length z (length NZF/2) plans
   int* perm_t;         // [NTP]
   int* perm_h;         // [NH]
-  double2* tw_t;       // pass twiddles of the two plans (pass_twiddles)
+  FftPlan pf;          // length NZF (output)
+  int* perm_f;         // [NZF]
+  double2* tw_t;       // pass twiddles of the plans (pass_twiddles)
   double2* tw_h;
+  double2* tw_f;       // of pf
   double2* tw_z;       // [NH+1] exp(-2 pi i k/NZF)
   double2* dR;         // [3][N] radial derivatives
   double2* W;          // [9][NR*NTP*NZ] theta-inverse intermediates
@@ -387,13 +390,15 @@ void launch_dr3(const Geom& g, const double* D, const double2* u, double2* dR, b
                 const Batch* bt = nullptr);
 
 // Physical space (output.hip): component u (one field) through the padded
-// inverse transform into out rows of `pitch` doubles (mode 0 values, 1
-// squares, 2 add squares), Wt = NR*NTP*NZ complex scratch; cross-section
-// integrals of F (NR*NTP rows) into q[NZF] with q1[NR*NZF] scratch.
+// inverse transform into out rows of `pitch` doubles, Wt = NR*NTP*NZ complex
+// scratch; cross-section integrals out[NZF] of ur^2 + ut^2 (q), then out[NZF]
+// of uz^2 (u2), with part = scratch of `room` >= 3 NZF doubles; mean axial
+// profile out[NR].
 void launch_physical(const Geom& g, const NlBufs& nb, const double2* u, double2* Wt, double* out, size_t pitch,
-                     int mode, hipStream_t s);
-void launch_cross(const Geom& g, const double* F, size_t pitch, const double* rdr, double* q1, double* q,
-                  hipStream_t s);
+                     hipStream_t s);
+void launch_cross(const Geom& g, const NlBufs& nb, const double2* u, const double* rdr, double* part, size_t room,
+                  double* out, bool q, bool u2, hipStream_t s);
+void launch_profile(const Geom& g, const double2* u, double* out, hipStream_t s);
 
 // Launchers (HIP sources).
 void launch_nonlinear(const Geom& g, const DevTables& t, const NlBufs& nb, const double2* u,
@@ -419,15 +424,17 @@ void launch_step_begin(int* st, double* err, hipStream_t s);
 void launch_converge(const unsigned long long* norm, int* st, double* err, double tol, int it, int maxit, hipStream_t s);
 void launch_setup_influence(const Geom& g, const DevTables& t, const DevInfluence& b,
                             double2* scratch_p, double* scratch_U, double* PH, hipStream_t s);
-void launch_diagnostics(const Geom& g, const DevTables& t, const double2* u, double* partial,
+// Diagnostics into out (seven doubles the device can write) with part =
+// diag_part_count doubles of scratch.
+size_t diag_part_count(const Geom& g);
+void launch_diagnostics(const Geom& g, const DevTables& t, const double2* u, double* part, double* out,
                         hipStream_t s);
-// Allocation-free diagnostics (nsp_diagnostics_noalloc): block partials of at
-// most kDiagMaxBlocks blocks of 256 modes in a static per-device array.
+// Allocation-free diagnostics (nsp_diagnostics_noalloc): the partials of at
+// most kDiagMaxBlocks blocks of 256 modes (or, in chunks of rows, 2048 blocks)
+// in a static per-device array.
 constexpr int kDiagMaxBlocks = 16384;
 constexpr int kDiagMaxModes = kDiagMaxBlocks * 256;
 hipError_t diag_scratch_init(int device);  // once per device, that device current
 double* diag_scratch(int device);          // its address on that device (null before init)
-void launch_diagnostics_noalloc(const Geom& g, const DevTables& t, const double2* u, double* part, double* out,
-                                hipStream_t s);
 
 }  // namespace nsp

@@ -1,6 +1,8 @@
 // State conversion and output kernels outside the time step: remesh onto
 // another grid (tools/Re_Mesh), physical-space fields and the cross-section
 // integrals of the reference's diagnostics files (mod_io_nonlinear.cu).
+#include <algorithm>
+
 #include "fft_device.h"
 #include "nsp_internal.h"
 
@@ -57,7 +59,10 @@ void launch_remesh(const Geom& gn, const Geom& go, const double* RM, const int2*
 // padForward_k (mod_io_nonlinear.cu:173-192) and the theta pass of the 2-D
 // inverse transform (mod_fft.cu:43-49) for one spectral component: block
 // (l-tile, i) transforms TL axial columns of level i; rows it < NT/2 go to
-// padded row it, the others to it + NT/2, rows NT/2..NT-1 stay zero.
+// padded row it, the others to it + NT/2, rows NT/2..NT-1 stay zero.  As many
+// columns as leave two workgroups a CU (launch_physical): 16 make a row's piece
+// 256 bytes and a pass's butterflies as many as the threads; 48 levels of
+// 96 x 513: 44 us with 4 columns -> 27.
 template <int TL>
 __global__ __launch_bounds__(256) void phys_theta_kernel(Geom g, FftPlan P, const int* __restrict__ perm,
                                                          const C* __restrict__ tw, const double2* __restrict__ u,
@@ -68,15 +73,11 @@ __global__ __launch_bounds__(256) void phys_theta_kernel(Geom g, FftPlan P, cons
   const int tid = threadIdx.x, nthr = blockDim.x;
   const int half = g.nt / 2;
   const double2* src = u + (size_t)i * g.modes;
-  for (int e = tid; e < g.ntp * TL; e += nthr) buf[lds_pos<TL>(e)] = C{0.0, 0.0};
-  __syncthreads();
-  for (int e = tid; e < g.nt * TL; e += nthr) {
-    const int it = e / TL, tl = e - it * TL, l = l0 + tl;
-    if (l < g.nz) {
-      const double2 v = src[(size_t)it * g.nz + l];
-      const int j = it < half ? it : it + half;
-      buf[lds_pos<TL>(perm[j] * TL + tl)] = C{v.x, v.y};
-    }
+  for (int e = tid; e < g.ntp * TL; e += nthr) {
+    const int j = e / TL, tl = e - j * TL, l = l0 + tl;
+    double2 v = make_double2(0.0, 0.0);
+    if ((j < half || j >= g.nt) && l < g.nz) v = src[(size_t)(j < half ? j : j - half) * g.nz + l];
+    buf[lds_pos<TL>(perm[j] * TL + tl)] = C{v.x, v.y};
   }
   __syncthreads();
   fft_passes<double, TL, +1>(buf, P, tw, tid, nthr);
@@ -88,97 +89,206 @@ __global__ __launch_bounds__(256) void phys_theta_kernel(Geom g, FftPlan P, cons
   }
 }
 
-// Axial real synthesis of one (i, theta) row of Wt: the NZF samples through a
-// complex transform of length NH = NZF/2 on z[m] = x[2m] + i x[2m+1]
-//   Z[k] = E + iO, E = X[k] + conj(X[NH-k]), O = (X[k] - conj(X[NH-k])) e^{+2 pi i k/NZF}
-// (imaginary parts of X[0] ignored, X[k] = 0 for k >= NZ).  Row `row` of out
-// (pitch doubles) receives the samples, then zeros up to the pitch; mode 1
-// stores their squares instead, mode 2 adds the squares.
-__global__ __launch_bounds__(256) void phys_z_kernel(Geom g, FftPlan P, const int* __restrict__ perm,
-                                                     const C* __restrict__ tw, const C* __restrict__ twz,
-                                                     const double2* __restrict__ Wt, double* __restrict__ out,
-                                                     size_t pitch, int mode) {
+// Axial real synthesis of rows 2 b and 2 b + 1 of Wt (the last may be alone) as
+// one complex transform of length NZF: with spectra X, Y (imaginary parts of
+// X[0], Y[0] ignored, zero from NZ on),
+//   Z[l] = X[l] + i Y[l],  Z[NZF-l] = conj(X[l]) + i conj(Y[l])
+// gives the samples of X as real and those of Y as imaginary parts.  A row of
+// out (pitch doubles) receives the samples, then zeros up to the pitch.  Bound
+// by the passes' LDS round trips; 6912 rows of 1536: 57 us one row a workgroup
+// (half-length transforms, radices to 5) -> 46.
+__global__ __launch_bounds__(512) void phys_z_kernel(Geom g, FftPlan P, const int* __restrict__ perm,
+                                                     const C* __restrict__ tw, const double2* __restrict__ Wt,
+                                                     double* __restrict__ out, size_t pitch) {
   extern __shared__ double2 smem[];
   C* buf = reinterpret_cast<C*>(smem);
-  const int row = blockIdx.x;
+  const int row = 2 * blockIdx.x;
+  const bool two = row + 1 < g.nr * g.ntp;
   const int tid = threadIdx.x, nthr = blockDim.x;
-  const int nh = g.nh, nz = g.nz;
+  const int nz = g.nz, nzf = g.nzf;
   const double2* X = Wt + (size_t)row * nz;
-  for (int k = tid; k < nh; k += nthr) {
-    const int kc = nh - k;
-    C a{0.0, 0.0}, b{0.0, 0.0};
-    if (k < nz) { const double2 v = X[k]; a = C{v.x, v.y}; }
-    if (kc < nz) { const double2 v = X[kc]; b = C{v.x, v.y}; }
-    if (k == 0) { a.y = 0.0; b.y = 0.0; }
-    const C E{a.x + b.x, a.y - b.y};
-    const C dlt{a.x - b.x, a.y + b.y};
-    const C w = twz[k];
-    const C O{dlt.x * w.x + dlt.y * w.y, dlt.y * w.x - dlt.x * w.y};  // dlt * conj(w)
-    buf[lds_pos<kPadCol>(perm[k])] = C{E.x - O.y, E.y + O.x};
+  for (int l = tid; l < nz; l += nthr) {
+    double2 a = X[l], b = make_double2(0.0, 0.0);
+    if (two) b = X[nz + l];
+    if (l == 0) a.y = b.y = 0.0;
+    buf[lds_pos<kPadCol>(perm[l])] = C{a.x - b.y, a.y + b.x};
+    if (l > 0) buf[lds_pos<kPadCol>(perm[nzf - l])] = C{a.x + b.y, b.x - a.y};
   }
+  for (int k = nz + tid; k <= nzf - nz; k += nthr) buf[lds_pos<kPadCol>(perm[k])] = C{0.0, 0.0};
   __syncthreads();
-  fft_passes<double, kPadCol, +1, kZRadix>(buf, P, tw, tid, nthr);
+  fft_passes<double, kPadCol, +1>(buf, P, tw, tid, nthr);
   double* o = out + (size_t)row * pitch;
-  for (size_t n = tid; n < pitch; n += nthr) {
-    double v = 0.0;
-    if (n < (size_t)g.nzf) {
-      const C zc = buf[lds_pos<kPadCol>((int)n >> 1)];
-      v = (n & 1) ? zc.y : zc.x;
+  for (int n = tid; n < (int)pitch; n += nthr) {
+    C v{0.0, 0.0};
+    if (n < nzf) v = buf[lds_pos<kPadCol>(n)];
+    o[n] = v.x;
+    if (two) o[pitch + n] = v.y;
+  }
+}
+
+// Cross-section integrals of u^2 (q0kernel_k, u0kernel_k and q1kernel_k,
+// mod_io_nonlinear.cu:54-103, intq, mod_cublasflux.cu:119-130).  The sum over
+// theta of the reference's periodic three-point rule is the mean over the NTP
+// points, and NTP >= 3 NT/2 points take the mean of a square exactly, so it
+// follows mode by mode, without the theta transform and the physical field:
+//   u(theta, n) = e_0(n) + 2 Re sum_{m>0} e^{i m theta} e_m(n),
+//   mean u^2 = |e_0|^2 + 2 sum_{m>0} |e_m|^2,
+// where e_m is the complex axial transform of the modes m and -m together,
+// S[l] = X_m[l], S[NZF-l] = conj(X_-m[l]), S[0] = (X_m[0] + conj(X_-m[0]))/2
+// (m = NT/2: only -m is stored).  A workgroup sums |e_m|^2 with the weights
+// rdr over its rows (level, m) in registers, then stores one partial row; the
+// next row's modes are in flight during a transform.  About 12 samples a
+// thread: a pass of radix 12 or 16 then has a butterfly for most threads.
+// Bound by the passes' LDS round trips at two waves a SIMD (228 registers; at
+// three, with a few of them in memory, 1.2 to 1.4 times as long).  Both
+// integrals of 48 x 96 x 513: 0.42 ms through the physical fields -> 0.096.
+template <int MPT>
+__global__ __launch_bounds__(512) void cross_kernel(Geom g, FftPlan P, const int* __restrict__ perm,
+                                                    const C* __restrict__ tw, const double2* __restrict__ u,
+                                                    const double* __restrict__ rdr, double* __restrict__ part) {
+  extern __shared__ double2 smem[];
+  C* buf = reinterpret_cast<C*>(smem);
+  const int tid = threadIdx.x, nthr = blockDim.x;
+  const int nz = g.nz, nzf = g.nzf, half = g.nt / 2, nm = half + 1, rows = g.nr * nm;
+  const double2* src = u + (size_t)blockIdx.y * g.n;
+  constexpr int LP = MPT / 3 + 1;  // LP nthr >= NZ (MPT nthr >= 3(NZ-1))
+  double2 A[LP], B[LP];
+  int pa[LP], pb[LP], pz[LP];  // LDS positions of l, NZF-l and the zeros between, the same for every row
+#pragma unroll
+  for (int q = 0; q < LP; q++) {
+    const int l = tid + q * nthr, k = nz + l;
+    pa[q] = lds_pos<kPadCol>(perm[min(l, nz - 1)]);
+    pb[q] = lds_pos<kPadCol>(perm[nzf - max(1, min(l, nz - 1))]);
+    pz[q] = k <= nzf - nz ? lds_pos<kPadCol>(perm[k]) : -1;
+  }
+  auto load = [&](int row) {
+    const int i = row / nm, m = row - i * nm;
+    const double2* lev = src + (size_t)i * g.modes;
+#pragma unroll
+    for (int q = 0; q < LP; q++) {
+      const int l = tid + q * nthr;
+      A[q] = B[q] = make_double2(0.0, 0.0);
+      if (l < nz) {
+        if (m < half) A[q] = lev[(size_t)m * nz + l];
+        B[q] = lev[(size_t)(m ? g.nt - m : 0) * nz + l];
+      }
     }
-    if (mode == 0) o[n] = v;
-    else if (mode == 1) o[n] = v * v;
-    else o[n] += v * v;
+  };
+  double acc[MPT] = {};
+  int row = blockIdx.x;
+  if (row < rows) load(row);
+  for (; row < rows; row += gridDim.x) {
+    const int i = row / nm;
+    const double w = (row == i * nm ? 1.0 : 2.0) * rdr[i];
+#pragma unroll
+    for (int q = 0; q < LP; q++) {
+      const int l = tid + q * nthr;
+      const double2 a = A[q], b = B[q];
+      if (l == 0) {
+        buf[pa[q]] = C{0.5 * (a.x + b.x), 0.5 * (a.y - b.y)};
+      } else if (l < nz) {
+        buf[pa[q]] = C{a.x, a.y};
+        buf[pb[q]] = C{b.x, -b.y};
+      }
+      if (pz[q] >= 0) buf[pz[q]] = C{0.0, 0.0};
+    }
+    if (row + (int)gridDim.x < rows) load(row + gridDim.x);
+    __syncthreads();
+    fft_passes<double, kPadCol, +1>(buf, P, tw, opaque(tid), nthr);
+#pragma unroll
+    for (int q = 0; q < MPT; q++) {
+      const int n = tid + q * nthr;
+      if (n < nzf) {
+        const C e = buf[lds_pos<kPadCol>(n)];
+        acc[q] += w * (e.x * e.x + e.y * e.y);
+      }
+    }
+    __syncthreads();
+  }
+  double* dst = part + ((size_t)blockIdx.y * gridDim.x + blockIdx.x) * nzf;
+#pragma unroll
+  for (int q = 0; q < MPT; q++) {
+    const int n = tid + q * nthr;
+    if (n < nzf) dst[n] = acc[q];
   }
 }
 
-// q1kernel_k (mod_io_nonlinear.cu:81-103) and the theta sum of intq
-// (mod_cublasflux.cu:119-130, weights qaux = 1): thread (n, i) sums the
-// periodic three-point rule 0.5/(3 NTP) (f[j-1] + 4 f[j] + f[j+1]) over j.
-__global__ __launch_bounds__(256) void cross_theta_kernel(Geom g, const double* __restrict__ F, size_t pitch,
-                                                          double* __restrict__ q1) {
-  const int n = blockIdx.x * blockDim.x + threadIdx.x;
-  const int i = blockIdx.y;
-  if (n >= g.nzf) return;
-  const double* f = F + (size_t)i * g.ntp * pitch + n;
-  const double w = 0.5 * (1.0 / (3.0 * double(g.ntp)));
+// Sums of the partial rows: out[n] over the first n0 rows, out[nzf + n] over the
+// rows n0 .. n1 (blockIdx.y).  16 samples by 16 rows at a time per workgroup.
+__global__ __launch_bounds__(256) void cross_sum_kernel(int nzf, int n0, int n1, const double* __restrict__ part,
+                                                        double* __restrict__ out) {
+  __shared__ double sm[16][17];
+  const int x = threadIdx.x & 15, y = threadIdx.x >> 4;
+  const int n = blockIdx.x * 16 + x;
+  const int b0 = blockIdx.y ? n0 : 0, b1 = blockIdx.y ? n1 : n0;
   double acc = 0.0;
-  for (int j = 0; j < g.ntp; j++) {
-    const int ja = j < 1 ? g.ntp - 1 : j - 1, jb = j > g.ntp - 2 ? 0 : j + 1;
-    acc += w * (f[(size_t)ja * pitch] + 4.0 * f[(size_t)j * pitch] + f[(size_t)jb * pitch]);
+  if (n < nzf) {
+#pragma unroll 4
+    for (int b = b0 + y; b < b1; b += 16) acc += part[(size_t)b * nzf + n];
   }
-  q1[(size_t)i * g.nzf + n] = acc;
+  sm[y][x] = acc;
+  __syncthreads();
+  if (y == 0 && n < nzf) {
+#pragma unroll
+    for (int k = 1; k < 16; k++) acc += sm[k][x];
+    out[(size_t)blockIdx.y * nzf + n] = acc;
+  }
 }
 
-// the radial sum of intq with the quadrature weights rdr
-__global__ __launch_bounds__(256) void cross_r_kernel(Geom g, const double* __restrict__ q1,
-                                                      const double* __restrict__ rdr, double* __restrict__ q) {
-  const int n = blockIdx.x * blockDim.x + threadIdx.x;
-  if (n >= g.nzf) return;
-  double acc = 0.0;
-  for (int i = 0; i < g.nr; i++) acc += q1[(size_t)i * g.nzf + n] * rdr[i];
-  q[n] = acc;
+// real part of uz at mode (0,0) of every level (wrt_mnp_k)
+__global__ __launch_bounds__(256) void profile_kernel(Geom g, const double2* __restrict__ u, double* __restrict__ out) {
+  for (int i = threadIdx.x; i < g.nr; i += blockDim.x) out[i] = u[2 * g.n + (size_t)i * g.modes].x;
+}
+
+// threads of the full-length axial kernels: about 12 samples each
+static int axial_threads(const Geom& g, int mpt) { return 64 * ((g.nzf + 64 * mpt - 1) / (64 * mpt)); }
+
+template <int TL>
+static void run_phys_theta(const Geom& g, const NlBufs& nb, const double2* u, double2* Wt, hipStream_t s) {
+  const size_t lds = size_t(g.ntp) * TL * sizeof(double2);
+  (void)hipFuncSetAttribute((const void*)phys_theta_kernel<TL>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  phys_theta_kernel<TL><<<dim3((g.nz + TL - 1) / TL, g.nr), 256, lds, s>>>(g, nb.pt, nb.perm_t, (const C*)nb.tw_t, u,
+                                                                           Wt);
 }
 
 void launch_physical(const Geom& g, const NlBufs& nb, const double2* u, double2* Wt, double* out, size_t pitch,
-                     int mode, hipStream_t s) {
-  const size_t col = size_t(g.ntp) * sizeof(double2);
-  const dim3 tg((g.nz + 3) / 4, g.nr), tg2((g.nz + 1) / 2, g.nr), tg1(g.nz, g.nr);
-  if (col * 4 <= 65536)
-    phys_theta_kernel<4><<<tg, 256, col * 4, s>>>(g, nb.pt, nb.perm_t, (const C*)nb.tw_t, u, Wt);
-  else if (col * 2 <= 65536)
-    phys_theta_kernel<2><<<tg2, 256, col * 2, s>>>(g, nb.pt, nb.perm_t, (const C*)nb.tw_t, u, Wt);
-  else
-    phys_theta_kernel<1><<<tg1, 256, col, s>>>(g, nb.pt, nb.perm_t, (const C*)nb.tw_t, u, Wt);
-  const size_t lz = size_t(lds_pos<kPadCol>(g.nh)) * sizeof(double2);
+                     hipStream_t s) {
+  const size_t col = size_t(g.ntp) * sizeof(double2), lim = 81920;  // two workgroups' LDS a CU
+  if (col * 16 <= lim) run_phys_theta<16>(g, nb, u, Wt, s);
+  else if (col * 8 <= lim) run_phys_theta<8>(g, nb, u, Wt, s);
+  else if (col * 4 <= lim) run_phys_theta<4>(g, nb, u, Wt, s);
+  else if (col * 2 <= lim) run_phys_theta<2>(g, nb, u, Wt, s);
+  else run_phys_theta<1>(g, nb, u, Wt, s);
+  const size_t lz = size_t(lds_pos<kPadCol>(g.nzf)) * sizeof(double2);
   (void)hipFuncSetAttribute((const void*)phys_z_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lz);
-  phys_z_kernel<<<g.nr * g.ntp, 256, lz, s>>>(g, nb.ph, nb.perm_h, (const C*)nb.tw_h, (const C*)nb.tw_z, Wt, out,
-                                             pitch, mode);
+  phys_z_kernel<<<(g.nr * g.ntp + 1) / 2, axial_threads(g, g.nzf > 6144 ? 18 : 12), lz, s>>>(
+      g, nb.pf, nb.perm_f, (const C*)nb.tw_f, Wt, out, pitch);
 }
 
-void launch_cross(const Geom& g, const double* F, size_t pitch, const double* rdr, double* q1, double* q,
-                  hipStream_t s) {
-  cross_theta_kernel<<<dim3((g.nzf + 255) / 256, g.nr), 256, 0, s>>>(g, F, pitch, q1);
-  cross_r_kernel<<<(g.nzf + 255) / 256, 256, 0, s>>>(g, q1, rdr, q);
+template <int MPT>
+static void run_cross(const Geom& g, const NlBufs& nb, const double2* u, const double* rdr, double* part, int blocks,
+                      int fields, hipStream_t s) {
+  const size_t lds = size_t(lds_pos<kPadCol>(g.nzf)) * sizeof(double2);
+  (void)hipFuncSetAttribute((const void*)cross_kernel<MPT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  cross_kernel<MPT><<<dim3(blocks, fields), axial_threads(g, MPT), lds, s>>>(g, nb.pf, nb.perm_f, (const C*)nb.tw_f, u,
+                                                                             rdr, part);
+}
+
+// At most 512 workgroups a field (six a CU for all three), one partial row each.
+void launch_cross(const Geom& g, const NlBufs& nb, const double2* u, const double* rdr, double* part, size_t room,
+                  double* out, bool q, bool u2, hipStream_t s) {
+  const int fields = (q ? 2 : 0) + (u2 ? 1 : 0);
+  const int blocks = (int)std::min<size_t>(std::min(512, g.nr * (g.nt / 2 + 1)), room / ((size_t)fields * g.nzf));
+  const double2* f = q ? u : u + 2 * g.n;
+  if (g.nzf <= 256) run_cross<4>(g, nb, f, rdr, part, blocks, fields, s);
+  else if (g.nzf <= 6144) run_cross<12>(g, nb, f, rdr, part, blocks, fields, s);
+  else run_cross<18>(g, nb, f, rdr, part, blocks, fields, s);
+  const int n0 = q ? 2 * blocks : blocks;
+  cross_sum_kernel<<<dim3((g.nzf + 15) / 16, q && u2 ? 2 : 1), 256, 0, s>>>(g.nzf, n0, fields * blocks, part, out);
+}
+
+void launch_profile(const Geom& g, const double2* u, double* out, hipStream_t s) {
+  profile_kernel<<<1, 256, 0, s>>>(g, u, out);
 }
 
 }  // namespace nsp

@@ -247,10 +247,10 @@ void build_radial_tables(int nr, RadialTables& T) {
   T.dr1.assign(T.D.begin() + (nr - 1) * STEN, T.D.begin() + nr * STEN);
 }
 
-// Radices of a length (product of 2, 3, 5) that minimise the passes' cost per
-// sample (at most max_radix): the butterfly's operations plus the LDS round trip, twiddle product
-// and barrier of a pass (taken as 12 operations).  The largest radix goes
-// first, where there are no twiddles.
+// Radices (at most max_radix) of a length (product of 2, 3, 5) that minimise
+// the passes' cost per sample: the butterfly's operations plus the LDS round
+// trip, twiddle product and barrier of a pass (taken as 12 operations).  The
+// largest radix goes first, where there are no twiddles.
 bool make_fft_plan(int L, FftPlan& p, std::vector<int>& perm, int max_radix) {
   static const struct {
     int r;

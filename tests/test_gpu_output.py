@@ -225,3 +225,26 @@ def test_output_leaves_the_nonlinear_workspace(prec):
     p.close()
     for c in range(3):
         assert np.array_equal(before[c], after[c])
+
+
+@pytest.mark.parametrize("nr,nt,nz", [(8, 2, 3), (9, 6, 81), (11, 10, 91), (300, 4, 5), (8, 200, 17), (8, 6, 2161),
+                                      (8, 4, 3073), (8, 768, 9), (8, 1600, 3)])
+def test_output_at_the_edges_of_its_launches(nr, nt, nz):
+    """Odd numbers of physical rows (one row without a partner), axial lengths
+    around the changes of the samples per thread (240, 270, 6480, 9216), levels
+    beyond a workgroup's threads, and each number of columns of the theta tiles."""
+    shape = dict(nr=nr, nt=nt, nz=nz, lz=2 * np.pi, re=500.0, dt=0.01)
+    print(f"[gpu] output {shape}", flush=True)
+    p, o = paired(shape, nsp.FP64, 23)
+    for c in range(3):
+        got, want = p.physical(c), o.physical(c)
+        assert rel_l2(got, want) <= 1e-12, c
+        assert np.all(got[:, :, -2:] == 0)
+    q, u2 = p.cross_sections()
+    qo, u2o = o.cross()
+    assert rel_l2(q, qo) <= 1e-12 and rel_l2(u2, u2o) <= 1e-12
+    assert np.array_equal(p.mean_profile(), p.get_state()[2][:, 0, 0].real)
+    got, want = p.diagnostics(), o.diagnostics()
+    for k in want:
+        assert abs(got[k] - want[k]) <= 1e-11 * abs(want[k]), k
+    p.close()
