@@ -137,6 +137,13 @@ __host__ __device__ __forceinline__ size_t sw_ph_count(const Geom& g) {
 // wave-uniform addresses become scalar-cache loads instead of vector loads.
 typedef const double __attribute__((address_space(4)))* ctab;
 
+// 16-byte store past the caches' usual replacement (values not read again soon;
+// p aligned to 16 bytes, as every double2 array is).
+__device__ __forceinline__ void store_nt(double2* p, double2 v) {
+  typedef double d2 __attribute__((ext_vector_type(2)));
+  __builtin_nontemporal_store(d2{v.x, v.y}, reinterpret_cast<d2*>(p));
+}
+
 // Device tables of one pipe.
 struct DevTables {
   double* r;     // [NR]

@@ -16,6 +16,15 @@ using C = cpx<double>;
 // times the old column, summed over the row's nonzero band in increasing
 // column order; other modes are zero.  ur, ut take the odd-in-r half for even
 // m, uz the even half (parity index |(|m| mod 2) - flag|, flag 1 for ur, ut).
+// A thread takes kRemeshRows new rows (blockIdx.z) with the old rows of a band
+// loaded eight at a time and the weights through the scalar cache; as one walk
+// of all rows with one load at a time the waves of present modes were a serial
+// chain while the rest only wrote zeros.  Bound by the stores (0.6 of the 0.72
+// GB of 48 x 96 x 513 to 64 x 192 x 1025): calls one after the other 322 us ->
+// 258 -> 181 with the new state stored past the caches, which so keep the old
+// rows that neighbouring chunks share (eight rows a chunk 194, sixteen 197); the
+// kernel 290 -> 205 where the new state is copied out between calls.
+constexpr int kRemeshRows = 4;
 __global__ __launch_bounds__(256) void remesh_kernel(Geom gn, Geom go, const double* __restrict__ RM,
                                                      const int2* __restrict__ band,
                                                      const double2* __restrict__ uo, double2* __restrict__ un) {
@@ -27,31 +36,42 @@ __global__ __launch_bounds__(256) void remesh_kernel(Geom gn, Geom go, const dou
   const bool src = m >= -go.nt / 2 && m < go.nt / 2 && l < go.nz;
   const int ko = src ? (m >= 0 ? m : m + go.nt) * go.nz + l : 0;
   const int par = abs((abs(m) % 2) - (c < 2 ? 1 : 0));
-  const double* R = RM + (size_t)par * gn.nr * go.nr;
+  const ctab R = ctab(RM);  // scalar loads: both parities' weights, selected per lane
+  const size_t odd = (size_t)gn.nr * go.nr;
   const double2* col = uo + (size_t)c * go.n + ko;
   double2* dst = un + (size_t)c * gn.n + k;
-  for (int i = 0; i < gn.nr; i++) {
+  const int i0 = blockIdx.z * kRemeshRows, i1 = min(i0 + kRemeshRows, gn.nr);
+  for (int i = i0; i < i1; i++) {
     double2 v = make_double2(0.0, 0.0);
     if (src) {
       const int2 bd = band[i];
-      for (int j = bd.x; j <= bd.y; j++) {
-        const double w = R[(size_t)i * go.nr + j];
-        const double2 a = col[(size_t)j * go.modes];
-        v.x += w * a.x;
-        v.y += w * a.y;
+      for (int j = bd.x; j <= bd.y; j += 8) {
+        double2 a[8];
+#pragma unroll
+        for (int q = 0; q < 8; q++)
+          if (j + q <= bd.y) a[q] = col[(size_t)(j + q) * go.modes];
+#pragma unroll
+        for (int q = 0; q < 8; q++) {
+          if (j + q <= bd.y) {
+            const size_t e = (size_t)i * go.nr + j + q;
+            const double w = par ? R[odd + e] : R[e];
+            v.x += w * a[q].x;
+            v.y += w * a[q].y;
+          }
+        }
       }
     }
     if (k == 0) {  // mode (0,0): no radial velocity, real ut and uz
       if (c == 0) v = make_double2(0.0, 0.0);
       else v.y = 0.0;
     }
-    dst[(size_t)i * gn.modes] = v;
+    store_nt(dst + (size_t)i * gn.modes, v);
   }
 }
 
 void launch_remesh(const Geom& gn, const Geom& go, const double* RM, const int2* band, const double2* uo,
                    double2* un, hipStream_t s) {
-  const dim3 grid((gn.modes + 255) / 256, 3);
+  const dim3 grid((gn.modes + 255) / 256, 3, (gn.nr + kRemeshRows - 1) / kRemeshRows);
   remesh_kernel<<<grid, 256, 0, s>>>(gn, go, RM, band, uo, un);
 }
 
