@@ -232,28 +232,41 @@ __global__ __launch_bounds__(256) void factor_kernel(Geom g, const double* __res
 // FP32 pairs.  Both are indexed with the FP64 sweep-side indices; the FP32
 // view is offset by the workgroup region's first FP64 index, so its values
 // fill the first half of the workgroup's own region.
-template <bool S32>
+// NT: streamed accesses, past the caches' usual replacement (sweep_kernel).
+template <bool S32, bool NT>
 struct Scr;
-template <>
-struct Scr<false> {
+template <bool NT>
+struct Scr<false, NT> {
   double2* p;
   __device__ static Scr at(double2* base, size_t) { return Scr{base}; }
   using V = double2;
-  __device__ V raw(size_t i) const { return p[i]; }
-  __device__ double2 ld(size_t i) const { return p[i]; }
-  __device__ void st(size_t i, double2 v) const { p[i] = v; }
+  __device__ V raw(size_t i) const {
+    if constexpr (NT) return load_nt(p + i);
+    else return p[i];
+  }
+  __device__ double2 ld(size_t i) const { return raw(i); }
+  __device__ void st(size_t i, double2 v) const {
+    if constexpr (NT) store_nt(p + i, v);
+    else p[i] = v;
+  }
 };
-template <>
-struct Scr<true> {
+template <bool NT>
+struct Scr<true, NT> {
   float2* p;
   __device__ static Scr at(double2* base, size_t region0) { return Scr{reinterpret_cast<float2*>(base) + region0}; }
   using V = float2;
-  __device__ V raw(size_t i) const { return p[i]; }
+  __device__ V raw(size_t i) const {
+    if constexpr (NT) return load_nt(p + i);
+    else return p[i];
+  }
   __device__ double2 ld(size_t i) const {
-    const float2 v = p[i];
+    const float2 v = raw(i);
     return make_double2(v.x, v.y);
   }
-  __device__ void st(size_t i, double2 v) const { p[i] = make_float2(float(v.x), float(v.y)); }
+  __device__ void st(size_t i, double2 v) const {
+    if constexpr (NT) store_nt(p + i, make_float2(float(v.x), float(v.y)));
+    else p[i] = make_float2(float(v.x), float(v.y));
+  }
 };
 
 __device__ __forceinline__ double2 wide(double2 v) { return v; }
@@ -344,7 +357,7 @@ struct Tab<1> {
 // 139 / 155 -> 117 / 117, 45x80x161 FP64 238 / 278 -> 154 / 189, 24x64x385
 // FP64 152 / 175 -> 108 / 126 and refined 161 / 148 -> 121 / 121, 64x64x513
 // mixed 370 / 409 -> 307 / 359 (a ring of 2 rows is equal, of 1 or 4 slower).
-template <int PASS, int PRED, int B, int HOLD = 0, int INC = 0, int LAT = 0>
+template <int PASS, int PRED, int B, int HOLD = 0, int INC = 0, int LAT = 0, int STR = 0>
 __global__ __launch_bounds__(128) void sweep_kernel(Lin2Args A, const Lin2Args* tab) {
   extern __shared__ double lat_tab[];  // LAT: 1/r [nr], D [2][nr][7], Lu [2][nr][7]
   if constexpr (B != 0) {
@@ -473,10 +486,18 @@ __global__ __launch_bounds__(128) void sweep_kernel(Lin2Args A, const Lin2Args* 
   constexpr bool S32 = decltype(s32_tag)::value;
   constexpr bool F32W = decltype(f32_tag)::value;
   constexpr bool N32 = decltype(n32_tag)::value;
-  const Scr<S32> SR = Scr<S32>::at(A.SR, (size_t)lb * nr * 384);
-  const Scr<S32> SP = Scr<S32>::at(A.SP, (size_t)lb * nr * 128);
-  const Scr<S32> E = Scr<S32>::at(A.E, (size_t)lb * nr * 384);
-  using SV = typename Scr<S32>::V;
+  // STR (launch_sweep2): column scratch, the solution written and the previous
+  // iterate go past the caches' usual replacement.  96 x 384 x 1537, FP32 N(u),
+  // scratch and factors, us: A (corrector) 1137 -> 1106, B 446 -> 398, C 1039 ->
+  // 941, D 1440/2030 -> 1422/1984.  Not the predictor's pass A (1704 -> 1820),
+  // and not the factors, which the two waves of a workgroup share (all passes
+  // 5-7% longer).
+  constexpr bool NT = STR && !(PASS == 0 && PRED);
+  using ScrT = Scr<S32, NT>;
+  const ScrT SR = ScrT::at(A.SR, (size_t)lb * nr * 384);
+  const ScrT SP = ScrT::at(A.SP, (size_t)lb * nr * 128);
+  const ScrT E = ScrT::at(A.E, (size_t)lb * nr * 384);
+  using SV = typename ScrT::V;
   using NV = std::conditional_t<N32, float2, double2>;
   using FT = std::conditional_t<F32W, float, double>;
   const NV* const Nv = reinterpret_cast<const NV*>(A.N);
@@ -484,7 +505,7 @@ __global__ __launch_bounds__(128) void sweep_kernel(Lin2Args A, const Lin2Args* 
 
   // ============================== pass A1 (up, INC predictor): E', Dh
   if constexpr (PASS == 4) {
-    const Scr<S32> DH = Scr<S32>::at(A.DH, (size_t)lb * nr * 128);
+    const ScrT DH = ScrT::at(A.DH, (size_t)lb * nr * 128);
     double2 uw[3][7];      // u^n +/- rows t-6..t
     double2 Hr[7];         // (H u^n)_r rows i-3..i+3
     double2 Ht[4], Hz[4];  // (H u^n)_t, (H u^n)_z rows i..i+3
@@ -596,7 +617,7 @@ __global__ __launch_bounds__(128) void sweep_kernel(Lin2Args A, const Lin2Args* 
   if constexpr (PASS == 0) {
     constexpr bool XPRED = PRED && !INC;  // INC: the predictor's explicit part comes from A1
     constexpr int LAG = XPRED ? 6 : 3;
-    const Scr<S32> DH = Scr<S32>::at(INC ? A.DH : A.SP, (size_t)lb * nr * 128);
+    const ScrT DH = ScrT::at(INC ? A.DH : A.SP, (size_t)lb * nr * 128);
     double2 uw[3][7];     // predictor: u^n +/- rows t-6..t
     double2 Rr[7];        // R_r rows i-3..i+3
     double2 Rt[4], Rz[4]; // R_t, R_z rows i..i+3
@@ -894,6 +915,10 @@ __global__ __launch_bounds__(128) void sweep_kernel(Lin2Args A, const Lin2Args* 
         xw[c][w] = z2;
         xh[c][w] = 0.0;
       }
+    auto load_d = [&](const double2* p) {
+      if constexpr (NT) return load_nt(p);
+      else return *p;
+    };
     auto backsub = [&](int i, double2* xo, double* ho) {
 #pragma unroll
       for (int c = 0; c < 3; c++) {
@@ -973,7 +998,7 @@ __global__ __launch_bounds__(128) void sweep_kernel(Lin2Args A, const Lin2Args* 
       const size_t h = (size_t)i * MS + k;
       if constexpr (!PRED) {
 #pragma unroll
-        for (int c = 0; c < 3; c++) R.uc[c] = A.u[c * n + h];
+        for (int c = 0; c < 3; c++) R.uc[c] = load_d(A.u + c * n + h);
       }
       if constexpr (INC) {
 #pragma unroll
@@ -1108,16 +1133,18 @@ __global__ __launch_bounds__(128) void sweep_kernel(Lin2Args A, const Lin2Args* 
       if (!PRED && k != 0) {  // mcor_k; mode (0,0) is measured after its fix-up
 #pragma unroll
         for (int c = 0; c < 3; c++) {
-          const double2 u1 = uc ? uc[c] : A.u[c * n + h];
+          const double2 u1 = uc ? uc[c] : load_d(A.u + c * n + h);
           const double dx = u1.x - o[c].x, dy = u1.y - o[c].y;
           const double a1 = dx * dx + dy * dy, a2 = u1.x * u1.x + u1.y * u1.y;
           num = (a1 > num || a1 != a1) ? a1 : num;
           den = (a2 > den || a2 != a2) ? a2 : den;
         }
       }
-      A.out[h] = o[0];
-      A.out[n + h] = o[1];
-      A.out[2 * n + h] = o[2];
+#pragma unroll
+      for (int c = 0; c < 3; c++) {
+        if constexpr (NT) store_nt(A.out + c * n + h, o[c]);
+        else A.out[c * n + h] = o[c];
+      }
     };
     if constexpr (LAT) {
       auto loadd = [&](int i, RowD& R) { loadrow(row_of(i), R); };
@@ -1251,13 +1278,13 @@ static void sweep_passes_inc(const Lin2Args& a, dim3 grid, hipStream_t s) {
 
 // pass D runs as HOLD = 1 for the FP64-form pipes and as HOLD = 0 for the
 // mixed-form ones (a batched launch of both forms makes both launches)
-template <int PRED, int B>
+template <int PRED, int B, int STR = 0>
 static void sweep_passes(const Lin2Args& a, const Lin2Args* tab, dim3 grid, bool fp64, bool mixed, hipStream_t s) {
-  sweep_kernel<0, PRED, B><<<grid, 128, 0, s>>>(a, tab);
-  sweep_kernel<1, PRED, B><<<grid, 128, 0, s>>>(a, tab);
-  sweep_kernel<2, PRED, B><<<grid, 128, 0, s>>>(a, tab);
-  if (fp64) sweep_kernel<3, PRED, B, 1><<<grid, 128, 0, s>>>(a, tab);
-  if (mixed) sweep_kernel<3, PRED, B, 0><<<grid, 128, 0, s>>>(a, tab);
+  sweep_kernel<0, PRED, B, 0, 0, 0, PRED ? 0 : STR><<<grid, 128, 0, s>>>(a, tab);
+  sweep_kernel<1, PRED, B, 0, 0, 0, STR><<<grid, 128, 0, s>>>(a, tab);
+  sweep_kernel<2, PRED, B, 0, 0, 0, STR><<<grid, 128, 0, s>>>(a, tab);
+  if (fp64) sweep_kernel<3, PRED, B, 1, 0, 0, STR><<<grid, 128, 0, s>>>(a, tab);
+  if (mixed) sweep_kernel<3, PRED, B, 0, 0, 0, STR><<<grid, 128, 0, s>>>(a, tab);
 }
 template <int PRED, int B>
 static void sweep_passes_lat(const Lin2Args& a, const Lin2Args* tab, dim3 grid, int nr, hipStream_t s) {
@@ -1281,6 +1308,17 @@ void launch_sweep2(const Lin2Args& a, hipStream_t s) {
     return;
   }
   const bool fp64 = a.form64 != 0;
+  // Streamed accesses where no array outlives a pass in the caches: states of
+  // more than 1 GiB, four times the 256 MB memory-side cache.  Steps of 96 x 384
+  // x 1537 (2.7 GB), by run: mixed 25.7-26.3 -> 25.5-25.6 ms, FP64 45.0-45.6 ->
+  // 43.8 (the passes themselves repeat to 1%: sweep_kernel); of 64 x 128 x 1025
+  // (0.4 GB): FP64 3.85 -> 3.81 ms but refined mixed 2.63 -> 2.74, as the kernels
+  // that follow find less of the new state in the caches.
+  if (3 * a.g.n * sizeof(double2) > (size_t(1) << 30)) {
+    if (a.predictor) sweep_passes<1, 0, 1>(a, nullptr, grid, fp64, !fp64, s);
+    else sweep_passes<0, 0, 1>(a, nullptr, grid, fp64, !fp64, s);
+    return;
+  }
   if (a.predictor) sweep_passes<1, 0>(a, nullptr, grid, fp64, !fp64, s);
   else sweep_passes<0, 0>(a, nullptr, grid, fp64, !fp64, s);
 }

@@ -137,11 +137,29 @@ __host__ __device__ __forceinline__ size_t sw_ph_count(const Geom& g) {
 // wave-uniform addresses become scalar-cache loads instead of vector loads.
 typedef const double __attribute__((address_space(4)))* ctab;
 
-// 16-byte store past the caches' usual replacement (values not read again soon;
-// p aligned to 16 bytes, as every double2 array is).
-__device__ __forceinline__ void store_nt(double2* p, double2 v) {
-  typedef double d2 __attribute__((ext_vector_type(2)));
-  __builtin_nontemporal_store(d2{v.x, v.y}, reinterpret_cast<d2*>(p));
+// Loads and stores past the caches' usual replacement (values not read again
+// soon).  A complex value is one access: p is aligned to its size, as every
+// double2 and float2 array is.
+template <typename T>
+struct StreamVec;
+template <>
+struct StreamVec<double2> {
+  typedef double type __attribute__((ext_vector_type(2)));
+};
+template <>
+struct StreamVec<float2> {
+  typedef float type __attribute__((ext_vector_type(2)));
+};
+template <typename T>
+__device__ __forceinline__ T load_nt(const T* p) {
+  using V = typename StreamVec<T>::type;
+  const V v = __builtin_nontemporal_load(reinterpret_cast<const V*>(p));
+  return T{v.x, v.y};
+}
+template <typename T>
+__device__ __forceinline__ void store_nt(T* p, T v) {
+  using V = typename StreamVec<T>::type;
+  __builtin_nontemporal_store(V{v.x, v.y}, reinterpret_cast<V*>(p));
 }
 
 // Device tables of one pipe.
