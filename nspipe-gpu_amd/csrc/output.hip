@@ -109,21 +109,24 @@ __global__ __launch_bounds__(256) void phys_theta_kernel(Geom g, FftPlan P, cons
   }
 }
 
-// Axial real synthesis of rows 2 b and 2 b + 1 of Wt (the last may be alone) as
-// one complex transform of length NZF: with spectra X, Y (imaginary parts of
-// X[0], Y[0] ignored, zero from NZ on),
+// Axial real synthesis of two rows of one level of Wt (the last of an odd
+// number is alone) as one complex transform of length NZF: with spectra X, Y
+// (imaginary parts of X[0], Y[0] ignored, zero from NZ on),
 //   Z[l] = X[l] + i Y[l],  Z[NZF-l] = conj(X[l]) + i conj(Y[l])
-// gives the samples of X as real and those of Y as imaginary parts.  A row of
-// out (pitch doubles) receives the samples, then zeros up to the pitch.  Bound
-// by the passes' LDS round trips; 6912 rows of 1536: 57 us one row a workgroup
-// (half-length transforms, radices to 5) -> 46.
+// gives the samples of X as real and those of Y as imaginary parts.  Both are
+// rounded at the scale of the larger: rows of one level are of one scale,
+// while a row of the wall's zeros beside one of the level inside would take
+// that row's rounding.  A row of out (pitch doubles) receives the samples, then
+// zeros up to the pitch.  Bound by the passes' LDS round trips; 6912 rows of
+// 1536: 57 us one row a workgroup (half-length transforms, radices to 5) -> 46.
 __global__ __launch_bounds__(512) void phys_z_kernel(Geom g, FftPlan P, const int* __restrict__ perm,
                                                      const C* __restrict__ tw, const double2* __restrict__ Wt,
                                                      double* __restrict__ out, size_t pitch) {
   extern __shared__ double2 smem[];
   C* buf = reinterpret_cast<C*>(smem);
-  const int row = 2 * blockIdx.x;
-  const bool two = row + 1 < g.nr * g.ntp;
+  const int pairs = (g.ntp + 1) / 2, lev = blockIdx.x / pairs, th = 2 * (blockIdx.x - lev * pairs);
+  const int row = lev * g.ntp + th;
+  const bool two = th + 1 < g.ntp;
   const int tid = threadIdx.x, nthr = blockDim.x;
   const int nz = g.nz, nzf = g.nzf;
   const double2* X = Wt + (size_t)row * nz;
@@ -281,7 +284,7 @@ void launch_physical(const Geom& g, const NlBufs& nb, const double2* u, double2*
   else run_phys_theta<1>(g, nb, u, Wt, s);
   const size_t lz = size_t(lds_pos<kPadCol>(g.nzf)) * sizeof(double2);
   (void)hipFuncSetAttribute((const void*)phys_z_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lz);
-  phys_z_kernel<<<(g.nr * g.ntp + 1) / 2, axial_threads(g, g.nzf > 6144 ? 18 : 12), lz, s>>>(
+  phys_z_kernel<<<g.nr * ((g.ntp + 1) / 2), axial_threads(g, g.nzf > 6144 ? 18 : 12), lz, s>>>(
       g, nb.pf, nb.perm_f, (const C*)nb.tw_f, Wt, out, pitch);
 }
 

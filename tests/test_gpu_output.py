@@ -248,3 +248,32 @@ def test_output_at_the_edges_of_its_launches(nr, nt, nz):
     for k in want:
         assert abs(got[k] - want[k]) <= 1e-11 * abs(want[k]), k
     p.close()
+
+
+@pytest.mark.parametrize("nr,nt,nz", [(8, 6, 9), (9, 6, 81), (8, 10, 17), (8, 8, 9)])
+def test_physical_rows_of_a_level_stay_apart_from_the_next(nr, nt, nz):
+    """A level's samples depend on that level alone, also where the number of
+    azimuthal points is odd (9, 15): with one level of the state nonzero the
+    others are exactly zero, as the wall's are in every no-slip state, and with
+    one level not finite the others keep their values."""
+    print(f"[gpu] physical rows by level {nr}x{nt}x{nz}", flush=True)
+    p = nsp.Pipe(nr, nt, nz, **BASE)
+    f = random_state(p, 31)
+    whole = [p.physical(c) for c in range(3)]
+    for i in (0, 3, nr - 2):
+        one = [np.zeros_like(a) for a in f]
+        holed = [a.copy() for a in f]
+        for c in range(3):
+            one[c][i] = f[c][i]
+            holed[c][i] = np.nan
+        p.set_state(*one)
+        for c in range(3):
+            got = p.physical(c)
+            assert np.all(np.delete(got, i, axis=0) == 0), (c, i)
+            assert np.array_equal(got[i], whole[c][i]), (c, i)
+        p.set_state(*holed)
+        for c in range(3):
+            got = p.physical(c)
+            assert np.array_equal(np.delete(got, i, axis=0), np.delete(whole[c], i, axis=0)), (c, i)
+            assert np.all(np.isnan(got[i, :, :-2])), (c, i)
+    p.close()
