@@ -261,7 +261,10 @@ const char* nsp_tuning(nsp_handle* h);
  * nsp_tuning's text, or just its "chosen" object.  Fails with
  * NSP_ERR_INVALID, keeping the current variants, if a named variant is not
  * compiled for this handle's sizes.  Runs one nonlinear evaluation of the
- * current state as the check. */
+ * current state as the check.  A key "s_kind" may name the kernels of the
+ * linear solves, which are chosen by the grid otherwise: 0 the general ones, 1
+ * those of small grids (NR <= 256), 2 those that stream past the caches
+ * (single pipes, not NSP_MIXED_REFINED). */
 nsp_status nsp_set_tuning(nsp_handle* h, const char* json);
 
 /* Ensembles of independent pipes (no reference counterpart: the reference runs

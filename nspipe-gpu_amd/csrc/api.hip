@@ -212,7 +212,7 @@ Lin2Args lin_args(nsp_handle* h, const Geom& g, const double2* N, const double2*
   a.norm = h->norm;
   a.predictor = predictor ? 1 : 0;
   a.ord = h->nb.var.s_ord;
-  a.lat = sweep_lat(g);
+  a.kind = sweep_kind(g, a.inc != 0, h->nb.var.s_kind);
   return a;
 }
 
@@ -239,11 +239,12 @@ std::string variant_json(const NlVariant& v) {
                   t.nthr, t.pad, t.ord);
     return std::string(o);
   };
-  char z[176];
+  char z[176], k[24] = "";
   std::snprintf(z, sizeof z,
-                ", \"z_alg\": %d, \"z_nthr\": %d, \"z_pad\": %d, \"z_pf\": %d, \"s_ord\": %d, \"nl_chunks\": %d}",
+                ", \"z_alg\": %d, \"z_nthr\": %d, \"z_pad\": %d, \"z_pf\": %d, \"s_ord\": %d, \"nl_chunks\": %d",
                 v.z_alg, v.z_nthr, v.z_pad, v.z_pf, v.s_ord, v.nl_chunks);
-  return "{\"theta_inv\": " + tvj(v.inv) + ", \"theta_fwd\": " + tvj(v.fwd) + z;
+  if (v.s_kind >= 0) std::snprintf(k, sizeof k, ", \"s_kind\": %d", v.s_kind);
+  return "{\"theta_inv\": " + tvj(v.inv) + ", \"theta_fwd\": " + tvj(v.fwd) + z + k + "}";
 }
 
 // Integer value of "key": n in text, searched from `from` (-1 if absent).
@@ -816,6 +817,10 @@ nsp_status nsp_set_tuning(nsp_handle* h, const char* json) {
   if (so >= 0) v.s_ord = so ? 1 : 0;
   const long nc = json_int(t, base, "nl_chunks");  // absent: stage after stage
   v.nl_chunks = nc >= 1 ? int(std::min<long>(nc, kNlMaxChunks)) : 1;
+  const long sk = json_int(t, base, "s_kind");  // absent: by the grid
+  v.s_kind = sk >= 0 ? int(sk) : -1;
+  if (sk >= 0 && !sweep_kind_exists(h->g, h->P.precision == NSP_MIXED_REFINED, int(std::min<long>(sk, 99))))
+    return fail(NSP_ERR_INVALID, "tuning names a sweep kind that does not exist for this grid and form");
   // accept only variants that are compiled for this size: one nonlinear
   // evaluation of the current state into the scratch of the nonlinear term
   const NlVariant old = h->nb.var;
@@ -1552,7 +1557,6 @@ struct nsp_ensemble {
   std::vector<Cls> cls;
   std::vector<int> order;          // table slot -> member
   int max_nr = 0, max_nt = 0, max_nz = 0, max_modes = 0, maxit = 0;
-  SweepExtent sweep;  // of the batched sweep launches
   double tol = 0.0;
   // device: NL tables per input role [3][M], sweep tables [3][M], records [M], norm pointers [M]
   NlMember* nl = nullptr;
@@ -1683,11 +1687,23 @@ nsp_status ens_capture(nsp_ensemble* e) {
   const int M = (int)e->m.size();
   hipStream_t s = e->stream;
   bool ok = true;
+  SweepExtent x;  // of the batched sweep launches
+  for (const nsp_handle* h : e->m) {
+    const Geom& g = h->g;
+    if (sweep_kind(g, false, h->nb.var.s_kind) == kSweepLat) {
+      x.lat_blocks = std::max(x.lat_blocks, (int)sw_nblk(g));
+      x.lat_nr = std::max(x.lat_nr, g.nr);
+    } else {
+      x.max_nt = std::max(x.max_nt, g.nt);
+      x.max_nz = std::max(x.max_nz, g.nz);
+      (h->nb.mixed ? x.mixed : x.fp64) = true;
+    }
+  }
   auto corrector = [&](int it) {
     const int role = (it % 2) ? 1 : 2;
     ok &= ens_nonlinear(e, role, s);
     launch_ens_norm_reset(e->norms, e->rec, M, s);
-    launch_sweep_batch(e->sw + role * M, M, 0, e->sweep, s);
+    launch_sweep_batch(e->sw + role * M, M, 0, x, s);
     launch_ens_converge(e->norms, e->rec, M, e->tol, it, e->maxit, s);
   };
   auto finish = [&](hipGraphExec_t* out) -> nsp_status {
@@ -1711,7 +1727,7 @@ nsp_status ens_capture(nsp_ensemble* e) {
   (void)hipMemcpyAsync(e->nl, e->stage_h, e->stage_bytes, hipMemcpyHostToDevice, s);
   launch_ens_begin(e->rec, M, s);
   ok &= ens_nonlinear(e, 0, s);
-  launch_sweep_batch(e->sw, M, 1, e->sweep, s);
+  launch_sweep_batch(e->sw, M, 1, x, s);
   if (e->maxit >= 1) corrector(1);
   nsp_status st = finish(&e->gexec);
   if (st != NSP_OK || e->maxit < 2) return st;
@@ -1777,15 +1793,6 @@ nsp_status nsp_ensemble_create(const nsp_params* params, int count, int device, 
     e->max_nt = std::max(e->max_nt, g.nt);
     e->max_nz = std::max(e->max_nz, g.nz);
     e->max_modes = std::max(e->max_modes, g.modes);
-    SweepExtent& x = e->sweep;
-    if (sweep_lat(g)) {
-      x.lat_blocks = std::max(x.lat_blocks, (int)sw_nblk(g));
-      x.lat_nr = std::max(x.lat_nr, g.nr);
-    } else {
-      x.max_nt = std::max(x.max_nt, g.nt);
-      x.max_nz = std::max(x.max_nz, g.nz);
-      (e->m[j]->nb.mixed ? x.mixed : x.fp64) = true;
-    }
   }
   for (auto& C : e->cls) {
     C.off = (int)e->order.size();

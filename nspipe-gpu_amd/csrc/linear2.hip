@@ -347,7 +347,7 @@ struct Tab<1> {
 //   C:   wall rows -u^n (so that u^n + delta vanishes there);
 //   D:   back substitution gives delta; u^n + delta takes the place of the
 //        solution from there on (wall divergence, correction, output).
-// LAT = 1 (grids with few workgroups, Lin2Args::lat): the walk is bound by the
+// LAT = 1 (grids with few workgroups, kSweepLat): the walk is bound by the
 // latency of each row's loads and of its arithmetic, not by bandwidth, and
 // registers cost nothing (less than one wave per SIMD).  Each pass then keeps
 // the loads of kLatRing rows in flight, reads the radial tables from an LDS
@@ -381,7 +381,7 @@ __global__ __launch_bounds__(128) void sweep_kernel(Lin2Args A, const Lin2Args* 
     A.SR = gmem(tab, A.SR);
     A.SP = gmem(tab, A.SP);
     A.norm = gmem(tab, A.norm);
-    if (A.lat != LAT) return;  // members of the other kind are the other launch's
+    if ((A.kind == kSweepLat) != (LAT != 0)) return;  // members of the other kind are the other launch's
     if constexpr (PASS == 3 && !LAT) {  // so are members of the other form
       // The form is tested on a copy the compiler cannot see through: knowing
       // the form past this test would let it drop the other form's paths
@@ -486,7 +486,7 @@ __global__ __launch_bounds__(128) void sweep_kernel(Lin2Args A, const Lin2Args* 
   constexpr bool S32 = decltype(s32_tag)::value;
   constexpr bool F32W = decltype(f32_tag)::value;
   constexpr bool N32 = decltype(n32_tag)::value;
-  // STR (launch_sweep2): column scratch, the solution written and the previous
+  // STR (kSweepStream): column scratch, the solution written and the previous
   // iterate go past the caches' usual replacement.  96 x 384 x 1537, FP32 N(u),
   // scratch and factors, us: A (corrector) 1137 -> 1106, B 446 -> 398, C 1039 ->
   // 941, D 1440/2030 -> 1422/1984.  Not the predictor's pass A (1704 -> 1820),
@@ -691,7 +691,7 @@ __global__ __launch_bounds__(128) void sweep_kernel(Lin2Args A, const Lin2Args* 
         double2 rh[3];
         if (XPRED) {
           // addLap_k (mod_linear.cu:12-51) on u^n, then rhs = N + that
-            const double2 nn[3] = {n0, n1, n2};
+          const double2 nn[3] = {n0, n1, n2};
 #pragma unroll
           for (int c = 0; c < 3; c++) {
             const TB Lc = Lt + (((c < 2) ? par_u : par_p) * STEN * nr + STEN * j);
@@ -1261,9 +1261,24 @@ void launch_factor(const Geom& g, const double* r, const double* Lu, const doubl
 // at 1088, 64x128x1025, the sweeps run at the memory's rate), and radial
 // tables that fit the default LDS limit.  The kind depends on the grid alone,
 // so a pipe runs the same kernels on its own and in an ensemble.
+//
+// Streamed accesses where no array outlives a pass in the caches: states of
+// more than 1 GiB, four times the 256 MB memory-side cache.  Steps of 96 x 384
+// x 1537 (2.7 GB), by run: mixed 25.7-26.3 -> 25.5-25.6 ms, FP64 45.0-45.6 ->
+// 43.8 (the passes themselves repeat to 1%: sweep_kernel); of 64 x 128 x 1025
+// (0.4 GB): FP64 3.85 -> 3.81 ms but refined mixed 2.63 -> 2.74, as the kernels
+// that follow find less of the new state in the caches.  The refined form and
+// batched launches do not stream.
 constexpr size_t kLatBlocks = 512;
 constexpr int kLatRows = 256;
-int sweep_lat(const Geom& g) { return sw_nblk(g) <= kLatBlocks && g.nr <= kLatRows ? 1 : 0; }
+bool sweep_kind_exists(const Geom& g, bool inc, int kind) {
+  return kind == kSweepPlain || (kind == kSweepLat && g.nr <= kLatRows) || (kind == kSweepStream && !inc);
+}
+int sweep_kind(const Geom& g, bool inc, int choice) {
+  if (choice >= 0 && sweep_kind_exists(g, inc, choice)) return choice;
+  if (sw_nblk(g) <= kLatBlocks && g.nr <= kLatRows) return kSweepLat;
+  return !inc && 3 * g.n * sizeof(double2) > (size_t(1) << 30) ? kSweepStream : kSweepPlain;
+}
 static size_t lat_lds(int nr) { return (size_t)nr * (1 + 4 * STEN) * sizeof(double); }
 
 template <int PRED, int LAT>
@@ -1297,24 +1312,19 @@ static void sweep_passes_lat(const Lin2Args& a, const Lin2Args* tab, dim3 grid, 
 
 void launch_sweep2(const Lin2Args& a, hipStream_t s) {
   const dim3 grid((a.g.nt / 2) * ((a.g.nz + 63) / 64));
+  const bool lat = a.kind == kSweepLat;
   if (a.inc) {
-    if (a.predictor) a.lat ? sweep_passes_inc<1, 1>(a, grid, s) : sweep_passes_inc<1, 0>(a, grid, s);
-    else a.lat ? sweep_passes_inc<0, 1>(a, grid, s) : sweep_passes_inc<0, 0>(a, grid, s);
+    if (a.predictor) lat ? sweep_passes_inc<1, 1>(a, grid, s) : sweep_passes_inc<1, 0>(a, grid, s);
+    else lat ? sweep_passes_inc<0, 1>(a, grid, s) : sweep_passes_inc<0, 0>(a, grid, s);
     return;
   }
-  if (a.lat) {
+  if (lat) {
     if (a.predictor) sweep_passes_lat<1, 0>(a, nullptr, grid, a.g.nr, s);
     else sweep_passes_lat<0, 0>(a, nullptr, grid, a.g.nr, s);
     return;
   }
   const bool fp64 = a.form64 != 0;
-  // Streamed accesses where no array outlives a pass in the caches: states of
-  // more than 1 GiB, four times the 256 MB memory-side cache.  Steps of 96 x 384
-  // x 1537 (2.7 GB), by run: mixed 25.7-26.3 -> 25.5-25.6 ms, FP64 45.0-45.6 ->
-  // 43.8 (the passes themselves repeat to 1%: sweep_kernel); of 64 x 128 x 1025
-  // (0.4 GB): FP64 3.85 -> 3.81 ms but refined mixed 2.63 -> 2.74, as the kernels
-  // that follow find less of the new state in the caches.
-  if (3 * a.g.n * sizeof(double2) > (size_t(1) << 30)) {
+  if (a.kind == kSweepStream) {
     if (a.predictor) sweep_passes<1, 0, 1>(a, nullptr, grid, fp64, !fp64, s);
     else sweep_passes<0, 0, 1>(a, nullptr, grid, fp64, !fp64, s);
     return;

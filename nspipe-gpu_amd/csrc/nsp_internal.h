@@ -242,9 +242,15 @@ struct Lin2Args {
   unsigned long long* norm;
   int predictor;
   int ord;              // block order (NlVariant::s_ord)
-  int lat;              // small grid: the LAT kernels (sweep_lat)
+  int kind;             // SweepKind
 };
-int sweep_lat(const Geom& g);  // whether a grid's sweeps run the LAT kernels (linear2.hip)
+// Kinds of the sweep kernels, of the same arithmetic: the general ones, those
+// of small grids (bound by latency) and those that stream past the caches.
+enum SweepKind { kSweepPlain = 0, kSweepLat = 1, kSweepStream = 2 };
+// The kind a grid's sweeps run (inc: refined form); choice >= 0 asks for one
+// (NlVariant::s_kind).
+int sweep_kind(const Geom& g, bool inc, int choice);
+bool sweep_kind_exists(const Geom& g, bool inc, int kind);
 // Members of a batched sweep: the largest extents of those that run the
 // bandwidth-bound kernels, whether some of them are of the FP64 or the mixed
 // form, and the largest workgroup and row counts of those that run the LAT ones.
@@ -293,6 +299,7 @@ struct NlVariant {
   int nl_chunks;  // nonlinear stage: 1 = stage after stage; K > 1 = the theta inverse and the z pass
                   // in K level chunks on two streams, the z pass of chunk c overlapping the theta
                   // inverse of chunk c + 1
+  int s_kind = -1;  // linear sweep: SweepKind asked for, -1 = by the grid (sweep_kind)
 };
 // Nonlinear-phase buffers and FFT data.
 struct NlBufs {

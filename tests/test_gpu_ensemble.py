@@ -237,3 +237,22 @@ def test_config4_full_size_ensemble_properties():
         assert d["wall_max"] < 1e-12, j
         assert abs(d["ke"] / ke0[j] - 1) < 1e-2, j
     ens.close()
+
+
+@pytest.mark.parametrize("nr,prec", [(20, nsp.FP64), (24, nsp.MIXED)], ids=["fp64", "mixed"])
+def test_streamed_sweeps_equal_the_batched_ones(nr, prec):
+    """States beyond 1 GiB: a single pipe's sweeps stream past the caches, the
+    ensemble's do not; same arithmetic, so the same bits."""
+    shape = dict(nr=nr, nt=768, nz=1537, lz=4 * np.pi, re=5300.0, dt=0.002)
+    assert 48 * nr * 768 * 1537 > 2**30
+    print(f"[gpu] streamed sweeps {shape} precision {prec}", flush=True)
+    out = []
+    for single in (True, False):
+        e = None if single else nsp.Ensemble([dict(shape, precision=prec)])
+        p = nsp.Pipe(**shape, precision=prec) if single else e.members[0]
+        p.seeded_ic(3, 8, 8, 0, 0.1)
+        (p if single else e).step(2)
+        out.append(p.get_state())
+        (p if single else e).close()
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)

@@ -780,3 +780,66 @@ def test_config3_mixed_against_fp64_hundred_steps():
         assert max(errs.values()) <= 1e-5, errs
         assert d32["wall_max"] < 1e-12 and d64["wall_max"] < 1e-12
         assert abs(d32["div_l2"] - d64["div_l2"]) <= 1e-3 * d64["div_l2"] + 1e-14
+
+
+# ---------------------------------------------------------------- kinds of the sweep kernels
+SWEEP_PLAIN, SWEEP_LAT, SWEEP_STREAM = 0, 1, 2
+FORMS = dict(fp64=(nsp.FP64, 1e-12), mixed=(nsp.MIXED, 1e-6), refined=(nsp.MIXED_REFINED, 1e-6))
+SWEEP_GRIDS = [(8, 64, 65), (13, 64, 65), (9, 96, 385)]  # two and seven chunks of axial modes, the last of one mode
+
+
+def kind_pipe(grid, form, kind, **kw):
+    p = nsp.Pipe(*grid, lz=4 * np.pi, re=2000.0, dt=0.005, precision=FORMS[form][0], **kw)
+    p.set_tuning(dict(PIPE_BASE, s_kind=kind))
+    p.seeded_ic(SEED1, 10, 20, 0, 0.1)
+    return p
+
+
+@pytest.mark.parametrize("grid", SWEEP_GRIDS, ids=lambda g: "x".join(map(str, g)))
+@pytest.mark.parametrize("form,kind", [("fp64", 0), ("fp64", 1), ("fp64", 2), ("mixed", 0), ("mixed", 1), ("mixed", 2),
+                                       ("refined", 0), ("refined", 1)])
+def test_every_sweep_kind_against_oracle(grid, form, kind):
+    """The general, small-grid and streamed sweeps of every form, on grids where
+    the rule by size would take one of them only."""
+    print(f"[gpu] sweeps kind {kind} {grid} {form}", flush=True)
+    p = kind_pipe(grid, form, kind)
+    o = Oracle(*grid, lz=4 * np.pi, re=2000.0, dt=0.005)
+    o.set_state(*p.get_state())
+    n_p, _, flags = p.step(2)
+    n_o, _ = o.step(2)
+    assert np.array_equal(n_p, n_o) and not flags.any()
+    fields_close(p.get_state(), o.get_state(), FORMS[form][1])
+    p.close()
+
+
+@pytest.mark.parametrize("form", ["fp64", "mixed"])
+def test_streamed_sweeps_equal_the_general_ones(form):
+    """Streaming past the caches changes no arithmetic: the same bits."""
+    print(f"[gpu] streamed sweeps {form}", flush=True)
+    out = []
+    for kind in (SWEEP_PLAIN, SWEEP_STREAM):
+        p = kind_pipe((24, 96, 385), form, kind, tol=1e-30, maxit=2)
+        out.append(p.step(2) + (p.get_state(),))
+        p.close()
+    assert np.array_equal(out[0][1], out[1][1])
+    for a, b in zip(out[0][3], out[1][3]):
+        assert np.array_equal(a, b)
+
+
+def test_set_tuning_rejects_missing_sweep_kind():
+    """The refined form does not stream, the small-grid kernels take NR <= 256;
+    the forms in place stay, and a choice is reported back and reread."""
+    p = kind_pipe((8, 64, 65), "refined", SWEEP_PLAIN)
+    for kind in (SWEEP_STREAM, 3, 1000):
+        with pytest.raises(nsp.NspError):
+            p.set_tuning(dict(PIPE_BASE, s_kind=kind))
+    chosen = json.loads(nsp.lib().nsp_tuning(p.h).decode())["chosen"]
+    assert chosen["s_kind"] == SWEEP_PLAIN
+    p.set_tuning(chosen)
+    p.set_tuning(PIPE_BASE)
+    assert "s_kind" not in json.loads(nsp.lib().nsp_tuning(p.h).decode())["chosen"]
+    p.close()
+    p = nsp.Pipe(257, 64, 65, lz=4 * np.pi, re=2000.0, dt=0.005)
+    with pytest.raises(nsp.NspError):
+        p.set_tuning(dict(PIPE_BASE, s_kind=SWEEP_LAT))
+    p.close()
