@@ -310,6 +310,20 @@ __device__ __forceinline__ void walk_rows(int t0, int t1, L&& load, F&& work) {
     walk_ring<PD, DIR>(ring, t0, t1, load, work);
   }
 }
+// 1/d (d > 0) as the sum of the largest double below it and the rest, and x/d
+// from it: x hi + x lo, rounded once but for 2^-104 of it, so the quotient of
+// an IEEE division except where that lies within 2^-51 of an ulp of a tie.
+// lo > 0, so that infinities and the sign of a zero come out as a division's.
+__device__ __forceinline__ double2 recip_of(double d) {
+  double hi = 1.0 / d;
+  if (__builtin_fma(-hi, d, 1.0) <= 0.0) hi = __longlong_as_double(__double_as_longlong(hi) - 1);
+  return make_double2(hi, __builtin_fma(-hi, d, 1.0) / d);
+}
+__device__ __forceinline__ double times_recip(double x, double2 r) { return __builtin_fma(x, r.x, x * r.y); }
+
+// Rounds a value where it is formed: the compiler does not fuse it with its use.
+__device__ __forceinline__ void fix(double& x) { asm volatile("" : "+v"(x)); }
+
 // A radial table: through the scalar cache, or (LAT kernels) from LDS.
 template <int LAT>
 struct Tab {
@@ -352,14 +366,17 @@ struct Tab<1> {
 // registers cost nothing (less than one wave per SIMD).  Each pass then keeps
 // the loads of kLatRing rows in flight, reads the radial tables from an LDS
 // copy (a first touch of a table row through the scalar cache is another
-// memory round trip per row) and multiplies by tabled 1/r.  Pass D holds the
-// wall rows (as HOLD = 1).  Sweeps, predictor / corrector, us: 32x64x65 FP64
-// 139 / 155 -> 117 / 117, 45x80x161 FP64 238 / 278 -> 154 / 189, 24x64x385
-// FP64 152 / 175 -> 108 / 126 and refined 161 / 148 -> 121 / 121, 64x64x513
-// mixed 370 / 409 -> 307 / 359 (a ring of 2 rows is equal, of 1 or 4 slower).
+// memory round trip per row) and multiplies by tabled reciprocals of two words
+// (recip_of; of one word, a rounding more per quotient, 24x64x65 took 92 / 93
+// instead of 94 / 95 us and larger grids the same).  Pass D holds the wall rows
+// (as HOLD = 1).  The results are the general kernels', bit for bit.
+// General / LAT, us, predictor and corrector: 24x64x65 FP64 118 / 94 and 121 /
+// 95, 64x64x385 FP64 400 / 248 and 437 / 293, refined 419 / 271 and 372 / 291,
+// 64x128x385 FP64 517 / 427 and 543 / 492, mixed 415 / 328 and 461 / 376 (a
+// ring of 2 rows is equal, of 1 or 4 slower; pass B keeps 8 rows in flight).
 template <int PASS, int PRED, int B, int HOLD = 0, int INC = 0, int LAT = 0, int STR = 0>
 __global__ __launch_bounds__(128) void sweep_kernel(Lin2Args A, const Lin2Args* tab) {
-  extern __shared__ double lat_tab[];  // LAT: 1/r [nr], D [2][nr][7], Lu [2][nr][7]
+  extern __shared__ double2 lat_tab[];  // LAT: recip_of r [nr], of r^2 [nr], D [2][nr][7], Lu [2][nr][7]
   if constexpr (B != 0) {
     A = tab[blockIdx.y];
     A.r = gmem(tab, A.r);
@@ -403,11 +420,17 @@ __global__ __launch_bounds__(128) void sweep_kernel(Lin2Args A, const Lin2Args* 
   const int it = (threadIdx.x < 64) ? pair : (pair == 0 ? nth : g.nt - pair);
   const int l = ch * 64 + (threadIdx.x & 63);
   if constexpr (LAT) {
+    constexpr bool R2 = PASS == 4 || (PASS == 0 && PRED && !INC);  // passes that divide by r^2
     const int n7 = 2 * STEN * g.nr;
-    for (int e = threadIdx.x; e < g.nr; e += 128) lat_tab[e] = 1.0 / A.r[e];
+    double* const rows = reinterpret_cast<double*>(lat_tab + 2 * g.nr);
+    for (int e = threadIdx.x; e < g.nr; e += 128) {
+      const double r = A.r[e];
+      lat_tab[e] = recip_of(r);
+      if constexpr (R2) lat_tab[g.nr + e] = recip_of(r * r);
+    }
     for (int e = threadIdx.x; e < n7; e += 128) {
-      lat_tab[g.nr + e] = A.Dc[e];
-      lat_tab[g.nr + n7 + e] = A.Luc[e];
+      rows[e] = A.Dc[e];
+      rows[n7 + e] = A.Luc[e];
     }
     __syncthreads();
   }
@@ -446,27 +469,25 @@ __global__ __launch_bounds__(128) void sweep_kernel(Lin2Args A, const Lin2Args* 
   const int par_u = __builtin_amdgcn_readfirstlane(abs((abs(q.m) % 2) - 1));  // parity table of ur, ut (u+, u-)
   const int par_p = 1 - par_u;                                                 // parity table of uz, p
   using TB = Tab<LAT>;
-  TB rt, Dt, Lt;
+  TB Dt, Lt;
   if constexpr (LAT) {
-    rt.l = lat_tab;
-    Dt.l = lat_tab + nr;
-    Lt.l = lat_tab + nr + 2 * STEN * nr;
+    Dt.l = reinterpret_cast<const double*>(lat_tab + 2 * nr);
+    Lt.l = Dt.l + 2 * STEN * nr;
   } else {
-    rt.g = ctab(A.r);
     Dt.g = ctab(A.Dc);
     Lt.g = ctab(A.Luc);
   }
   // x / r and x / r^2 at row i: the LAT kernels multiply by the tabled
-  // reciprocal (an IEEE division is a chain of a dozen dependent instructions)
+  // reciprocals (an IEEE division is a chain of a dozen dependent instructions)
   auto over_r = [&](double x, int i) -> double {
-    if constexpr (LAT) return x * rt[i];
-    else return x / rt[i];
+    if constexpr (LAT) return times_recip(x, lat_tab[i]);
+    else return x / ctab(A.r)[i];
   };
   auto over_r2 = [&](double x, int i) -> double {
     if constexpr (LAT) {
-      return x * (rt[i] * rt[i]);
+      return times_recip(x, lat_tab[nr + i]);
     } else {
-      const double r2 = rt[i] * rt[i];
+      const double r2 = ctab(A.r)[i] * ctab(A.r)[i];
       return x / r2;
     }
   };
@@ -1005,7 +1026,35 @@ __global__ __launch_bounds__(128) void sweep_kernel(Lin2Args A, const Lin2Args* 
         for (int c = 0; c < 3; c++) R.un[c] = A.un[c * n + h];
       }
     };
-    auto solve = [&](int i, const RowD& R, double2* xo, double* ho) {
+    // A row's last products x / U_ii.  LAT kernels: rounded, or fused with the
+    // sums that follow, as in the general kernels, so that all kinds give the
+    // same bits.  In the FP64 form (HOLD) the products of u+ and u-, and of the
+    // wall rows held (round_uz), are rounded: a run-time test of backsub, or the
+    // rows between, part them from their sums.  In the others all are fused, in
+    // the wall rows too, whose products are therefore formed anew (emit_wall).
+    auto product = [&](const RowD& R, int c, double2 x, bool round_uz) -> double2 {
+      x = make_double2(x.x * R.f[c][0], x.y * R.f[c][0]);
+      if constexpr (LAT && !N32) {
+        if (c < 2 || round_uz) {
+          fix(x.x);
+          fix(x.y);
+        }
+      }
+      return x;
+    };
+    auto add_un = [&](const RowD& R, double2* xo) {
+      if constexpr (INC) {  // the solution is u^n + delta (FP64)
+        double2 a = R.un[0], b = R.un[1];
+        pm_of(a, b);
+        const double2 c = R.un[2];
+        xo[0] = make_double2(xo[0].x + a.x, xo[0].y + a.y);
+        xo[1] = make_double2(xo[1].x + b.x, xo[1].y + b.y);
+        xo[2] = make_double2(xo[2].x + c.x, xo[2].y + c.y);
+      }
+    };
+    auto wall_rounds_uz = [&](int s) { return s < 3 || !PRED; };
+    // s >= 0: wall row nr - 1 - s, whose eliminated row before the product is kept in xe
+    auto solve = [&](int i, const RowD& R, double2* xo, double* ho, int s = -1, double2* xe = nullptr) {
 #pragma unroll
       for (int c = 0; c < 3; c++) {
         const double ru = R.f[c][0], u1 = R.f[c][1], u2 = R.f[c][2], u3 = R.f[c][3];
@@ -1016,7 +1065,8 @@ __global__ __launch_bounds__(128) void sweep_kernel(Lin2Args A, const Lin2Args* 
         x.y -= u2 * xw[c][1].y;
         x.x -= u3 * xw[c][2].x;
         x.y -= u3 * xw[c][2].y;
-        x = make_double2(x.x * ru, x.y * ru);
+        if (s >= 0) xe[c] = x;
+        x = product(R, c, x, s >= 0 && wall_rounds_uz(s));
         double hh = (i == nr - 1) ? 1.0 : 0.0;
         hh -= u1 * xh[c][0];
         hh -= u2 * xh[c][1];
@@ -1031,21 +1081,14 @@ __global__ __launch_bounds__(128) void sweep_kernel(Lin2Args A, const Lin2Args* 
         xo[c] = x;
         ho[c] = hh;
       }
-      if constexpr (INC) {  // the solution is u^n + delta (FP64)
-        double2 a = R.un[0], b = R.un[1];
-        pm_of(a, b);
-        const double2 c = R.un[2];
-        xo[0] = make_double2(xo[0].x + a.x, xo[0].y + a.y);
-        xo[1] = make_double2(xo[1].x + b.x, xo[1].y + b.y);
-        xo[2] = make_double2(xo[2].x + c.x, xo[2].y + c.y);
-      }
+      add_un(R, xo);
     };
     // wall divergence of the provisional solution (divWall_k on r/theta
     // form) from the four wall rows. Without HOLD the walk that emits the
     // solution repeats their back substitution (same arithmetic, same
     // values), which keeps the pass at 3 waves per SIMD instead of 2.
     double2 urw[4], utw = z2, uzw = z2;
-    double2 xs[HOLD || LAT ? 4 : 1][3];  // HOLD, LAT: wall rows NR-1..NR-4
+    double2 xs[HOLD || LAT ? 4 : 1][3];  // HOLD, LAT: wall rows NR-1..NR-4 (LAT: before the product)
     double xhs[HOLD || LAT ? 4 : 1][3];
     RowD ring[LAT ? 4 : 1];
     if constexpr (LAT) {
@@ -1056,12 +1099,12 @@ __global__ __launch_bounds__(128) void sweep_kernel(Lin2Args A, const Lin2Args* 
     for (int s = 0; s < 4; s++) {
       double2 xo[3];
       double ho[3];
-      if constexpr (LAT) solve(nr - 1 - s, ring[s], xo, ho);
+      if constexpr (LAT) solve(nr - 1 - s, ring[s], xo, ho, s, xs[s]);
       else backsub(nr - 1 - s, xo, ho);
       if constexpr (HOLD || LAT) {
 #pragma unroll
         for (int c = 0; c < 3; c++) {
-          xs[s][c] = xo[c];
+          if constexpr (!LAT) xs[s][c] = xo[c];
           xhs[s][c] = ho[c];
         }
       }
@@ -1135,7 +1178,9 @@ __global__ __launch_bounds__(128) void sweep_kernel(Lin2Args A, const Lin2Args* 
         for (int c = 0; c < 3; c++) {
           const double2 u1 = uc ? uc[c] : load_d(A.u + c * n + h);
           const double dx = u1.x - o[c].x, dy = u1.y - o[c].y;
-          const double a1 = dx * dx + dy * dy, a2 = u1.x * u1.x + u1.y * u1.y;
+          // fused the same way in every kind of kernel
+          const double a1 = N32 && c == 0 ? __builtin_fma(dy, dy, dx * dx) : __builtin_fma(dx, dx, dy * dy);
+          const double a2 = __builtin_fma(u1.x, u1.x, u1.y * u1.y);
           num = (a1 > num || a1 != a1) ? a1 : num;
           den = (a2 > den || a2 != a2) ? a2 : den;
         }
@@ -1148,11 +1193,22 @@ __global__ __launch_bounds__(128) void sweep_kernel(Lin2Args A, const Lin2Args* 
     };
     if constexpr (LAT) {
       auto loadd = [&](int i, RowD& R) { loadrow(row_of(i), R); };
+      auto emit_wall = [&](int s) {
+        double2 xo[3];
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+          fix(xs[s][c].x);
+          fix(xs[s][c].y);
+          xo[c] = product(ring[s], c, xs[s][c], wall_rounds_uz(s));
+        }
+        add_un(ring[s], xo);
+        emit(nr - 1 - s, xo, xhs[s], ring[s].pd, PRED ? nullptr : ring[s].uc);
+      };
       RowD nxt[kLatRing];
 #pragma unroll
       for (int s = 0; s < 4; s++) {
         if (s < kLatRing) loadd(nr - 5 - s, nxt[s < kLatRing ? s : 0]);
-        emit(nr - 1 - s, xs[s], xhs[s], ring[s].pd, PRED ? nullptr : ring[s].uc);
+        emit_wall(s);
       }
       walk_ring<kLatRing, -1>(nxt, nr - 5, -1, loadd, [&](int i, const RowD& R) {
         double2 xo[3];
@@ -1279,7 +1335,7 @@ int sweep_kind(const Geom& g, bool inc, int choice) {
   if (sw_nblk(g) <= kLatBlocks && g.nr <= kLatRows) return kSweepLat;
   return !inc && 3 * g.n * sizeof(double2) > (size_t(1) << 30) ? kSweepStream : kSweepPlain;
 }
-static size_t lat_lds(int nr) { return (size_t)nr * (1 + 4 * STEN) * sizeof(double); }
+static size_t lat_lds(int nr) { return (size_t)nr * (4 + 4 * STEN) * sizeof(double); }
 
 template <int PRED, int LAT>
 static void sweep_passes_inc(const Lin2Args& a, dim3 grid, hipStream_t s) {

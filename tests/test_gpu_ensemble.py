@@ -256,3 +256,27 @@ def test_streamed_sweeps_equal_the_batched_ones(nr, prec):
         (p if single else e).close()
     for a, b in zip(*out):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("kind", [0, 1], ids=["general", "small-grid"])
+def test_batched_sweeps_of_either_kind_match_single_pipes(kind):
+    """Batched sweeps of both kinds give every member the bits and convergence
+    measures of the pipe stepped alone with the general sweeps."""
+    ms = [dict(A), dict(A, nr=13), dict(A, precision=nsp.MIXED), dict(B), dict(B, precision=nsp.MIXED)]
+    ms = [dict(kw, tol=1e-30, maxit=2) for kw in ms]
+    print(f"[gpu] batched sweeps of kind {kind}", flush=True)
+    ens = nsp.Ensemble(ms)
+    for j in range(len(ms)):
+        ens[j].set_tuning(dict(PAIR_VARIANT, s_kind=kind))
+        seed_member(ens[j], j)
+    _, err_e, _ = ens.step(2)
+    for j, kw in enumerate(ms):
+        p = nsp.Pipe(**kw)
+        p.set_tuning(dict(PAIR_VARIANT, s_kind=0))
+        seed_member(p, j)
+        _, err_p, _ = p.step(2)
+        assert np.array_equal(err_p, err_e[:, j]), j
+        for a, b in zip(ens[j].get_state(), p.get_state()):
+            assert np.array_equal(a, b), j
+        p.close()
+    ens.close()

@@ -843,3 +843,21 @@ def test_set_tuning_rejects_missing_sweep_kind():
     with pytest.raises(nsp.NspError):
         p.set_tuning(dict(PIPE_BASE, s_kind=SWEEP_LAT))
     p.close()
+
+
+@pytest.mark.parametrize("grid", [(8, 64, 65), (11, 128, 65), (33, 96, 385), (256, 64, 65), (20, 192, 385)],
+                         ids=lambda g: "x".join(map(str, g)))
+@pytest.mark.parametrize("form", list(FORMS))
+def test_small_grid_sweeps_equal_the_general_ones(grid, form):
+    """The small-grid sweeps (divisions by tabled reciprocals, wall rows held, a
+    ring of rows) give the general ones' fields and convergence measures bit for
+    bit; (256, ...) has the largest tables."""
+    print(f"[gpu] small-grid against general sweeps {grid} {form}", flush=True)
+    out = []
+    for kind in (SWEEP_PLAIN, SWEEP_LAT):
+        p = kind_pipe(grid, form, kind, tol=1e-30, maxit=3)
+        out.append(p.step(2) + (p.get_state(),))
+        p.close()
+    assert np.array_equal(out[0][1], out[1][1])
+    for a, b in zip(out[0][3], out[1][3]):
+        assert np.array_equal(a, b)
