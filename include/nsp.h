@@ -264,7 +264,7 @@ const char* nsp_tuning(nsp_handle* h);
  * current state as the check.  A key "s_kind" may name the kernels of the
  * linear solves, which are chosen by the grid otherwise: 0 the general ones, 1
  * those of small grids (NR <= 256), 2 those that stream past the caches
- * (single pipes, not NSP_MIXED_REFINED). */
+ * (single pipes, not NSP_MIXED_REFINED).  All give the same bits. */
 nsp_status nsp_set_tuning(nsp_handle* h, const char* json);
 
 /* Ensembles of independent pipes (no reference counterpart: the reference runs

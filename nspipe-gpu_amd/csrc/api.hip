@@ -1687,17 +1687,16 @@ nsp_status ens_capture(nsp_ensemble* e) {
   const int M = (int)e->m.size();
   hipStream_t s = e->stream;
   bool ok = true;
-  SweepExtent x;  // of the batched sweep launches
-  for (const nsp_handle* h : e->m) {
-    const Geom& g = h->g;
-    if (sweep_kind(g, false, h->nb.var.s_kind) == kSweepLat) {
-      x.lat_blocks = std::max(x.lat_blocks, (int)sw_nblk(g));
-      x.lat_nr = std::max(x.lat_nr, g.nr);
-    } else {
-      x.max_nt = std::max(x.max_nt, g.nt);
-      x.max_nz = std::max(x.max_nz, g.nz);
-      (h->nb.mixed ? x.mixed : x.fp64) = true;
+  SweepBatch x;
+  for (int j : e->order) {
+    const nsp_handle* h = e->m[j];
+    const int choice = h->nb.var.s_kind;
+    if (sweep_kind(h->g, false, choice) != kSweepLat) {
+      x.large.add(h->g, h->nb.mixed);
+      continue;
     }
+    x.small.add(h->g, h->nb.mixed);
+    x.small_kind = sweep_batch_kind(x.small, choice);
   }
   auto corrector = [&](int it) {
     const int role = (it % 2) ? 1 : 2;

@@ -27,6 +27,8 @@
 // Scratch SR (3 complex per row) and SP (1 complex per row) carry the column
 // between passes.  Scratch, E, the factors and PH are stored per workgroup
 // (sweep-side layout, nsp_internal.h): a workgroup's column is contiguous.
+#include <algorithm>
+
 #include "nsp_internal.h"
 
 namespace nsp {
@@ -374,11 +376,14 @@ struct Tab<1> {
 // 95, 64x64x385 FP64 400 / 248 and 437 / 293, refined 419 / 271 and 372 / 291,
 // 64x128x385 FP64 517 / 427 and 543 / 492, mixed 415 / 328 and 461 / 376 (a
 // ring of 2 rows is equal, of 1 or 4 slower; pass B keeps 8 rows in flight).
+// small (B): takes the members whose own grid is small, or the others.  (In an
+// argument of its own: read from A, it made every access a flat one.)
 template <int PASS, int PRED, int B, int HOLD = 0, int INC = 0, int LAT = 0, int STR = 0>
-__global__ __launch_bounds__(128) void sweep_kernel(Lin2Args A, const Lin2Args* tab) {
+__global__ __launch_bounds__(128) void sweep_kernel(Lin2Args A, const Lin2Args* tab, int small) {
   extern __shared__ double2 lat_tab[];  // LAT: recip_of r [nr], of r^2 [nr], D [2][nr][7], Lu [2][nr][7]
   if constexpr (B != 0) {
     A = tab[blockIdx.y];
+    if ((A.kind == kSweepLat) != (small != 0)) return;  // the other launch's
     A.r = gmem(tab, A.r);
     A.rdr = gmem(tab, A.rdr);
     A.uc = gmem(tab, A.uc);
@@ -398,8 +403,7 @@ __global__ __launch_bounds__(128) void sweep_kernel(Lin2Args A, const Lin2Args* 
     A.SR = gmem(tab, A.SR);
     A.SP = gmem(tab, A.SP);
     A.norm = gmem(tab, A.norm);
-    if ((A.kind == kSweepLat) != (LAT != 0)) return;  // members of the other kind are the other launch's
-    if constexpr (PASS == 3 && !LAT) {  // so are members of the other form
+    if constexpr (PASS == 3 && !LAT) {  // members of the other form are the other launch's
       // The form is tested on a copy the compiler cannot see through: knowing
       // the form past this test would let it drop the other form's paths
       // and then contract the remaining arithmetic differently from the
@@ -1313,10 +1317,24 @@ void launch_factor(const Geom& g, const double* r, const double* Lu, const doubl
   factor_kernel<<<grid, 256, 0, s>>>(g, r, Lu, Lp, F, F32);
 }
 
-// Small grids run the LAT kernels: at most kLatBlocks workgroups (two per CU;
-// at 1088, 64x128x1025, the sweeps run at the memory's rate), and radial
-// tables that fit the default LDS limit.  The kind depends on the grid alone,
-// so a pipe runs the same kernels on its own and in an ensemble.
+// Small grids run the LAT kernels: at most kLatBlocks workgroups (two per CU)
+// and radial tables that fit the default LDS limit.  Sweeps, general / LAT, us,
+// predictor and corrector: at 448 workgroups as above; at 544 to 864 the one or
+// the other is up to a tenth faster by form and row count (64x64x1025 FP64 601 /
+// 633 and 647 / 654, mixed 496 / 574 and 554 / 535; 64x192x385 FP64 646 / 702 and
+// 683 / 723, refined 655 / 623 and 615 / 580).
+//
+// A batch's small members go in launches of their own (in one launch with the
+// larger ones the XCD order, made for the largest, would leave half the chip
+// without work of theirs: 32 x 48x96x513 and 32 x 64x128x1025 mixed 142 -> 146 ms)
+// and count their modes together, as the last chunks of axial modes are nearly
+// empty where NZ is a little above a multiple of 64: LAT up to kLatModes, 400
+// full workgroups.  Ensemble steps, general / LAT, ms: 12 x 32x64x65 (50k modes)
+// FP64 1.44 / 1.45, mixed 1.10 / 1.07, 2 x 24x64x385 (49k) FP64 1.10 / 1.06, mixed
+// 0.73 / 0.69; 2 x 64x64x513 (66k) 3.27 / 3.36 and 2.22 / 2.26, 2 x 48x96x513
+// (98k) 3.35 / 3.46 and 2.16 / 2.24, 64 x 32x64x65 6.86 / 7.17 and 4.71 / 4.84, 64
+// x 48x96x513 mixed 62.2 / 64.3.  A pipe may so run one kind alone and another
+// in an ensemble: the arithmetic, and so every bit of the results, is the same.
 //
 // Streamed accesses where no array outlives a pass in the caches: states of
 // more than 1 GiB, four times the 256 MB memory-side cache.  Steps of 96 x 384
@@ -1327,6 +1345,7 @@ void launch_factor(const Geom& g, const double* r, const double* Lu, const doubl
 // batched launches do not stream.
 constexpr size_t kLatBlocks = 512;
 constexpr int kLatRows = 256;
+constexpr size_t kLatModes = 400 * 128;
 bool sweep_kind_exists(const Geom& g, bool inc, int kind) {
   return kind == kSweepPlain || (kind == kSweepLat && g.nr <= kLatRows) || (kind == kSweepStream && !inc);
 }
@@ -1335,35 +1354,46 @@ int sweep_kind(const Geom& g, bool inc, int choice) {
   if (sw_nblk(g) <= kLatBlocks && g.nr <= kLatRows) return kSweepLat;
   return !inc && 3 * g.n * sizeof(double2) > (size_t(1) << 30) ? kSweepStream : kSweepPlain;
 }
+void SweepExtent::add(const Geom& g, bool mixed_form) {
+  max_nr = std::max(max_nr, g.nr);
+  max_nt = std::max(max_nt, g.nt);
+  max_nz = std::max(max_nz, g.nz);
+  modes += g.modes;
+  (mixed_form ? mixed : fp64) = true;
+}
+int sweep_batch_kind(const SweepExtent& small, int choice) {
+  return choice == kSweepLat || small.modes <= kLatModes ? kSweepLat : kSweepPlain;
+}
 static size_t lat_lds(int nr) { return (size_t)nr * (4 + 4 * STEN) * sizeof(double); }
 
 template <int PRED, int LAT>
 static void sweep_passes_inc(const Lin2Args& a, dim3 grid, hipStream_t s) {
   const size_t lds = LAT ? lat_lds(a.g.nr) : 0;
-  if (PRED) sweep_kernel<4, PRED, 0, 0, 1, LAT><<<grid, 128, lds, s>>>(a, nullptr);
-  sweep_kernel<0, PRED, 0, 0, 1, LAT><<<grid, 128, lds, s>>>(a, nullptr);
-  sweep_kernel<1, PRED, 0, 0, 1, LAT><<<grid, 128, lds, s>>>(a, nullptr);
-  sweep_kernel<2, PRED, 0, 0, 1, LAT><<<grid, 128, lds, s>>>(a, nullptr);
-  sweep_kernel<3, PRED, 0, 0, 1, LAT><<<grid, 128, lds, s>>>(a, nullptr);
+  if (PRED) sweep_kernel<4, PRED, 0, 0, 1, LAT><<<grid, 128, lds, s>>>(a, nullptr, 0);
+  sweep_kernel<0, PRED, 0, 0, 1, LAT><<<grid, 128, lds, s>>>(a, nullptr, 0);
+  sweep_kernel<1, PRED, 0, 0, 1, LAT><<<grid, 128, lds, s>>>(a, nullptr, 0);
+  sweep_kernel<2, PRED, 0, 0, 1, LAT><<<grid, 128, lds, s>>>(a, nullptr, 0);
+  sweep_kernel<3, PRED, 0, 0, 1, LAT><<<grid, 128, lds, s>>>(a, nullptr, 0);
 }
 
 // pass D runs as HOLD = 1 for the FP64-form pipes and as HOLD = 0 for the
 // mixed-form ones (a batched launch of both forms makes both launches)
 template <int PRED, int B, int STR = 0>
-static void sweep_passes(const Lin2Args& a, const Lin2Args* tab, dim3 grid, bool fp64, bool mixed, hipStream_t s) {
-  sweep_kernel<0, PRED, B, 0, 0, 0, PRED ? 0 : STR><<<grid, 128, 0, s>>>(a, tab);
-  sweep_kernel<1, PRED, B, 0, 0, 0, STR><<<grid, 128, 0, s>>>(a, tab);
-  sweep_kernel<2, PRED, B, 0, 0, 0, STR><<<grid, 128, 0, s>>>(a, tab);
-  if (fp64) sweep_kernel<3, PRED, B, 1, 0, 0, STR><<<grid, 128, 0, s>>>(a, tab);
-  if (mixed) sweep_kernel<3, PRED, B, 0, 0, 0, STR><<<grid, 128, 0, s>>>(a, tab);
+static void sweep_passes(const Lin2Args& a, const Lin2Args* tab, int small, dim3 grid, bool fp64, bool mixed,
+                         hipStream_t s) {
+  sweep_kernel<0, PRED, B, 0, 0, 0, PRED ? 0 : STR><<<grid, 128, 0, s>>>(a, tab, small);
+  sweep_kernel<1, PRED, B, 0, 0, 0, STR><<<grid, 128, 0, s>>>(a, tab, small);
+  sweep_kernel<2, PRED, B, 0, 0, 0, STR><<<grid, 128, 0, s>>>(a, tab, small);
+  if (fp64) sweep_kernel<3, PRED, B, 1, 0, 0, STR><<<grid, 128, 0, s>>>(a, tab, small);
+  if (mixed) sweep_kernel<3, PRED, B, 0, 0, 0, STR><<<grid, 128, 0, s>>>(a, tab, small);
 }
 template <int PRED, int B>
-static void sweep_passes_lat(const Lin2Args& a, const Lin2Args* tab, dim3 grid, int nr, hipStream_t s) {
+static void sweep_passes_lat(const Lin2Args& a, const Lin2Args* tab, int small, dim3 grid, int nr, hipStream_t s) {
   const size_t lds = lat_lds(nr);
-  sweep_kernel<0, PRED, B, 0, 0, 1><<<grid, 128, lds, s>>>(a, tab);
-  sweep_kernel<1, PRED, B, 0, 0, 1><<<grid, 128, lds, s>>>(a, tab);
-  sweep_kernel<2, PRED, B, 0, 0, 1><<<grid, 128, lds, s>>>(a, tab);
-  sweep_kernel<3, PRED, B, 0, 0, 1><<<grid, 128, lds, s>>>(a, tab);
+  sweep_kernel<0, PRED, B, 0, 0, 1><<<grid, 128, lds, s>>>(a, tab, small);
+  sweep_kernel<1, PRED, B, 0, 0, 1><<<grid, 128, lds, s>>>(a, tab, small);
+  sweep_kernel<2, PRED, B, 0, 0, 1><<<grid, 128, lds, s>>>(a, tab, small);
+  sweep_kernel<3, PRED, B, 0, 0, 1><<<grid, 128, lds, s>>>(a, tab, small);
 }
 
 void launch_sweep2(const Lin2Args& a, hipStream_t s) {
@@ -1375,31 +1405,33 @@ void launch_sweep2(const Lin2Args& a, hipStream_t s) {
     return;
   }
   if (lat) {
-    if (a.predictor) sweep_passes_lat<1, 0>(a, nullptr, grid, a.g.nr, s);
-    else sweep_passes_lat<0, 0>(a, nullptr, grid, a.g.nr, s);
+    if (a.predictor) sweep_passes_lat<1, 0>(a, nullptr, 0, grid, a.g.nr, s);
+    else sweep_passes_lat<0, 0>(a, nullptr, 0, grid, a.g.nr, s);
     return;
   }
   const bool fp64 = a.form64 != 0;
   if (a.kind == kSweepStream) {
-    if (a.predictor) sweep_passes<1, 0, 1>(a, nullptr, grid, fp64, !fp64, s);
-    else sweep_passes<0, 0, 1>(a, nullptr, grid, fp64, !fp64, s);
+    if (a.predictor) sweep_passes<1, 0, 1>(a, nullptr, 0, grid, fp64, !fp64, s);
+    else sweep_passes<0, 0, 1>(a, nullptr, 0, grid, fp64, !fp64, s);
     return;
   }
-  if (a.predictor) sweep_passes<1, 0>(a, nullptr, grid, fp64, !fp64, s);
-  else sweep_passes<0, 0>(a, nullptr, grid, fp64, !fp64, s);
+  if (a.predictor) sweep_passes<1, 0>(a, nullptr, 0, grid, fp64, !fp64, s);
+  else sweep_passes<0, 0>(a, nullptr, 0, grid, fp64, !fp64, s);
 }
 
-void launch_sweep_batch(const Lin2Args* tab, int count, int predictor, const SweepExtent& x, hipStream_t s) {
+void launch_sweep_batch(const Lin2Args* tab, int count, int predictor, const SweepBatch& b, hipStream_t s) {
   Lin2Args dummy{};
-  if (x.fp64 || x.mixed) {
+  for (const int small : {1, 0}) {
+    const SweepExtent& x = small ? b.small : b.large;
+    if (x.modes == 0) continue;
     const dim3 grid((x.max_nt / 2) * ((x.max_nz + 63) / 64), count);
-    if (predictor) sweep_passes<1, 1>(dummy, tab, grid, x.fp64, x.mixed, s);
-    else sweep_passes<0, 1>(dummy, tab, grid, x.fp64, x.mixed, s);
-  }
-  if (x.lat_nr > 0) {
-    const dim3 grid(x.lat_blocks, count);
-    if (predictor) sweep_passes_lat<1, 1>(dummy, tab, grid, x.lat_nr, s);
-    else sweep_passes_lat<0, 1>(dummy, tab, grid, x.lat_nr, s);
+    if (small && b.small_kind == kSweepLat) {
+      if (predictor) sweep_passes_lat<1, 1>(dummy, tab, small, grid, x.max_nr, s);
+      else sweep_passes_lat<0, 1>(dummy, tab, small, grid, x.max_nr, s);
+    } else {
+      if (predictor) sweep_passes<1, 1>(dummy, tab, small, grid, x.fp64, x.mixed, s);
+      else sweep_passes<0, 1>(dummy, tab, small, grid, x.fp64, x.mixed, s);
+    }
   }
 }
 

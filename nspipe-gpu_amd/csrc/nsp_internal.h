@@ -251,22 +251,29 @@ enum SweepKind { kSweepPlain = 0, kSweepLat = 1, kSweepStream = 2 };
 // (NlVariant::s_kind).
 int sweep_kind(const Geom& g, bool inc, int choice);
 bool sweep_kind_exists(const Geom& g, bool inc, int kind);
-// Members of a batched sweep: the largest extents of those that run the
-// bandwidth-bound kernels, whether some of them are of the FP64 or the mixed
-// form, and the largest workgroup and row counts of those that run the LAT ones.
+// Some members of a batched sweep: the largest extents among them, all their
+// modes and whether some are of the FP64 or the mixed form.
 struct SweepExtent {
-  int max_nt = 0, max_nz = 0;
+  int max_nr = 0, max_nt = 0, max_nz = 0;
+  size_t modes = 0;
   bool fp64 = false, mixed = false;
-  int lat_blocks = 0, lat_nr = 0;
+  void add(const Geom& g, bool mixed_form);
 };
+// A batch's members by their own grids, and the kind the small ones run
+// (kSweepPlain or kSweepLat).
+struct SweepBatch {
+  SweepExtent small, large;  // members of kind kSweepLat, the others
+  int small_kind = kSweepPlain;
+};
+int sweep_batch_kind(const SweepExtent& small, int choice);  // choice: as for sweep_kind
 // F32 (may be null): FP32 copies of the u+, u-, uz factor sets, same indices
 void launch_factor(const Geom& g, const double* r, const double* Lu, const double* Lp, double* F, float* F32,
                    hipStream_t s);
 size_t factor_count(const Geom& g);    // doubles of the stored LU factors
 size_t factor32_count(const Geom& g);  // floats of the FP32 u+, u-, uz sets
 void launch_sweep2(const Lin2Args& a, hipStream_t s);
-// one launch per pass and kind of kernel for `count` pipes (tab in device memory)
-void launch_sweep_batch(const Lin2Args* tab, int count, int predictor, const SweepExtent& x, hipStream_t s);
+// one launch per pass for the small and one for the large members of `count` pipes (tab in device memory)
+void launch_sweep_batch(const Lin2Args* tab, int count, int predictor, const SweepBatch& x, hipStream_t s);
 // centred stencil table: w-th weight of row i multiplies column i-3+w
 std::vector<double> centred_table(int nr, const std::vector<double>& T);
 
