@@ -55,3 +55,35 @@ def test_noalloc_diagnostics_match_existing_entry_point():
             p.close()
     finally:
         hip.hipFree(dev)
+
+
+# row chunks of the device reduction: 2; 3 of 13 rows; 75; 1 (more than 1024 blocks of modes)
+CHUNKED = [(8, 64, 65), (13, 20, 17), (300, 4, 5), (9, 768, 385)]
+
+
+@pytest.mark.parametrize("grid", CHUNKED, ids=lambda g: "x".join(map(str, g)))
+def test_both_diagnostics_match_the_oracle(grid):
+    """nsp_diagnostics and the allocation-free variant run the same kernels, so
+    each is held to the oracle's sums over the same state: random values at every
+    mode and level, the wall's among them.  Relative 1e-11: sums of up to 3e6
+    products of either sign, in another order."""
+    from oracle_lib import Oracle
+    hip = _hip()
+    dev = ctypes.c_void_p()
+    assert hip.hipMalloc(ctypes.byref(dev), 7 * 8) == 0
+    shape = dict(zip(("nr", "nt", "nz"), grid), lz=4 * np.pi, re=2000.0, dt=0.005)
+    print(f"[gpu] diagnostics against the oracle {shape}", flush=True)
+    p = nsp.Pipe(**shape)
+    try:
+        rng = np.random.default_rng(41)
+        u = [rng.standard_normal(p.shape) + 1j * rng.standard_normal(p.shape) for _ in range(3)]
+        p.set_state(*u)
+        o = Oracle(**shape)
+        o.set_state(*u)
+        want = o.diagnostics()
+        for got in (p.diagnostics(), _noalloc(hip, p, dev)):
+            for k in KEYS:
+                assert abs(got[k] - want[k]) <= 1e-11 * abs(want[k]), (k, got[k], want[k])
+    finally:
+        p.close()
+        hip.hipFree(dev)
