@@ -1116,14 +1116,12 @@ nsp_status nsp_cross_sections(nsp_handle* h, double* q, double* u2) {
   if (!h) return fail(NSP_ERR_INVALID, "null handle");
   HIPCHK(hipSetDevice(h->device));
   const Geom& g = h->g;
-  double2* Wt;
-  double* F;
-  CHECK(phys_scratch(h, &Wt, &F));
-  if (((size_t)g.nr + 1) * g.nzf * sizeof(double) > sw_field(g) * sizeof(double2))
-    return fail(NSP_ERR_INVALID, "cross-section integrals exceed the workspace");
+  // the partial rows of NZF doubles go to E: at least one for each of three fields
+  const size_t room = 6 * sw_field(g);
+  if (room < 3 * (size_t)g.nzf) return fail(NSP_ERR_INVALID, "cross-section integrals exceed the workspace");
   if (!q && !u2) return NSP_OK;
   // q0kernel_k: ur^2 + ut^2; u0kernel_k: uz^2
-  launch_cross(g, h->nb, h->u, h->t.rdr, reinterpret_cast<double*>(Wt), 6 * sw_field(g), h->out_h, q, u2, h->stream);
+  launch_cross(g, h->nb, h->u, h->t.rdr, reinterpret_cast<double*>(h->E), room, h->out_h, q, u2, h->stream);
   HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(h->stream));
   if (q) std::copy(h->out_h, h->out_h + g.nzf, q);
