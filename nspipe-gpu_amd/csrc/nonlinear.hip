@@ -392,7 +392,8 @@ static void theta_dispatch(const Geom& g, const DevTables& t, const NlBufs& nb, 
 template <int MPT>
 static void run_z(const Geom& g, const DevTables& t, const NlBufs& nb, hipStream_t s) {
   const size_t lds = size_t(lds_pos<kPadCol>(g.nh)) * sizeof(double2);
-  const int nthr = 64 * ((g.nzf + 64 * MPT - 1) / (64 * MPT));
+  // beyond 256 threads one workgroup fills a CU's registers: all 512
+  const int waves = (g.nzf + 64 * MPT - 1) / (64 * MPT), nthr = waves > 4 ? 512 : 64 * waves;
   (void)hipFuncSetAttribute((const void*)zpass_kernel<MPT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   zpass_kernel<MPT><<<g.nr * g.ntp, nthr, lds, s>>>(g, nb.ph, nb.perm_h, (const C*)nb.tw_h, (const C*)nb.tw_z, t.r,
                                                     nb.W, nb.wstride, nb.Y);
@@ -495,11 +496,18 @@ void launch_nonlinear(const Geom& g, const DevTables& t, const NlBufs& nb, const
   theta_dispatch(g, t, nb, u, N, s, true);
   if (pf) pf->end(s);
   if (pf) pf->begin(K_ZPASS, s);
-  // samples per thread: a row of up to 512 is one wave
+  // Samples per thread: a row of up to 512 is one wave, of up to 4608 four,
+  // which two workgroups a CU hold; longer rows take 512 threads and as few
+  // samples each as cover them.  N(u) of 16 levels of 40 x 2049 (rows of 6144), ms:
+  // 18 samples on 384 threads 1.94, 12 on 512 1.11 (24 on 256, before these
+  // kernels, 1.73); of 40 x 2401: 18 on 448 2.25, 16 on 512 1.96 (2.17).
   if (g.nzf <= 64) run_z<1>(g, t, nb, s);
   else if (g.nzf <= 128) run_z<2>(g, t, nb, s);
   else if (g.nzf <= 256) run_z<4>(g, t, nb, s);
   else if (g.nzf <= 8 * 512) run_z<8>(g, t, nb, s);
+  else if (g.nzf <= 18 * 256) run_z<18>(g, t, nb, s);
+  else if (g.nzf <= 12 * 512) run_z<12>(g, t, nb, s);
+  else if (g.nzf <= 16 * 512) run_z<16>(g, t, nb, s);
   else run_z<18>(g, t, nb, s);
   if (pf) pf->end(s);
   if (pf) pf->begin(K_THETA_FWD, s);

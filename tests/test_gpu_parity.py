@@ -861,3 +861,17 @@ def test_small_grid_sweeps_equal_the_general_ones(grid, form):
     assert np.array_equal(out[0][1], out[1][1])
     for a, b in zip(out[0][3], out[1][3]):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("nz", [1537, 1601, 2049, 2161, 2701, 2881])
+def test_long_rows_without_compiled_plans(nz):
+    """Axial lengths (4608, 4800, 6144, 6480, 8100, 8640) on both sides of each
+    change of the samples per thread of the run-time z pass."""
+    shape = dict(nr=8, nt=6, nz=nz, lz=4 * np.pi, re=2000.0, dt=0.005)
+    print(f"[gpu] long rows {shape}", flush=True)
+    p = nsp.Pipe(**shape)
+    o = Oracle(**shape)
+    p.seeded_ic(SEED1, 2, nz - 2, 0, 0.1)
+    u = p.get_state()
+    fields_close(p.nonlinear(*u), o.nonlinear(*u), 1e-12)
+    p.close()
