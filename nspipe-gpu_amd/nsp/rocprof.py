@@ -242,38 +242,43 @@ def counters(args):
 def ensemble(args):
     """Per-stage time per ensemble step from the kernel trace of a bench
     ensemble run whose last args.steps ensemble steps are the timed ones.
-    Each step starts with the batched radial derivative of u^n and has one
-    batched predictor pass A (sweep_kernel<0, 1, 1, ...>); the last `steps`
-    of those anchor the window.  Per stage: summed duration per step and the
-    number of evaluations per step (nonlinear stages: radial-derivative
-    launches, one per evaluation for all members; sweeps: pass-A launches)."""
+    Every evaluation of an ensemble step starts with one batched radial
+    derivative for all members; the one whose solves are the predictor's
+    (sweep_kernel<0, 1, 1, ...>) starts the step, and the last `steps` of those
+    anchor the window.  Per stage: summed duration per step and the number of
+    evaluations per step, however many launches an evaluation takes (small and
+    large members, or the classes of transform plans, go in launches of their
+    own)."""
     rows = []
     with open(args.trace) as f:
         for r in csv.DictReader(f):
             rows.append((int(r["Start_Timestamp"]), int(r["End_Timestamp"]), r["Kernel_Name"]))
     rows.sort()
-    pred_a = [i for i, (_, _, n) in enumerate(rows) if re.search(r"sweep_kernel<0, 1, 1", n)]
-    if len(pred_a) < args.steps:
-        raise SystemExit("fewer batched predictor launches than steps")
-    first = pred_a[-args.steps]
-    start = max(i for i in range(first) if "dr3_kernel" in rows[i][2])
-    tot, cnt = {}, {}
+    evals = []  # first row of each evaluation, and whether its solves are the predictor's
+    for i, (_, _, n) in enumerate(rows):
+        if "dr3_kernel" in n:
+            evals.append([i, False])
+        elif evals and re.search(r"sweep_kernel<0, 1, 1", n):
+            evals[-1][1] = True
+    steps = [i for i, pred in evals if pred]
+    if len(steps) < args.steps:
+        raise SystemExit("fewer batched predictor evaluations than steps")
+    start = steps[-args.steps]
+    tot = {}
     for t0, t1, n in rows[start:]:
         st = stage_of(n)
-        if st is None:
-            continue
-        tot[st] = tot.get(st, 0.0) + (t1 - t0) / 1e3
-        if "dr3_kernel" in n or re.search(r"sweep_kernel<0, ", n):
-            cnt[st] = cnt.get(st, 0) + 1
-    evals = cnt.get("dr3_kernel", 0) / args.steps
+        if st is not None:
+            tot[st] = tot.get(st, 0.0) + (t1 - t0) / 1e3
+    preds = sum(1 for i, pred in evals if i >= start and pred)
+    count = {"linear_sweep_kernel(predictor)": preds,
+             "linear_sweep_kernel(corrector)": sum(1 for i, _ in evals if i >= start) - preds}
+    every = sum(count.values())
     out = {}
     if os.path.exists(args.out):
         with open(args.out) as f:
             out = json.load(f)
-    stages = {}
-    for st, us in tot.items():
-        ev = evals if not st.startswith("linear_sweep") else cnt.get(st, 0) / args.steps
-        stages[st] = dict(us_per_step=us / args.steps, launches_per_step=ev)
+    stages = {st: dict(us_per_step=us / args.steps, launches_per_step=count.get(st, every) / args.steps)
+              for st, us in tot.items()}
     out[args.form] = dict(command=args.command, steps=args.steps, stages=stages)
     with open(args.out, "w") as f:
         json.dump(out, f, indent=1, sort_keys=True)
