@@ -376,11 +376,18 @@ struct Tab<1> {
 // 95, 64x64x385 FP64 400 / 248 and 437 / 293, refined 419 / 271 and 372 / 291,
 // 64x128x385 FP64 517 / 427 and 543 / 492, mixed 415 / 328 and 461 / 376 (a
 // ring of 2 rows is equal, of 1 or 4 slower; pass B keeps 8 rows in flight).
+// LAP: the passes that apply the Laplacian (Lu, 1/r^2).
+template <int PASS, int PRED, int INC>
+constexpr bool lat_lap() {
+  return PASS == 4 || (PASS == 0 && PRED && !INC);
+}
 // small (B): takes the members whose own grid is small, or the others.  (In an
 // argument of its own: read from A, it made every access a flat one.)
 template <int PASS, int PRED, int B, int HOLD = 0, int INC = 0, int LAT = 0, int STR = 0>
 __global__ __launch_bounds__(128) void sweep_kernel(Lin2Args A, const Lin2Args* tab, int small) {
-  extern __shared__ double2 lat_tab[];  // LAT: recip_of r [nr], of r^2 [nr], D [2][nr][7], Lu [2][nr][7]
+  // LAT, not pass B: recip_of r [nr], LAP: of r^2 [nr], D [2][nr][7], LAP: Lu [2][nr][7]
+  extern __shared__ double2 lat_tab[];
+  constexpr bool LAP = lat_lap<PASS, PRED, INC>();
   if constexpr (B != 0) {
     A = tab[blockIdx.y];
     if ((A.kind == kSweepLat) != (small != 0)) return;  // the other launch's
@@ -423,18 +430,17 @@ __global__ __launch_bounds__(128) void sweep_kernel(Lin2Args A, const Lin2Args* 
   const int nth = g.nt / 2;
   const int it = (threadIdx.x < 64) ? pair : (pair == 0 ? nth : g.nt - pair);
   const int l = ch * 64 + (threadIdx.x & 63);
-  if constexpr (LAT) {
-    constexpr bool R2 = PASS == 4 || (PASS == 0 && PRED && !INC);  // passes that divide by r^2
+  if constexpr (LAT && PASS != 1) {
     const int n7 = 2 * STEN * g.nr;
-    double* const rows = reinterpret_cast<double*>(lat_tab + 2 * g.nr);
+    double* const rows = reinterpret_cast<double*>(lat_tab + (LAP ? 2 : 1) * g.nr);
     for (int e = threadIdx.x; e < g.nr; e += 128) {
       const double r = A.r[e];
       lat_tab[e] = recip_of(r);
-      if constexpr (R2) lat_tab[g.nr + e] = recip_of(r * r);
+      if constexpr (LAP) lat_tab[g.nr + e] = recip_of(r * r);
     }
     for (int e = threadIdx.x; e < n7; e += 128) {
       rows[e] = A.Dc[e];
-      rows[n7 + e] = A.Luc[e];
+      if constexpr (LAP) rows[n7 + e] = A.Luc[e];
     }
     __syncthreads();
   }
@@ -475,7 +481,7 @@ __global__ __launch_bounds__(128) void sweep_kernel(Lin2Args A, const Lin2Args* 
   using TB = Tab<LAT>;
   TB Dt, Lt;
   if constexpr (LAT) {
-    Dt.l = reinterpret_cast<const double*>(lat_tab + 2 * nr);
+    Dt.l = reinterpret_cast<const double*>(lat_tab + (LAP ? 2 : 1) * nr);
     Lt.l = Dt.l + 2 * STEN * nr;
   } else {
     Dt.g = ctab(A.Dc);
@@ -1364,16 +1370,23 @@ void SweepExtent::add(const Geom& g, bool mixed_form) {
 int sweep_batch_kind(const SweepExtent& small, int choice) {
   return choice == kSweepLat || small.modes <= kLatModes ? kSweepLat : kSweepPlain;
 }
-static size_t lat_lds(int nr) { return (size_t)nr * (4 + 4 * STEN) * sizeof(double); }
+template <int PASS, int PRED, int INC>
+static size_t lat_lds(int nr) {
+  return PASS == 1 ? 0 : (size_t)nr * (2 + 2 * STEN) * (lat_lap<PASS, PRED, INC>() ? 2 : 1) * sizeof(double);
+}
 
+template <int PASS, int PRED, int LAT>
+static void sweep_pass_inc(const Lin2Args& a, dim3 grid, hipStream_t s) {
+  const size_t lds = LAT ? lat_lds<PASS, PRED, 1>(a.g.nr) : 0;
+  sweep_kernel<PASS, PRED, 0, 0, 1, LAT><<<grid, 128, lds, s>>>(a, nullptr, 0);
+}
 template <int PRED, int LAT>
 static void sweep_passes_inc(const Lin2Args& a, dim3 grid, hipStream_t s) {
-  const size_t lds = LAT ? lat_lds(a.g.nr) : 0;
-  if (PRED) sweep_kernel<4, PRED, 0, 0, 1, LAT><<<grid, 128, lds, s>>>(a, nullptr, 0);
-  sweep_kernel<0, PRED, 0, 0, 1, LAT><<<grid, 128, lds, s>>>(a, nullptr, 0);
-  sweep_kernel<1, PRED, 0, 0, 1, LAT><<<grid, 128, lds, s>>>(a, nullptr, 0);
-  sweep_kernel<2, PRED, 0, 0, 1, LAT><<<grid, 128, lds, s>>>(a, nullptr, 0);
-  sweep_kernel<3, PRED, 0, 0, 1, LAT><<<grid, 128, lds, s>>>(a, nullptr, 0);
+  if constexpr (PRED) sweep_pass_inc<4, PRED, LAT>(a, grid, s);
+  sweep_pass_inc<0, PRED, LAT>(a, grid, s);
+  sweep_pass_inc<1, PRED, LAT>(a, grid, s);
+  sweep_pass_inc<2, PRED, LAT>(a, grid, s);
+  sweep_pass_inc<3, PRED, LAT>(a, grid, s);
 }
 
 // pass D runs as HOLD = 1 for the FP64-form pipes and as HOLD = 0 for the
@@ -1389,11 +1402,10 @@ static void sweep_passes(const Lin2Args& a, const Lin2Args* tab, int small, dim3
 }
 template <int PRED, int B>
 static void sweep_passes_lat(const Lin2Args& a, const Lin2Args* tab, int small, dim3 grid, int nr, hipStream_t s) {
-  const size_t lds = lat_lds(nr);
-  sweep_kernel<0, PRED, B, 0, 0, 1><<<grid, 128, lds, s>>>(a, tab, small);
-  sweep_kernel<1, PRED, B, 0, 0, 1><<<grid, 128, lds, s>>>(a, tab, small);
-  sweep_kernel<2, PRED, B, 0, 0, 1><<<grid, 128, lds, s>>>(a, tab, small);
-  sweep_kernel<3, PRED, B, 0, 0, 1><<<grid, 128, lds, s>>>(a, tab, small);
+  sweep_kernel<0, PRED, B, 0, 0, 1><<<grid, 128, lat_lds<0, PRED, 0>(nr), s>>>(a, tab, small);
+  sweep_kernel<1, PRED, B, 0, 0, 1><<<grid, 128, lat_lds<1, PRED, 0>(nr), s>>>(a, tab, small);
+  sweep_kernel<2, PRED, B, 0, 0, 1><<<grid, 128, lat_lds<2, PRED, 0>(nr), s>>>(a, tab, small);
+  sweep_kernel<3, PRED, B, 0, 0, 1><<<grid, 128, lat_lds<3, PRED, 0>(nr), s>>>(a, tab, small);
 }
 
 void launch_sweep2(const Lin2Args& a, hipStream_t s) {
