@@ -7,8 +7,8 @@
 // combines r sub-transforms of length S into one of length S*r in place, so
 // no staging buffer is needed and each thread may process any number of
 // butterflies.  Radices up to 16 (make_fft_plan picks few, large ones: a pass
-// is bound by its LDS round trip and barrier, so a length of 480 takes two
-// passes of 16 and 15 with a third of 2 rather than four of 4, 4, 5, 3, 2).
+// is bound by its LDS round trip and barrier, so a length of 480 takes three
+// passes of 10, 8 and 6 rather than five of 4, 4, 2, 3 and 5).
 // Twiddles come from the per-pass tables of pass_twiddles.
 #pragma once
 

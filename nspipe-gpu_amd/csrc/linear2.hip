@@ -1343,12 +1343,13 @@ void launch_factor(const Geom& g, const double* r, const double* Lu, const doubl
 // in an ensemble: the arithmetic, and so every bit of the results, is the same.
 //
 // Streamed accesses where no array outlives a pass in the caches: states of
-// more than 1 GiB, four times the 256 MB memory-side cache.  Steps of 96 x 384
-// x 1537 (2.7 GB), by run: mixed 25.7-26.3 -> 25.5-25.6 ms, FP64 45.0-45.6 ->
-// 43.8 (the passes themselves repeat to 1%: sweep_kernel); of 64 x 128 x 1025
-// (0.4 GB): FP64 3.85 -> 3.81 ms but refined mixed 2.63 -> 2.74, as the kernels
-// that follow find less of the new state in the caches.  The refined form and
-// batched launches do not stream.
+// more than 1 GiB, four times the 256 MB memory-side cache.  Steps of one pipe,
+// general and streamed in turn, ms: 96 x 384 x 1537 (2.5 GiB) FP64 45.1 -> 44.5,
+// mixed 25.9 -> 25.4; 48 x 384 x 1537 (1.3 GiB) 22.7 -> 22.4 and 13.0 -> 12.8; 40 x
+// 384 x 1537 (1.06 GiB) mixed 10.9 -> 10.75; of 64 x 128 x 1025 (0.4 GB): FP64 3.85
+// -> 3.81 ms but refined mixed 2.63 -> 2.74, as the kernels that follow find less
+// of the new state in the caches.  The refined form and batched launches do
+// not stream (not measured above the limit).
 constexpr size_t kLatBlocks = 512;
 constexpr int kLatRows = 256;
 constexpr size_t kLatModes = 400 * 128;
