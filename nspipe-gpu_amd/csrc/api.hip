@@ -213,6 +213,7 @@ Lin2Args lin_args(nsp_handle* h, const Geom& g, const double2* N, const double2*
   a.predictor = predictor ? 1 : 0;
   a.ord = h->nb.var.s_ord;
   a.kind = sweep_kind(g, a.inc != 0, h->nb.var.s_kind);
+  a.small = sweep_small(g);
   return a;
 }
 
@@ -1686,16 +1687,7 @@ nsp_status ens_capture(nsp_ensemble* e) {
   hipStream_t s = e->stream;
   bool ok = true;
   SweepBatch x;
-  for (int j : e->order) {
-    const nsp_handle* h = e->m[j];
-    const int choice = h->nb.var.s_kind;
-    if (sweep_kind(h->g, false, choice) != kSweepLat) {
-      x.large.add(h->g, h->nb.mixed);
-      continue;
-    }
-    x.small.add(h->g, h->nb.mixed);
-    x.small_kind = sweep_batch_kind(x.small, choice);
-  }
+  for (int j : e->order) x.add(e->m[j]->g, e->m[j]->nb.mixed, e->m[j]->nb.var.s_kind);
   auto corrector = [&](int it) {
     const int role = (it % 2) ? 1 : 2;
     ok &= ens_nonlinear(e, role, s);

@@ -390,7 +390,7 @@ __global__ __launch_bounds__(128) void sweep_kernel(Lin2Args A, const Lin2Args* 
   constexpr bool LAP = lat_lap<PASS, PRED, INC>();
   if constexpr (B != 0) {
     A = tab[blockIdx.y];
-    if ((A.kind == kSweepLat) != (small != 0)) return;  // the other launch's
+    if (A.small != small) return;  // the other launch's
     A.r = gmem(tab, A.r);
     A.rdr = gmem(tab, A.rdr);
     A.uc = gmem(tab, A.uc);
@@ -1356,9 +1356,10 @@ constexpr size_t kLatModes = 400 * 128;
 bool sweep_kind_exists(const Geom& g, bool inc, int kind) {
   return kind == kSweepPlain || (kind == kSweepLat && g.nr <= kLatRows) || (kind == kSweepStream && !inc);
 }
+int sweep_small(const Geom& g) { return sw_nblk(g) <= kLatBlocks && g.nr <= kLatRows ? 1 : 0; }
 int sweep_kind(const Geom& g, bool inc, int choice) {
   if (choice >= 0 && sweep_kind_exists(g, inc, choice)) return choice;
-  if (sw_nblk(g) <= kLatBlocks && g.nr <= kLatRows) return kSweepLat;
+  if (sweep_small(g)) return kSweepLat;
   return !inc && 3 * g.n * sizeof(double2) > (size_t(1) << 30) ? kSweepStream : kSweepPlain;
 }
 void SweepExtent::add(const Geom& g, bool mixed_form) {
@@ -1368,8 +1369,12 @@ void SweepExtent::add(const Geom& g, bool mixed_form) {
   modes += g.modes;
   (mixed_form ? mixed : fp64) = true;
 }
-int sweep_batch_kind(const SweepExtent& small, int choice) {
-  return choice == kSweepLat || small.modes <= kLatModes ? kSweepLat : kSweepPlain;
+void SweepBatch::add(const Geom& g, bool mixed_form, int choice) {
+  const int small = sweep_small(g);
+  SweepExtent& x = part[small];
+  x.add(g, mixed_form);
+  const bool lat = choice >= 0 ? choice == kSweepLat : small && x.modes <= kLatModes;
+  kind[small] = lat && x.max_nr <= kLatRows ? kSweepLat : kSweepPlain;
 }
 template <int PASS, int PRED, int INC>
 static size_t lat_lds(int nr) {
@@ -1435,10 +1440,10 @@ void launch_sweep2(const Lin2Args& a, hipStream_t s) {
 void launch_sweep_batch(const Lin2Args* tab, int count, int predictor, const SweepBatch& b, hipStream_t s) {
   Lin2Args dummy{};
   for (const int small : {1, 0}) {
-    const SweepExtent& x = small ? b.small : b.large;
+    const SweepExtent& x = b.part[small];
     if (x.modes == 0) continue;
     const dim3 grid((x.max_nt / 2) * ((x.max_nz + 63) / 64), count);
-    if (small && b.small_kind == kSweepLat) {
+    if (b.kind[small] == kSweepLat) {
       if (predictor) sweep_passes_lat<1, 1>(dummy, tab, small, grid, x.max_nr, s);
       else sweep_passes_lat<0, 1>(dummy, tab, small, grid, x.max_nr, s);
     } else {

@@ -242,7 +242,8 @@ struct Lin2Args {
   unsigned long long* norm;
   int predictor;
   int ord;              // block order (NlVariant::s_ord)
-  int kind;             // SweepKind
+  int kind;             // SweepKind (single pipes)
+  int small;            // sweep_small: the batched launches that take this member
 };
 // Kinds of the sweep kernels, of the same arithmetic: the general ones, those
 // of small grids (bound by latency) and those that stream past the caches.
@@ -251,6 +252,7 @@ enum SweepKind { kSweepPlain = 0, kSweepLat = 1, kSweepStream = 2 };
 // (NlVariant::s_kind).
 int sweep_kind(const Geom& g, bool inc, int choice);
 bool sweep_kind_exists(const Geom& g, bool inc, int kind);
+int sweep_small(const Geom& g);  // whether the grid alone asks for kSweepLat
 // Some members of a batched sweep: the largest extents among them, all their
 // modes and whether some are of the FP64 or the mixed form.
 struct SweepExtent {
@@ -259,13 +261,13 @@ struct SweepExtent {
   bool fp64 = false, mixed = false;
   void add(const Geom& g, bool mixed_form);
 };
-// A batch's members by their own grids, and the kind the small ones run
-// (kSweepPlain or kSweepLat).
+// A batch's members by their own grids (sweep_small), as the launches take
+// them, and the kind of each launch: kSweepPlain or kSweepLat.
 struct SweepBatch {
-  SweepExtent small, large;  // members of kind kSweepLat, the others
-  int small_kind = kSweepPlain;
+  SweepExtent part[2];  // the large members, the small ones
+  int kind[2] = {kSweepPlain, kSweepPlain};
+  void add(const Geom& g, bool mixed_form, int choice);  // choice: as for sweep_kind (the last member's holds)
 };
-int sweep_batch_kind(const SweepExtent& small, int choice);  // choice: as for sweep_kind
 // F32 (may be null): FP32 copies of the u+, u-, uz factor sets, same indices
 void launch_factor(const Geom& g, const double* r, const double* Lu, const double* Lp, double* F, float* F32,
                    hipStream_t s);

@@ -280,3 +280,26 @@ def test_batched_sweeps_of_either_kind_match_single_pipes(kind):
             assert np.array_equal(a, b), j
         p.close()
     ens.close()
+
+
+def test_member_tuning_between_steps_skips_no_member():
+    """A sweep kind chosen on a member after the ensemble's graphs exist: the
+    launches of the step go on taking every member."""
+    print("[gpu] member tuning between ensemble steps", flush=True)
+    ms = [dict(A, nr=9), dict(A), dict(B)]
+    ens = nsp.Ensemble(ms)
+    pipes = [nsp.Pipe(**kw) for kw in ms]
+    for j, p in enumerate(pipes):
+        for q in (ens[j], p):
+            q.set_tuning(PAIR_VARIANT)
+            seed_member(q, j)
+    ens.step(1)
+    for j, kind in ((1, 0), (2, 1)):
+        ens[j].set_tuning(dict(PAIR_VARIANT, s_kind=kind))
+    ens.step(1)
+    for j, p in enumerate(pipes):
+        p.step(2)
+        for a, b in zip(ens[j].get_state(), p.get_state()):
+            assert np.array_equal(a, b), j
+        p.close()
+    ens.close()
