@@ -46,6 +46,7 @@ struct nsp_handle {
   double* F = nullptr;      // banded LU factors (u+ all modes, u- row NT/2, uz and p rows <= NT/2)
   float* F32 = nullptr;     // mixed form: FP32 copies of the u+, u-, uz sets (read for |m| >= kM32)
   double* PH = nullptr;     // homogeneous pressure data (rows it <= NT/2), sweep-side layout
+  double2* rr = nullptr;    // two-word reciprocals of r and r^2
   double* Dc = nullptr;     // centred D table
   double* Luc = nullptr;    // centred Lu table
   unsigned long long* norm = nullptr;  // device [2]
@@ -185,6 +186,7 @@ Lin2Args lin_args(nsp_handle* h, const Geom& g, const double2* N, const double2*
   Lin2Args a;
   a.g = g;
   a.r = h->t.r;
+  a.rr = h->rr;
   a.rdr = h->t.rdr;
   a.uc = h->t.uc;
   a.qc = h->t.qc;
@@ -479,6 +481,7 @@ static nsp_status create_handle(const nsp_params* p, int device, const nsp_handl
     if (h->nb.mixed) TRY(dalloc(h, &h->F32, factor32_count(g)));
     TRY(dalloc(h, &h->PH, sw_ph_count(g)));
   }
+  TRY(upload(h, &h->rr, recip_table(h->host.r)));
   TRY(upload(h, &h->Dc, centred_table(g.nr, h->host.D)));
   TRY(upload(h, &h->Luc, centred_table(g.nr, h->host.Lu)));
   if (share)

@@ -312,15 +312,9 @@ __device__ __forceinline__ void walk_rows(int t0, int t1, L&& load, F&& work) {
     walk_ring<PD, DIR>(ring, t0, t1, load, work);
   }
 }
-// 1/d (d > 0) as the sum of the largest double below it and the rest, and x/d
-// from it: x hi + x lo, rounded once but for 2^-104 of it, so the quotient of
-// an IEEE division except where that lies within 2^-51 of an ulp of a tie.
-// lo > 0, so that infinities and the sign of a zero come out as a division's.
-__device__ __forceinline__ double2 recip_of(double d) {
-  double hi = 1.0 / d;
-  if (__builtin_fma(-hi, d, 1.0) <= 0.0) hi = __longlong_as_double(__double_as_longlong(hi) - 1);
-  return make_double2(hi, __builtin_fma(-hi, d, 1.0) / d);
-}
+// x / d from d's two-word reciprocal (recip_table): x hi + x lo, rounded once but
+// for 2^-104 of it, so the quotient of an IEEE division except where that lies
+// within 2^-51 of an ulp of a tie.
 __device__ __forceinline__ double times_recip(double x, double2 r) { return __builtin_fma(x, r.x, x * r.y); }
 
 // Rounds a value where it is formed: the compiler does not fuse it with its use.
@@ -369,8 +363,8 @@ struct Tab<1> {
 // the loads of kLatRing rows in flight, reads the radial tables from an LDS
 // copy (a first touch of a table row through the scalar cache is another
 // memory round trip per row) and multiplies by tabled reciprocals of two words
-// (recip_of; of one word, a rounding more per quotient, 24x64x65 took 92 / 93
-// instead of 94 / 95 us and larger grids the same).  Pass D holds the wall rows
+// (of one word, a rounding more per quotient, 24x64x65 took 92 / 93 instead of 94 /
+// 95 us and larger grids the same).  Pass D holds the wall rows
 // (as HOLD = 1).  The results are the general kernels', bit for bit.
 // General / LAT, us, predictor and corrector: 24x64x65 FP64 118 / 94 and 121 /
 // 95, 64x64x385 FP64 400 / 248 and 437 / 293, refined 419 / 271 and 372 / 291,
@@ -385,13 +379,14 @@ constexpr bool lat_lap() {
 // argument of its own: read from A, it made every access a flat one.)
 template <int PASS, int PRED, int B, int HOLD = 0, int INC = 0, int LAT = 0, int STR = 0>
 __global__ __launch_bounds__(128) void sweep_kernel(Lin2Args A, const Lin2Args* tab, int small) {
-  // LAT, not pass B: recip_of r [nr], LAP: of r^2 [nr], D [2][nr][7], LAP: Lu [2][nr][7]
+  // LAT, not pass B: reciprocals of r [nr] and, LAP, of r^2 [nr], D [2][nr][7], LAP: Lu [2][nr][7]
   extern __shared__ double2 lat_tab[];
   constexpr bool LAP = lat_lap<PASS, PRED, INC>();
   if constexpr (B != 0) {
     A = tab[blockIdx.y];
     if (A.small != small) return;  // the other launch's
     A.r = gmem(tab, A.r);
+    A.rr = gmem(tab, A.rr);
     A.rdr = gmem(tab, A.rdr);
     A.uc = gmem(tab, A.uc);
     A.qc = gmem(tab, A.qc);
@@ -433,11 +428,7 @@ __global__ __launch_bounds__(128) void sweep_kernel(Lin2Args A, const Lin2Args* 
   if constexpr (LAT && PASS != 1) {
     const int n7 = 2 * STEN * g.nr;
     double* const rows = reinterpret_cast<double*>(lat_tab + (LAP ? 2 : 1) * g.nr);
-    for (int e = threadIdx.x; e < g.nr; e += 128) {
-      const double r = A.r[e];
-      lat_tab[e] = recip_of(r);
-      if constexpr (LAP) lat_tab[g.nr + e] = recip_of(r * r);
-    }
+    for (int e = threadIdx.x; e < (LAP ? 2 : 1) * g.nr; e += 128) lat_tab[e] = A.rr[e];
     for (int e = threadIdx.x; e < n7; e += 128) {
       rows[e] = A.Dc[e];
       if constexpr (LAP) rows[n7 + e] = A.Luc[e];

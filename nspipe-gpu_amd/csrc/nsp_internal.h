@@ -215,6 +215,7 @@ struct Batch {
 struct Lin2Args {
   Geom g;
   const double* r;      // [NR]
+  const double2* rr;    // [2][NR] recip_table
   const double* rdr;    // [NR]
   const double* uc;     // [NR] flux profile
   const double* qc;     // [1]
@@ -278,6 +279,8 @@ void launch_sweep2(const Lin2Args& a, hipStream_t s);
 void launch_sweep_batch(const Lin2Args* tab, int count, int predictor, const SweepBatch& x, hipStream_t s);
 // centred stencil table: w-th weight of row i multiplies column i-3+w
 std::vector<double> centred_table(int nr, const std::vector<double>& T);
+// two-word reciprocals of r, then of r^2
+std::vector<double2> recip_table(const std::vector<double>& r);
 
 // Kernel variant of one theta stage: alg 0 = LDS-scatter form (tl 4, 8 or 16
 // columns, 256 threads; pad 1 = one LDS slot per 16 or 8 elements, pad 2 =

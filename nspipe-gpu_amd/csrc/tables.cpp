@@ -313,6 +313,20 @@ std::vector<double> centred_table(int nr, const std::vector<double>& T) {
   return C;
 }
 
+// 1/d as hi + lo with hi the largest double below it: lo > 0, so that x hi + x lo
+// keeps infinities and the sign of a zero x, as a division does.
+std::vector<double2> recip_table(const std::vector<double>& r) {
+  std::vector<double2> t;
+  for (int square = 0; square < 2; square++)
+    for (double d : r) {
+      if (square) d *= d;
+      double hi = 1.0 / d;
+      if (std::fma(-hi, d, 1.0) <= 0.0) hi = std::nextafter(hi, 0.0);
+      t.push_back(make_double2(hi, std::fma(-hi, d, 1.0) / d));
+    }
+  return t;
+}
+
 std::vector<double2> pass_twiddles(const std::vector<int>& radices) {
   std::vector<double2> tw;
   int S = 1;
